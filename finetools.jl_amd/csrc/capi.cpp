@@ -215,6 +215,44 @@ feasm_matrix *coo_path(feasm_mesh *m, const FormParams &fp, int rule, int order,
     return sparse_device(ctx, nt, dp<int32_t>(I), dp<int32_t>(J), dp<double>(V), m->nalldofs, m->nalldofs);
 }
 
+// The matrix of a mesh whose distinct DOF numbers are not node-major
+// (essential boundary conditions number the fixed DOFs last): the node-block
+// pattern serves it too, with the entries' places ranked once per numbering,
+// so the staged blocks are summed straight into the CSC.  H8 36x33x31
+// elasticity FP64: the COO path moves 21 M triples through a radix sort
+// (1.92 ms); this path takes 0.14 ms, 0.33 ms when it builds the pattern first.  Null where the
+// node pattern cannot hold the mesh (the COO path then serves it).
+feasm_matrix *general_path(feasm_mesh *m, const FormParams &fp, int rule, int order, int precision) {
+    feasm_ctx *ctx = m->ctx;
+    if (!m->dofs_unique || m->general_unsupported || m->nelem == 0) return nullptr;
+    const DevQTable &qt = device_qtable(ctx, m->etype, rule, order);
+    const int64_t kd = (int64_t)m->ndn * m->npe;
+    check_sparse_args(m->nelem * kd * kd, m->nalldofs, m->nalldofs);
+    if (!m->general) {
+        try {
+            m->general = build_general_pattern(m);
+        } catch (const Error &e) {
+            if (e.code != FEASM_EUNSUPPORTED) throw;
+            m->general_unsupported = true;
+            return nullptr;
+        }
+    }
+    const GeneralPattern &g = *m->general;
+    build_contributions(m, *g.nodes);
+    std::unique_ptr<feasm_matrix> M(new feasm_matrix);
+    M->ctx = ctx;
+    M->m = M->n = m->nalldofs;
+    M->nnz = g.nodes->nnz;
+    M->colptr = g.colptr;
+    M->rowval = g.rowval;
+    M->nzval = dev_alloc(std::max<size_t>(M->nnz * sizeof(double), 8));
+    void *stage = ensure_stage(m, fp.form, precision);
+    launch_element_stage(ctx, m, qt, fp, precision, stage);
+    launch_gather(ctx, m, *g.nodes, fp, precision, stage, dp<double>(M->nzval), &g);
+    FEASM_HIP(hipStreamSynchronize(ctx->stream));
+    return M.release();
+}
+
 }  // namespace
 
 void feasm_ctx::timing_configure(int slots) {
@@ -423,6 +461,8 @@ static void set_dofs(feasm_mesh *m, int ndn, const std::vector<int64_t> &rowmajo
     m->dofs = dev_alloc(std::max<size_t>(d0.size() * sizeof(int32_t), 4));
     FEASM_HIP(hipMemcpy(m->dofs->p, d0.data(), d0.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     if (m->ndn != ndn) m->pattern.reset();
+    m->general.reset();
+    m->general_unsupported = false;
     m->ndn = ndn;
     m->nalldofs = nalldofs;
     m->nodemajor = nm;
@@ -628,7 +668,8 @@ extern "C" int feasm_bilform(feasm_mesh *m, int form, int rule, int order, const
     check_rule(m, rule);
     const FormParams fp = make_form_params(form, m->ndn, coeff, ncoeff);
     if (!m->nodemajor) {
-        *out = coo_path(m, fp, rule, order, precision);
+        *out = general_path(m, fp, rule, order, precision);
+        if (!*out) *out = coo_path(m, fp, rule, order, precision);
         return FEASM_OK;
     }
     ensure_pattern(m, m->numeric_path == 1 ||

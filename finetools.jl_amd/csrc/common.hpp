@@ -182,6 +182,18 @@ struct Pattern {
     feasm::DevPtr bmult;     // uint16 [nblocks+1] contributions of each block (until the lists are built)
 };
 
+// The DOF-level CSC of a mesh whose DOF numbers are distinct but not
+// node-major (essential boundary conditions, a permuted entity order): the
+// node-block pattern with its contribution lists, and where each entry goes.
+// The ndn columns of a node have the same rows, the numbers of its
+// neighbours' DOFs sorted, so one rank list per node serves them all.
+struct GeneralPattern {
+    std::shared_ptr<Pattern> nodes;  // node-block pattern (no DOF-level arrays)
+    feasm::DevPtr colptr;            // int64 [nalldofs+1]
+    feasm::DevPtr rowval;            // int32 [nnz]
+    feasm::DevPtr rank;              // uint16 [nblocks*ndn] slot of (block, row component) in the node's columns
+};
+
 struct feasm_mesh {
     CtxRef ctx;
     int etype = 0, npe = 0;
@@ -195,6 +207,8 @@ struct feasm_mesh {
     bool nodemajor = false;
     feasm::DevPtr dofs;     // int32 [nnodes*ndn] 0-based DOF numbers (node-major rows)
     std::shared_ptr<Pattern> pattern;
+    std::shared_ptr<GeneralPattern> general;  // for the current numbering, once assembled
+    bool general_unsupported = false;         // beyond the node pattern's limits: the COO path
     feasm::DevPtr stage;    // per-element staging of the node-pair blocks
     // numeric path: 0 = automatic (fused tiles when the element/rule has a
     // fused kernel), 1 = staged element blocks + ordered gather, 2 = fused
@@ -269,7 +283,9 @@ feasm_matrix *symm_plus_transpose(feasm_ctx *ctx, const feasm_matrix *S);
 void build_node_to_element(feasm_mesh *m);
 // with_contrib: the staged path will run first, so the adjacency pass also
 // writes the contribution lists (build_contributions then only scans)
-std::shared_ptr<Pattern> build_pattern(feasm_mesh *m, int ndn, bool with_contrib = false);
+std::shared_ptr<Pattern> build_pattern(feasm_mesh *m, int ndn, bool with_contrib = false, bool dof_level = true);
+// the DOF-level CSC of the mesh's own (distinct, not node-major) numbering
+std::shared_ptr<GeneralPattern> build_general_pattern(feasm_mesh *m);
 // every entry of the device connectivity d_conn[0..n) lies in [0, nnodes)
 bool conn_in_range(feasm_ctx *ctx, const int32_t *d_conn, int64_t n, int64_t nnodes);
 void build_contributions(feasm_mesh *m, Pattern &p);
@@ -287,8 +303,9 @@ void launch_element_stage(feasm_ctx *ctx, const feasm_mesh *m, const DevQTable &
                           int precision, void *stage);
 void launch_element_coo(feasm_ctx *ctx, const feasm_mesh *m, const DevQTable &qt, const FormParams &fp,
                         int precision, int32_t *I, int32_t *J, double *V);
+// general: the entries go where that numbering has them (null: node-major)
 void launch_gather(feasm_ctx *ctx, const feasm_mesh *m, const Pattern &p, const FormParams &fp, int precision,
-                   const void *stage, double *nzval);
+                   const void *stage, double *nzval, const GeneralPattern *general = nullptr);
 
 // coo.hip
 feasm_matrix *sparse_device(feasm_ctx *ctx, int64_t ntrip, const int32_t *I, const int32_t *J, const double *V,

@@ -16,12 +16,14 @@ namespace feasm {
 
 namespace {
 
-template <int NDN, int SW, bool DOT, typename S>
+template <int NDN, int SW, bool DOT, bool GENERAL, typename S>
 __global__ __launch_bounds__(256) void k_gather(const int64_t *__restrict__ adj_ptr, const int32_t *__restrict__ bcol,
                                                 const int64_t *__restrict__ cptr,
                                                 const uint32_t *__restrict__ contrib, int64_t nblocks, int npairs,
                                                 const S *__restrict__ stage, FormParams fp,
-                                                double *__restrict__ nzval) {
+                                                const int32_t *__restrict__ dofs,
+                                                const int64_t *__restrict__ gcolptr,
+                                                const uint16_t *__restrict__ rank, double *__restrict__ nzval) {
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < nblocks;
          t += (int64_t)gridDim.x * blockDim.x) {
         const int32_t c = bcol[t];
@@ -62,10 +64,15 @@ __global__ __launch_bounds__(256) void k_gather(const int64_t *__restrict__ adj_
                 }
             }
         }
-        // block (m, c): entry (k, l) sits in DOF column c*NDN + l at row slot r*NDN + k
+        // block (m, c): entry (k, l) sits in DOF column c*NDN + l at row slot
+        // r*NDN + k, or where the general numbering has it
         const int64_t base = (int64_t)NDN * NDN * b0 + r * NDN;
+        int slot[NDN];
 #pragma unroll
-        for (int l = 0; l < NDN; l++)
+        for (int k = 0; k < NDN; k++) slot[k] = GENERAL ? (int)rank[t * NDN + k] : k;
+#pragma unroll
+        for (int l = 0; l < NDN; l++) {
+            const int64_t col = GENERAL ? gcolptr[dofs[(int64_t)c * NDN + l]] : base + (int64_t)l * NDN * deg;
 #pragma unroll
             for (int k = 0; k < NDN; k++) {
                 double v;
@@ -73,31 +80,36 @@ __global__ __launch_bounds__(256) void k_gather(const int64_t *__restrict__ adj_
                     v = acc[0] * fp.coef[NDN * k + l];
                 else
                     v = acc[SW == 9 ? 3 * k + l : 0];
-                nzval[base + (int64_t)l * NDN * deg + k] = v;
+                nzval[col + slot[k]] = v;
             }
+        }
     }
 }
 
 template <int NDN, int SW, bool DOT, typename S>
 void go(feasm_ctx *ctx, const feasm_mesh *m, const Pattern &p, const FormParams &fp, const void *stage,
-        double *nzval) {
-    hipLaunchKernelGGL((k_gather<NDN, SW, DOT, S>), dim3(grid_for(p.nblocks, 256)), dim3(256), 0, ctx->stream,
-                       dp<int64_t>(p.adj_ptr), dp<int32_t>(p.bcol), dp<int64_t>(p.cptr), dp<uint32_t>(p.contrib),
-                       p.nblocks, npairs(m->npe), static_cast<const S *>(stage), fp, nzval);
+        double *nzval, const GeneralPattern *g) {
+    const auto launch = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(grid_for(p.nblocks, 256)), dim3(256), 0, ctx->stream, dp<int64_t>(p.adj_ptr),
+                           dp<int32_t>(p.bcol), dp<int64_t>(p.cptr), dp<uint32_t>(p.contrib), p.nblocks,
+                           npairs(m->npe), static_cast<const S *>(stage), fp, dp<int32_t>(m->dofs),
+                           g ? dp<int64_t>(g->colptr) : nullptr, g ? dp<uint16_t>(g->rank) : nullptr, nzval);
+    };
+    g ? launch(k_gather<NDN, SW, DOT, true, S>) : launch(k_gather<NDN, SW, DOT, false, S>);
     FEASM_HIP(hipGetLastError());
 }
 
 template <typename S>
 void by_form(feasm_ctx *ctx, const feasm_mesh *m, const Pattern &p, const FormParams &fp, const void *stage,
-             double *nzval) {
+             double *nzval, const GeneralPattern *g) {
     switch (fp.form) {
-        case FEASM_FORM_LIN_ELASTIC: return go<3, 9, false, S>(ctx, m, p, fp, stage, nzval);
+        case FEASM_FORM_LIN_ELASTIC: return go<3, 9, false, S>(ctx, m, p, fp, stage, nzval, g);
         case FEASM_FORM_DIFFUSION_ISO:
-        case FEASM_FORM_DIFFUSION_MAT: return go<1, 1, false, S>(ctx, m, p, fp, stage, nzval);
+        case FEASM_FORM_DIFFUSION_MAT: return go<1, 1, false, S>(ctx, m, p, fp, stage, nzval, g);
         case FEASM_FORM_DOT:
-            if (fp.ndn == 1) return go<1, 1, true, S>(ctx, m, p, fp, stage, nzval);
-            if (fp.ndn == 2) return go<2, 1, true, S>(ctx, m, p, fp, stage, nzval);
-            if (fp.ndn == 3) return go<3, 1, true, S>(ctx, m, p, fp, stage, nzval);
+            if (fp.ndn == 1) return go<1, 1, true, S>(ctx, m, p, fp, stage, nzval, g);
+            if (fp.ndn == 2) return go<2, 1, true, S>(ctx, m, p, fp, stage, nzval, g);
+            if (fp.ndn == 3) return go<3, 1, true, S>(ctx, m, p, fp, stage, nzval, g);
             break;
     }
     throw Error(FEASM_EUNSUPPORTED, "unsupported form / ndn in gather");
@@ -106,12 +118,12 @@ void by_form(feasm_ctx *ctx, const feasm_mesh *m, const Pattern &p, const FormPa
 }  // namespace
 
 void launch_gather(feasm_ctx *ctx, const feasm_mesh *m, const Pattern &p, const FormParams &fp, int precision,
-                   const void *stage, double *nzval) {
+                   const void *stage, double *nzval, const GeneralPattern *general) {
     if (p.nblocks == 0) return;
     if (precision == FEASM_MIXED)
-        by_form<float>(ctx, m, p, fp, stage, nzval);
+        by_form<float>(ctx, m, p, fp, stage, nzval, general);
     else
-        by_form<double>(ctx, m, p, fp, stage, nzval);
+        by_form<double>(ctx, m, p, fp, stage, nzval, general);
 }
 
 }  // namespace feasm

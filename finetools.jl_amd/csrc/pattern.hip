@@ -463,7 +463,90 @@ void launch_dof_pattern(feasm_ctx *ctx, const Pattern &P) {
     FEASM_HIP(hipGetLastError());
 }
 
+// General numbering: one thread per node, the lengths of its NDN columns.
+template <int NDN>
+__global__ __launch_bounds__(256) void k_general_count(const int64_t *__restrict__ adj_ptr, int64_t nnodes,
+                                                       const int32_t *__restrict__ dofs, int32_t *__restrict__ len) {
+    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < nnodes;
+         c += (int64_t)gridDim.x * blockDim.x) {
+        const int deg = (int)(adj_ptr[c + 1] - adj_ptr[c]);
+        if (deg == 0) continue;  // a node of no element: its DOF numbers are unchecked and have no entry
+#pragma unroll
+        for (int l = 0; l < NDN; l++) len[dofs[c * NDN + l]] = NDN * deg;
+    }
+}
+
+// One wavefront per node: the rank of each of its neighbours' DOF numbers
+// among them (all distinct), by counting the smaller ones in LDS -- up to 768
+// of them, 81 for an interior H8 node with 3 DOFs -- and the row indices of
+// the node's NDN columns.
+template <int NDN>
+__global__ __launch_bounds__(64) void k_general_rank(const int64_t *__restrict__ adj_ptr,
+                                                     const int32_t *__restrict__ adj, int64_t nnodes,
+                                                     const int32_t *__restrict__ dofs,
+                                                     const int64_t *__restrict__ colptr,
+                                                     uint16_t *__restrict__ rank, int32_t *__restrict__ rowval) {
+    __shared__ __align__(16) int32_t d[kCap * NDN + 4];
+    const int lane = threadIdx.x;
+    for (int64_t c = blockIdx.x; c < nnodes; c += gridDim.x) {
+        const int64_t b = adj_ptr[c];
+        const int n = (int)(adj_ptr[c + 1] - b) * NDN;
+        for (int i = lane; i < n; i += 64) d[i] = dofs[(int64_t)adj[b + i / NDN] * NDN + i % NDN];
+        const int n4 = (n + 3) & ~3;  // padded for the 16-byte reads; a pad is above every DOF number
+        if (lane < n4 - n) d[n + lane] = 0x7fffffff;
+        __syncthreads();
+        int64_t base[NDN];
+        if (n > 0) {
+#pragma unroll
+            for (int l = 0; l < NDN; l++) base[l] = colptr[dofs[c * NDN + l]];
+        }
+        for (int i = lane; i < n; i += 64) {
+            const int32_t v = d[i];
+            int r = 0;
+            for (int j = 0; j < n4; j += 4) {
+                const int4 w = *reinterpret_cast<const int4 *>(d + j);
+                r += (w.x < v) + (w.y < v) + (w.z < v) + (w.w < v);
+            }
+            rank[b * NDN + i] = (uint16_t)r;
+#pragma unroll
+            for (int l = 0; l < NDN; l++) rowval[base[l] + r] = v;
+        }
+        __syncthreads();
+    }
+}
+
+template <int NDN>
+void launch_general_pattern(feasm_ctx *ctx, const feasm_mesh *m, GeneralPattern &G) {
+    const Pattern &P = *G.nodes;
+    const int64_t nn = m->nnodes, n = m->nalldofs;
+    DevPtr len = dev_alloc((n + 1) * sizeof(int32_t));
+    FEASM_HIP(hipMemsetAsync(len->p, 0, (n + 1) * sizeof(int32_t), ctx->stream));
+    hipLaunchKernelGGL(k_general_count<NDN>, dim3(grid_for(nn, 256)), dim3(256), 0, ctx->stream,
+                       dp<int64_t>(P.adj_ptr), nn, dp<int32_t>(m->dofs), dp<int32_t>(len));
+    FEASM_HIP(hipGetLastError());
+    G.colptr = dev_alloc((n + 1) * sizeof(int64_t));
+    exclusive_scan_i32_to_i64(ctx, dp<int32_t>(len), dp<int64_t>(G.colptr), n + 1);
+    G.rowval = dev_alloc(std::max<size_t>(P.nnz * sizeof(int32_t), 4));
+    G.rank = dev_alloc(std::max<size_t>(P.nblocks * NDN * sizeof(uint16_t), 4));
+    hipLaunchKernelGGL(k_general_rank<NDN>, dim3(grid_for(nn, 1, 1 << 17)), dim3(64), 0, ctx->stream,
+                       dp<int64_t>(P.adj_ptr), dp<int32_t>(P.adj), nn, dp<int32_t>(m->dofs), dp<int64_t>(G.colptr),
+                       dp<uint16_t>(G.rank), dp<int32_t>(G.rowval));
+    FEASM_HIP(hipGetLastError());
+}
+
 }  // namespace
+
+std::shared_ptr<GeneralPattern> build_general_pattern(feasm_mesh *m) {
+    auto G = std::make_shared<GeneralPattern>();
+    G->nodes = build_pattern(m, m->ndn, true, false);
+    if (m->ndn == 1)
+        launch_general_pattern<1>(m->ctx, m, *G);
+    else if (m->ndn == 2)
+        launch_general_pattern<2>(m->ctx, m, *G);
+    else
+        launch_general_pattern<3>(m->ctx, m, *G);
+    return G;
+}
 
 void exclusive_scan_i32_to_i64(feasm_ctx *ctx, const int32_t *in, int64_t *out, int64_t n) {
     size_t bytes = 0;
@@ -560,7 +643,7 @@ void build_contributions(feasm_mesh *m, Pattern &P_) {
     P->bmult.reset();
 }
 
-std::shared_ptr<Pattern> build_pattern(feasm_mesh *m, int ndn, bool with_contrib) {
+std::shared_ptr<Pattern> build_pattern(feasm_mesh *m, int ndn, bool with_contrib, bool dof_level) {
     feasm_ctx *ctx = m->ctx;
     if (!m->n2e_ptr) build_node_to_element(m);
     auto P = std::make_shared<Pattern>();
@@ -624,6 +707,7 @@ std::shared_ptr<Pattern> build_pattern(feasm_mesh *m, int ndn, bool with_contrib
     P->n = nn * ndn;
     P->nnz = P->nblocks * ndn * ndn;
     FEASM_REQUIRE(P->n < (1ll << 31), FEASM_EUNSUPPORTED, "more than 2^31 DOFs");
+    if (!dof_level) return P;
     P->colptr = dev_alloc((P->n + 1) * sizeof(int64_t));
     P->rowval = dev_alloc(std::max<size_t>(P->nnz * sizeof(int32_t), 4));
     if (nn == 0) {
