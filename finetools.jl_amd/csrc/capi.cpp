@@ -462,6 +462,7 @@ static void set_dofs(feasm_mesh *m, int ndn, const std::vector<int64_t> &rowmajo
     FEASM_HIP(hipMemcpy(m->dofs->p, d0.data(), d0.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     if (m->ndn != ndn) m->pattern.reset();
     m->general.reset();
+    m->diag.reset();
     m->general_unsupported = false;
     m->ndn = ndn;
     m->nalldofs = nalldofs;
@@ -517,7 +518,7 @@ void linform_into(feasm_mesh *m, int rule, int order, const double *force, int n
     feasm_ctx *ctx = m->ctx;
     if (!m->n2e_ptr) build_node_to_element(m);  // the gather walks each node's elements
     const DevQTable &qt = device_qtable(ctx, m->etype, rule, order);
-    double *stage = static_cast<double *>(ctx->scratch_get((size_t)m->nelem * m->npe * m->ndn * sizeof(double)));
+    double *stage = static_cast<double *>(ctx->scratch_get((size_t)m->nelem * m->npe * sizeof(double)));
     Timer tm(ctx);
     tm.mark(0);
     launch_linform_dot(ctx, m, qt, force, stage, F);

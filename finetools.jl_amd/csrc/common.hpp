@@ -194,6 +194,13 @@ struct GeneralPattern {
     feasm::DevPtr rank;              // uint16 [nblocks*ndn] slot of (block, row component) in the node's columns
 };
 
+// The diagonal CSC of the DOFs that some element touches (lumped mass).
+struct DiagPattern {
+    int64_t nnz = 0;
+    feasm::DevPtr colptr;  // int64 [nalldofs+1]
+    feasm::DevPtr rowval;  // int32 [nnz]
+};
+
 struct feasm_mesh {
     CtxRef ctx;
     int etype = 0, npe = 0;
@@ -208,6 +215,7 @@ struct feasm_mesh {
     feasm::DevPtr dofs;     // int32 [nnodes*ndn] 0-based DOF numbers (node-major rows)
     std::shared_ptr<Pattern> pattern;
     std::shared_ptr<GeneralPattern> general;  // for the current numbering, once assembled
+    std::shared_ptr<DiagPattern> diag;        // for the current numbering, once lumped
     bool general_unsupported = false;         // beyond the node pattern's limits: the COO path
     feasm::DevPtr stage;    // per-element staging of the node-pair blocks
     // numeric path: 0 = automatic (fused tiles when the element/rule has a
@@ -257,8 +265,14 @@ bool cubic_symmetry(const double *D);
 // tables.cpp
 const DevQTable &device_qtable(feasm_ctx *ctx, int etype, int rule, int order);
 
-// vector.hip: load vector of a constant force (ndn values) into F (nalldofs,
-// device); stage holds nelem*npe*ndn doubles
+// vector.hip: nodal sums over the elements into out, times f[k] for component
+// k: of N_a J w, or for the lumped mass (lumped_sums: the sum of the
+// coefficient's entries and of its diagonal) of the scaled diagonal.  direct:
+// out is indexed by the node-major DOF; else by place[DOF] (place null: the
+// DOF).  stage holds nelem*npe doubles.
+void launch_nodal_sums(feasm_ctx *ctx, const feasm_mesh *m, const DevQTable &qt, const double *lumped_sums,
+                       const double *f, bool direct, const int64_t *place, double *stage, double *out);
+// load vector of a constant force (ndn values) into F (nalldofs, device)
 void launch_linform_dot(feasm_ctx *ctx, const feasm_mesh *m, const DevQTable &qt, const double *force,
                         double *stage, double *F);
 

@@ -1,226 +1,209 @@
-// Load-vector assembly: linform_dot with a constant force on solid elements
-// (m = 3) and the SysvecAssembler (src/FEMMBaseModule.jl:1207-1241,
-// src/AssemblyModule.jl:853-917).
+// Nodal sums over the elements: the load vector of a constant force
+// (linform_dot on solid elements, m = 3, with the SysvecAssembler;
+// src/FEMMBaseModule.jl:1207-1241, src/AssemblyModule.jl:853-917) and the
+// diagonal of the HRZ-lumped mass (lumped.hip).
 //
-// k_vec_elem: one thread per element forms the element vector exactly as the
-// reference loop does -- per quadrature point Factor = det J * w, NkxF = N_k *
-// Factor, elvec[(k, mx)] += NkxF * force[mx] -- and stages it in HBM.
-// (k_vec_factor / k_vec_factor_gather below do the same with less staging
-// for H8 and T10 with their usual rules.)
-// k_vec_gather: one thread per node adds, for each of its DOFs, the staged
-// entries of its elements in ascending element number (the node -> element
-// lists are sorted), starting from zero: the same additions, in the same
-// order, as assemble!'s F[gi] += vec[i] over the element loop.
+// Both are one number per (element, local node) times constants:
+//   load    s_a = sum_q N_a J w            F[(n, k)] = sum_e s_a f_k
+//   lumped  s_a = (em2 / dem2) sum_q N_a^2 J w, with em2 the sum of the element
+//           mass matrix's entries, (sum_a N_a)^2 J w summed over the points times
+//           the sum of c, and dem2 the sum of its diagonal;
+//           M[(n, k), (n, k)] = c_kk sum_e s_a
+// k_nodal_elem: one thread per element stages s_a in npe planes, so that a
+// wavefront's stores, and the reads of neighbouring nodes, fill whole lines;
+// k_nodal_gather: one thread per node adds its elements' numbers in ascending
+// element order (the node -> element lists are sorted), the order of
+// assemble!.
+//
+// What bounds them is the gathers (24-byte node records, then 8-byte staged
+// numbers), so few wide loads per thread: a connectivity row as 16- or 8-byte
+// loads, a node as one 16- and one 8-byte load.  H8 87x79x61 load vector, 40 MB
+// compulsory: staging the points' J w (64 B read per list entry) 54 us, the
+// nodal numbers (8 B) 31 us; HRZ mass of H8 73x61x59: forming the 24 x 24
+// entries 208 us with its scan, this 46 us.
 #include "common.hpp"
 
 namespace feasm {
 
 namespace {
 
+constexpr int kBlock = 128;
+
+// three doubles from an 8-byte aligned address (16- and 8-byte loads)
+struct __attribute__((packed, aligned(8))) Node3 {
+    double x, y, z;
+};
+
 template <int NPE>
-__global__ __launch_bounds__(256) void k_vec_elem(const int32_t *__restrict__ conn, const double *__restrict__ xyz,
-                                                  int64_t nelem, int nqp, const double *__restrict__ N,
-                                                  const double *__restrict__ dN, const double *__restrict__ w,
-                                                  double f0, double f1, double f2, int ndn,
-                                                  double *__restrict__ stage) {
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < nelem; e += (int64_t)gridDim.x * blockDim.x) {
-    double X[NPE][3];
+__device__ __forceinline__ void load_row(const int32_t *__restrict__ conn, int64_t e, int32_t (&c)[NPE]) {
+    if constexpr (NPE == 8) {  // 32-byte rows
+        const int4 *r = reinterpret_cast<const int4 *>(conn + e * NPE);
+        const int4 a = r[0], b = r[1];
+        c[0] = a.x; c[1] = a.y; c[2] = a.z; c[3] = a.w;
+        c[4] = b.x; c[5] = b.y; c[6] = b.z; c[7] = b.w;
+    } else {  // 40-byte rows
+        const int2 *r = reinterpret_cast<const int2 *>(conn + e * NPE);
 #pragma unroll
-    for (int a = 0; a < NPE; a++) {
-        const double *p = xyz + 3 * (int64_t)conn[e * NPE + a];
-        X[a][0] = p[0];
-        X[a][1] = p[1];
-        X[a][2] = p[2];
-    }
-    const double force[3] = {f0, f1, f2};
-    double ev[NPE * 3];
-#pragma unroll
-    for (int i = 0; i < NPE * 3; i++) ev[i] = 0.0;
-    for (int q = 0; q < nqp; q++) {
-        double J[9];
-#pragma unroll
-        for (int i = 0; i < 9; i++) J[i] = 0.0;
-#pragma unroll
-        for (int a = 0; a < NPE; a++) {
-            const double d0 = dN[(q * NPE + a) * 3], d1 = dN[(q * NPE + a) * 3 + 1], d2 = dN[(q * NPE + a) * 3 + 2];
-            J[0] += X[a][0] * d0; J[1] += X[a][0] * d1; J[2] += X[a][0] * d2;
-            J[3] += X[a][1] * d0; J[4] += X[a][1] * d1; J[5] += X[a][1] * d2;
-            J[6] += X[a][2] * d0; J[7] += X[a][2] * d1; J[8] += X[a][2] * d2;
-        }
-        const double det = J[0] * (J[4] * J[8] - J[7] * J[5]) - J[1] * (J[3] * J[8] - J[5] * J[6]) +
-                           J[2] * (J[3] * J[7] - J[4] * J[6]);
-        const double Factor = det * w[q];
-#pragma unroll
-        for (int a = 0; a < NPE; a++) {
-            const double NkxF = N[q * NPE + a] * Factor;
-#pragma unroll
-            for (int k = 0; k < 3; k++)
-                if (k < ndn) ev[a * 3 + k] = ev[a * 3 + k] + NkxF * force[k];
+        for (int i = 0; i < NPE / 2; i++) {
+            const int2 a = r[i];
+            c[2 * i] = a.x;
+            c[2 * i + 1] = a.y;
         }
     }
-    double *out = stage + e * NPE * ndn;
-#pragma unroll
-    for (int a = 0; a < NPE; a++)
-#pragma unroll
-        for (int k = 0; k < 3; k++)
-            if (k < ndn) out[a * ndn + k] = ev[a * 3 + k];
-  }
 }
 
-__global__ __launch_bounds__(256) void k_vec_gather(const int64_t *__restrict__ n2e_ptr,
-                                                    const uint32_t *__restrict__ n2e, int64_t nnodes, int npe,
-                                                    int ndn, const double *__restrict__ stage,
-                                                    const int32_t *__restrict__ dofs, double *__restrict__ F) {
-  for (int64_t n = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; n < nnodes; n += (int64_t)gridDim.x * blockDim.x) {
-    if (n2e_ptr[n] == n2e_ptr[n + 1]) continue;  // a node of no element: its DOFs are never touched
-    double acc[3] = {0.0, 0.0, 0.0};
-    for (int64_t s = n2e_ptr[n]; s < n2e_ptr[n + 1]; s++) {
-        const uint32_t v = n2e[s];
-        const int64_t e = v >> 4;
-        const int a = (int)(v & 15u);
-        const double *p = stage + (e * npe + a) * ndn;
-        for (int k = 0; k < ndn; k++) acc[k] = acc[k] + p[k];
-    }
-    for (int k = 0; k < ndn; k++) F[dofs[n * ndn + k]] = acc[k];
-  }
-}
-
-// The common element families (H8 with 8 points, T10 with 4): the element
-// kernel stages only Factor = det J * w per point, and the gather forms each
-// element vector entry from it -- NkxF = N_k * Factor, elvec += NkxF *
-// force[mx] over the points in order -- before adding it to the node's sum:
-// the same operations, in the same order, as the staged element vectors.
-template <int NPE, int NQP>
-__global__ __launch_bounds__(256) void k_vec_factor(const int32_t *__restrict__ conn, const double *__restrict__ xyz,
-                                                    int64_t nelem, const double *__restrict__ dN,
-                                                    const double *__restrict__ w, double *__restrict__ fac) {
+// The points are a loop: unrolled, their tables (33 doubles a point) spill the
+// scalar registers.
+template <int NPE, bool LUMPED>
+__global__ __launch_bounds__(kBlock) void k_nodal_elem(const int32_t *__restrict__ conn, const double *__restrict__ xyz,
+                                                    int64_t nelem, int nqp, const double *__restrict__ N,
+                                                    const double *__restrict__ dN, const double *__restrict__ w,
+                                                    double csum, double ctrace, double *__restrict__ stage) {
     for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < nelem;
          e += (int64_t)gridDim.x * blockDim.x) {
-        double X[NPE][3];
+        int32_t c[NPE];
+        load_row<NPE>(conn, e, c);
+        Node3 X[NPE];
 #pragma unroll
-        for (int a = 0; a < NPE; a++) {
-            const double *p = xyz + 3 * (int64_t)conn[e * NPE + a];
-            X[a][0] = p[0];
-            X[a][1] = p[1];
-            X[a][2] = p[2];
-        }
+        for (int a = 0; a < NPE; a++) X[a] = reinterpret_cast<const Node3 *>(xyz)[c[a]];
+        double s[NPE], total = 0.0;
 #pragma unroll
-        for (int q = 0; q < NQP; q++) {
+        for (int a = 0; a < NPE; a++) s[a] = 0.0;
+#pragma unroll 1
+        for (int q = 0; q < nqp; q++) {
             double J[9];
 #pragma unroll
             for (int i = 0; i < 9; i++) J[i] = 0.0;
 #pragma unroll
             for (int a = 0; a < NPE; a++) {
                 const double d0 = dN[(q * NPE + a) * 3], d1 = dN[(q * NPE + a) * 3 + 1], d2 = dN[(q * NPE + a) * 3 + 2];
-                J[0] += X[a][0] * d0; J[1] += X[a][0] * d1; J[2] += X[a][0] * d2;
-                J[3] += X[a][1] * d0; J[4] += X[a][1] * d1; J[5] += X[a][1] * d2;
-                J[6] += X[a][2] * d0; J[7] += X[a][2] * d1; J[8] += X[a][2] * d2;
+                J[0] += X[a].x * d0; J[1] += X[a].x * d1; J[2] += X[a].x * d2;
+                J[3] += X[a].y * d0; J[4] += X[a].y * d1; J[5] += X[a].y * d2;
+                J[6] += X[a].z * d0; J[7] += X[a].z * d1; J[8] += X[a].z * d2;
             }
             const double det = J[0] * (J[4] * J[8] - J[7] * J[5]) - J[1] * (J[3] * J[8] - J[5] * J[6]) +
                                J[2] * (J[3] * J[7] - J[4] * J[6]);
-            fac[e * NQP + q] = det * w[q];
+            const double jw = det * w[q];
+            double ns = 0.0;
+#pragma unroll
+            for (int a = 0; a < NPE; a++) {
+                const double na = N[q * NPE + a];
+                if (LUMPED) ns += na;
+                s[a] += LUMPED ? na * na * jw : na * jw;
+            }
+            if (LUMPED) total += ns * ns * jw;
+        }
+        double f = 1.0;
+        if (LUMPED) {
+            double d = 0.0;
+#pragma unroll
+            for (int a = 0; a < NPE; a++) d += s[a];
+            f = (total * csum) / (d * ctrace);
+        }
+#pragma unroll
+        for (int a = 0; a < NPE; a++) stage[a * nelem + e] = LUMPED ? s[a] * f : s[a];
+    }
+}
+
+// The node's list entries, then their numbers, are loaded eight at a time (all
+// of an interior H8 node's) before any is added.  DIRECT: the DOFs are
+// node-major and out[d] is DOF d's, so that a node of no element gets its
+// zeros here.  Otherwise DOF d goes to out[place[d]] (place null: out[d]),
+// and the DOFs of a node of no element are left alone.
+template <int NDN, bool DIRECT>
+__global__ __launch_bounds__(kBlock) void k_nodal_gather(const int64_t *__restrict__ n2e_ptr,
+                                                      const uint32_t *__restrict__ n2e, int64_t nnodes,
+                                                      int64_t nelem, const double *__restrict__ stage, double f0, double f1,
+                                                      double f2, const int32_t *__restrict__ dofs,
+                                                      const int64_t *__restrict__ place, double *__restrict__ out) {
+    for (int64_t n = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; n < nnodes;
+         n += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t s0 = n2e_ptr[n], s1 = n2e_ptr[n + 1];
+        if (!DIRECT && s0 == s1) continue;
+        double a0 = 0.0, a1 = 0.0, a2 = 0.0;
+        constexpr int U = 8;
+        for (int64_t s = s0; s < s1; s += U) {
+            uint32_t v[U];
+            double x[U];
+#pragma unroll
+            for (int j = 0; j < U; j++) v[j] = s + j < s1 ? n2e[s + j] : 0u;
+#pragma unroll
+            for (int j = 0; j < U; j++) x[j] = stage[(int64_t)(v[j] & 15u) * nelem + (v[j] >> 4)];
+#pragma unroll
+            for (int j = 0; j < U; j++) {
+                if (s + j >= s1) break;
+                a0 += x[j] * f0;
+                if (NDN > 1) a1 += x[j] * f1;
+                if (NDN > 2) a2 += x[j] * f2;
+            }
+        }
+        const double a[3] = {a0, a1, a2};
+#pragma unroll
+        for (int k = 0; k < NDN; k++) {
+            if (DIRECT) {
+                out[n * NDN + k] = a[k];
+            } else {
+                const int32_t d = dofs[n * NDN + k];
+                out[place ? place[d] : d] = a[k];
+            }
         }
     }
 }
 
-template <int NPE, int NQP>
-__global__ __launch_bounds__(256) void k_vec_factor_gather(const int64_t *__restrict__ n2e_ptr,
-                                                           const uint32_t *__restrict__ n2e, int64_t nnodes,
-                                                           const double *__restrict__ N, int ndn, double f0,
-                                                           double f1, double f2, const double *__restrict__ fac,
-                                                           const int32_t *__restrict__ dofs, double *__restrict__ F) {
-    __shared__ double sN[NQP * NPE];
-    for (int i = threadIdx.x; i < NQP * NPE; i += blockDim.x) sN[i] = N[i];
-    __syncthreads();
-    for (int64_t n = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; n < nnodes;
-         n += (int64_t)gridDim.x * blockDim.x) {
-        if (n2e_ptr[n] == n2e_ptr[n + 1]) continue;  // a node of no element: its DOFs are never touched
-        double acc0 = 0.0, acc1 = 0.0, acc2 = 0.0;
-        // the node's elements four at a time: their list entries, then their
-        // point factors, are loaded before any is used (the sums still run
-        // in list order)
-        constexpr int U = 4;
-        const int64_t s0 = n2e_ptr[n], s1 = n2e_ptr[n + 1];
-        for (int64_t s = s0; s < s1; s += U) {
-            uint32_t v[U];
-#pragma unroll
-            for (int j = 0; j < U; j++) v[j] = s + j < s1 ? n2e[s + j] : 0u;
-            double fq[U][NQP];
-#pragma unroll
-            for (int j = 0; j < U; j++) {
-                const double *fe = fac + (int64_t)(v[j] >> 4) * NQP;
-                if (s + j < s1) {
-#pragma unroll
-                    for (int q = 0; q < NQP; q++) fq[j][q] = fe[q];
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < U; j++) {
-                if (s + j >= s1) break;
-                const int a = (int)(v[j] & 15u);
-                double ev0 = 0.0, ev1 = 0.0, ev2 = 0.0;
-#pragma unroll
-                for (int q = 0; q < NQP; q++) {
-                    const double NkxF = sN[q * NPE + a] * fq[j][q];
-                    ev0 = ev0 + NkxF * f0;
-                    ev1 = ev1 + NkxF * f1;
-                    ev2 = ev2 + NkxF * f2;
-                }
-                acc0 = acc0 + ev0;
-                acc1 = acc1 + ev1;
-                acc2 = acc2 + ev2;
-            }
-        }
-        const int32_t *d = dofs + n * ndn;
-        F[d[0]] = acc0;
-        if (ndn > 1) F[d[1]] = acc1;
-        if (ndn > 2) F[d[2]] = acc2;
-    }
+template <int NPE, bool LUMPED>
+void launch_elem(feasm_ctx *ctx, const feasm_mesh *m, const DevQTable &qt, double csum, double ctrace, double *stage) {
+    if (m->nelem == 0) return;
+    hipLaunchKernelGGL((k_nodal_elem<NPE, LUMPED>), dim3(grid_for(m->nelem, kBlock)), dim3(kBlock), 0, ctx->stream,
+                       dp<int32_t>(m->conn), dp<double>(m->xyz), m->nelem, qt.nqp, qt.N(), qt.dN(), qt.w(), csum,
+                       ctrace, stage);
+    FEASM_HIP(hipGetLastError());
+}
+
+template <int NDN>
+void launch_gather_t(feasm_ctx *ctx, const feasm_mesh *m, const double *stage, const double *f, bool direct,
+                     const int64_t *place, double *out) {
+    if (m->nnodes == 0) return;
+    const auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(grid_for(m->nnodes, kBlock)), dim3(kBlock), 0, ctx->stream, dp<int64_t>(m->n2e_ptr),
+                           dp<uint32_t>(m->n2e), m->nnodes, m->nelem, stage, f[0], f[1], f[2], dp<int32_t>(m->dofs), place, out);
+    };
+    direct ? go(k_nodal_gather<NDN, true>) : go(k_nodal_gather<NDN, false>);
+    FEASM_HIP(hipGetLastError());
+}
+
+void launch_gather_n(feasm_ctx *ctx, const feasm_mesh *m, const double *stage, const double *f, bool direct,
+                     const int64_t *place, double *out) {
+    if (m->ndn == 1) return launch_gather_t<1>(ctx, m, stage, f, direct, place, out);
+    if (m->ndn == 2) return launch_gather_t<2>(ctx, m, stage, f, direct, place, out);
+    return launch_gather_t<3>(ctx, m, stage, f, direct, place, out);
 }
 
 }  // namespace
 
+void launch_nodal_sums(feasm_ctx *ctx, const feasm_mesh *m, const DevQTable &qt, const double *lumped_sums,
+                       const double *f, bool direct, const int64_t *place, double *stage, double *out) {
+    FEASM_REQUIRE(m->conn && m->xyz && m->n2e_ptr && m->n2e && m->dofs && stage && out, FEASM_ESTATE,
+                  "nodal sums: mesh arrays missing");
+    FEASM_REQUIRE(m->npe == 8 || m->npe == 10, FEASM_EUNSUPPORTED, "nodal sums cover H8 and T10 meshes");
+    const double csum = lumped_sums ? lumped_sums[0] : 0.0, ctrace = lumped_sums ? lumped_sums[1] : 0.0;
+    if (m->npe == 8) {
+        lumped_sums ? launch_elem<8, true>(ctx, m, qt, csum, ctrace, stage)
+                    : launch_elem<8, false>(ctx, m, qt, csum, ctrace, stage);
+        launch_gather_n(ctx, m, stage, f, direct, place, out);
+    } else {
+        lumped_sums ? launch_elem<10, true>(ctx, m, qt, csum, ctrace, stage)
+                    : launch_elem<10, false>(ctx, m, qt, csum, ctrace, stage);
+        launch_gather_n(ctx, m, stage, f, direct, place, out);
+    }
+}
+
 void launch_linform_dot(feasm_ctx *ctx, const feasm_mesh *m, const DevQTable &qt, const double *force,
                         double *stage, double *F) {
-    FEASM_REQUIRE(m->conn && m->xyz && m->n2e_ptr && m->n2e && m->dofs && stage && F, FEASM_ESTATE,
-                  "load vector: mesh arrays missing");
-    const int ndn = m->ndn;
-    const double f0 = force[0], f1 = ndn > 1 ? force[1] : 0.0, f2 = ndn > 2 ? force[2] : 0.0;
-    FEASM_HIP(hipMemsetAsync(F, 0, (size_t)m->nalldofs * sizeof(double), ctx->stream));
-    const unsigned ge = grid_for(m->nelem, 256);
-    if ((m->npe == 8 && qt.nqp == 8) || (m->npe == 10 && qt.nqp == 4)) {  // stage holds nelem*npe*ndn >= nelem*nqp
-        const unsigned gn = grid_for(m->nnodes, 256);
-        if (m->npe == 8) {
-            hipLaunchKernelGGL((k_vec_factor<8, 8>), dim3(ge), dim3(256), 0, ctx->stream, dp<int32_t>(m->conn),
-                               dp<double>(m->xyz), m->nelem, qt.dN(), qt.w(), stage);
-            FEASM_HIP(hipGetLastError());
-            hipLaunchKernelGGL((k_vec_factor_gather<8, 8>), dim3(gn), dim3(256), 0, ctx->stream,
-                               dp<int64_t>(m->n2e_ptr), dp<uint32_t>(m->n2e), m->nnodes, qt.N(), ndn, f0, f1, f2,
-                               (const double *)stage, dp<int32_t>(m->dofs), F);
-        } else {
-            hipLaunchKernelGGL((k_vec_factor<10, 4>), dim3(ge), dim3(256), 0, ctx->stream, dp<int32_t>(m->conn),
-                               dp<double>(m->xyz), m->nelem, qt.dN(), qt.w(), stage);
-            FEASM_HIP(hipGetLastError());
-            hipLaunchKernelGGL((k_vec_factor_gather<10, 4>), dim3(gn), dim3(256), 0, ctx->stream,
-                               dp<int64_t>(m->n2e_ptr), dp<uint32_t>(m->n2e), m->nnodes, qt.N(), ndn, f0, f1, f2,
-                               (const double *)stage, dp<int32_t>(m->dofs), F);
-        }
-        FEASM_HIP(hipGetLastError());
-        return;
-    }
-    if (m->npe == 8)
-        hipLaunchKernelGGL((k_vec_elem<8>), dim3(ge), dim3(256), 0, ctx->stream, dp<int32_t>(m->conn),
-                           dp<double>(m->xyz), m->nelem, qt.nqp, qt.N(), qt.dN(), qt.w(), f0, f1, f2, ndn, stage);
-    else if (m->npe == 10)
-        hipLaunchKernelGGL((k_vec_elem<10>), dim3(ge), dim3(256), 0, ctx->stream, dp<int32_t>(m->conn),
-                           dp<double>(m->xyz), m->nelem, qt.nqp, qt.N(), qt.dN(), qt.w(), f0, f1, f2, ndn, stage);
-    else
-        throw Error(FEASM_EUNSUPPORTED, "load vectors cover H8 and T10 meshes");
-    FEASM_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_vec_gather, dim3(grid_for(m->nnodes, 256)), dim3(256), 0, ctx->stream,
-                       dp<int64_t>(m->n2e_ptr), dp<uint32_t>(m->n2e), m->nnodes, m->npe, ndn, stage,
-                       dp<int32_t>(m->dofs), F);
-    FEASM_HIP(hipGetLastError());
+    const double f[3] = {force[0], m->ndn > 1 ? force[1] : 0.0, m->ndn > 2 ? force[2] : 0.0};
+    // node-major: every entry of F is some node's; otherwise F may hold
+    // numbers of no DOF
+    if (!m->nodemajor) FEASM_HIP(hipMemsetAsync(F, 0, (size_t)m->nalldofs * sizeof(double), ctx->stream));
+    launch_nodal_sums(ctx, m, qt, nullptr, f, m->nodemajor, nullptr, stage, F);
 }
 
 }  // namespace feasm
