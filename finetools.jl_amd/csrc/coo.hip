@@ -14,7 +14,14 @@
 //
 // Steps 1-3 (phase A) end with one read-back of the entry count and the range
 // flag; step 4 (phase B) then writes the outputs.
+//
+// Triples that come in runs of one column -- assemble! buffers element matrices
+// column by column, 24 triples at a time for an H8 elasticity element -- take a
+// shorter way (sparse_by_columns): the runs are listed by column, then one
+// wavefront per column sorts the column's rows in registers and folds the
+// duplicates, reading every triple once and in place.
 #include "common.hpp"
+#include "wavesort.hpp"
 
 #include <rocprim/rocprim.hpp>
 
@@ -79,13 +86,318 @@ __global__ void k_colptr(const uint64_t *__restrict__ keys, const int64_t *__res
     }
 }
 
+__global__ void k_fill_i32(int32_t *__restrict__ p, int64_t n, int32_t v) {
+    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x)
+        p[t] = v;
+}
+
 // colptr of a matrix with no entries (a fill kernel rather than a memset)
 __global__ void k_fill_i64(int64_t *__restrict__ p, int64_t n, int64_t v) {
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x)
         p[t] = v;
 }
 
+// ---- sparse_by_columns
+// What bounds it: one read of I, J and V and one write of the result (240 MB for
+// the 11.3 M triples of H8 29x27x25 elasticity), against a radix sort of 64-bit
+// keys that moves them through memory four times (886 us in all; this way
+// 302 us).
+//
+// A run is a stretch of triples of one column within 64 consecutive triples
+// (one wavefront's load).  The runs are put into lists by column with counting
+// atomics, in any order; a column's wavefront orders its few runs by their
+// first triple.
+
+constexpr int kSmallColumn = 256, kMaxColumn = 1024;  // triples of one column the wavefront sorts hold
+// mean run length from which this way pays: the lists take 8 bytes a run
+constexpr int64_t kMinRun = 4;
+// state bits: a row out of range; a column too long or its rows too far apart;
+// a column of more than kSmallColumn triples
+constexpr unsigned kBadRow = 1, kTooWide = 2, kBigColumn = 4;
+
+// the run that starts at this lane's triple: its length, 0 when none does
+__device__ __forceinline__ int run_at(int32_t j, bool in, int lane) {
+    const int32_t prev = __shfl_up(j, 1, 64);
+    const uint64_t heads = __ballot(in && (lane == 0 || prev != j)), all = __ballot(in);
+    if (!((heads >> lane) & 1)) return 0;
+    const uint64_t above = lane < 63 ? heads >> (lane + 1) : 0;
+    return above ? __ffsll((unsigned long long)above) : __popcll(all >> lane);
+}
+
+// per column: its runs (high word) and triples (low word); bad is set for a
+// column index outside [0, n)
+__global__ __launch_bounds__(256) void k_run_count(const int32_t *__restrict__ J, int64_t nt, int64_t n,
+                                                   unsigned long long *__restrict__ cnt,
+                                                   unsigned int *__restrict__ bad) {
+    const int lane = threadIdx.x & 63;
+    const int64_t step = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t - lane < nt; t += step) {
+        const int32_t j = t < nt ? J[t] : 0;
+        const bool ok = j >= 0 && (int64_t)j < n;
+        const int len = run_at(j, t < nt, lane);
+        if (len > 0) {
+            if (ok)
+                atomicAdd(&cnt[j], (1ull << 32) | (unsigned)len);
+            else
+                atomicOr(bad, 1u);
+        }
+    }
+}
+
+// the runs into their columns' lists: (first triple, length), counting the
+// column's runs down.  place[c]: the column's first run (high word) and first
+// place in column order (low word).
+__global__ __launch_bounds__(256) void k_run_fill(const int32_t *__restrict__ J, int64_t nt,
+                                                  const uint64_t *__restrict__ place,
+                                                  unsigned long long *__restrict__ cnt, uint2 *__restrict__ runs) {
+    const int lane = threadIdx.x & 63;
+    const int64_t step = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t - lane < nt; t += step) {
+        const int32_t j = t < nt ? J[t] : 0;
+        const int len = run_at(j, t < nt, lane);
+        if (len > 0) {
+            const unsigned left = (unsigned)(atomicAdd(&cnt[j], ~0ull << 32) >> 32);  // one run fewer
+            runs[(place[j] >> 32) + left - 1] = make_uint2((uint32_t)t, (uint32_t)len);
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void k_col_check(const uint64_t *__restrict__ place, int64_t n,
+                                                   unsigned int *__restrict__ state) {
+    unsigned st = 0;
+    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x) {
+        const uint32_t L = (uint32_t)place[c + 1] - (uint32_t)place[c];
+        st |= (L > kMaxColumn ? kTooWide : 0u) | (L > kSmallColumn ? kBigColumn : 0u);
+    }
+    if (st) atomicOr(state, st);
+}
+
+// One column of L <= 64 E triples in nr runs: its runs ordered, its rows sorted
+// (ties by input order: the key's low B bits are the place in the column),
+// duplicates folded left to right.  The distinct rows and their sums go to
+// trow / tval; returns their number.  lds: 4 * 64 E words of the wavefront's own.
+template <int E, int B>
+__device__ __forceinline__ int sort_column(const int32_t *__restrict__ I, const double *__restrict__ V, int64_t m,
+                                           const uint2 *__restrict__ runs, int nr, int L, int lane, int32_t *lds,
+                                           int32_t *__restrict__ trow, double *__restrict__ tval, unsigned int &state) {
+    constexpr int32_t kPad = 0x7fffffff;
+    // the places of the runs, in order of their first triple (by counting the
+    // triples of earlier runs), and what takes a place to its triple
+    uint32_t *const sS = reinterpret_cast<uint32_t *>(lds), *const sN = sS + 64 * E, *const sAt = sN + 64 * E,
+                    *const sSh = sAt + 64 * E;
+    for (int j = lane; j < nr; j += 64) {
+        const uint2 r = runs[j];
+        sS[j] = r.x;
+        sN[j] = r.y;
+    }
+    wave_fence();
+    for (int j = lane; j < nr; j += 64) {
+        const uint32_t s = sS[j];
+        uint32_t at = 0, rank = 0;
+        for (int k = 0; k < nr; k++) {
+            const bool before = sS[k] < s;
+            at += before ? sN[k] : 0u;
+            rank += before ? 1u : 0u;
+        }
+        sAt[rank] = at;
+        sSh[rank] = s - at;
+    }
+    wave_fence();
+    uint32_t t[E];
+    const int top = nr > 1 ? 1 << (31 - __clz(nr - 1)) : 0;  // the largest power of two below nr
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const uint32_t p = lane + 64 * e;
+        int r = 0;  // the last run at or before place p
+        for (int w = top; w > 0; w >>= 1)
+            if (r + w < nr && sAt[r + w] <= p) r += w;
+        t[e] = p + sSh[r];
+    }
+    wave_fence();
+    double *const sV = reinterpret_cast<double *>(lds);
+    int32_t *const sK = lds + 2 * 64 * E;
+    int32_t x[E], lo = kPad, hi = -1;
+    double v[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int p = lane + 64 * e;
+        x[e] = p < L ? I[t[e]] : kPad;
+        v[e] = p < L ? V[t[e]] : 0.0;
+    }
+    bool out = false;
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const bool in = lane + 64 * e < L;
+        out |= in && (x[e] < 0 || (int64_t)x[e] >= m);
+        lo = in ? min(lo, x[e]) : lo;
+        hi = in ? max(hi, x[e]) : hi;
+        sV[lane + 64 * e] = v[e];
+    }
+#pragma unroll
+    for (int j = 1; j < 64; j <<= 1) {
+        lo = min(lo, lane_xor(lo, j, lane));
+        hi = max(hi, lane_xor(hi, j, lane));
+    }
+    if (__any(out)) {
+        state |= kBadRow;
+        return 0;
+    }
+    if (hi - lo >= (1 << (31 - B)) - 1) {
+        state |= kTooWide;
+        return 0;
+    }
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int p = lane + 64 * e;
+        x[e] = p < L ? ((x[e] - lo) << B) | p : kPad;
+    }
+    wave_sort<E>(x, lane);
+#pragma unroll
+    for (int e = 0; e < E; e++) sK[lane + 64 * e] = x[e];
+    wave_fence();
+    int base = 0;
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int i = lane + 64 * e;
+        const bool head = i < L && (i == 0 || (sK[i > 0 ? i - 1 : 0] >> B) != (x[e] >> B));
+        const uint64_t hm = __ballot(head);
+        if (head) {
+            const int32_t row = x[e] >> B;
+            double a = sV[x[e] & ((1 << B) - 1)];
+            for (int q = i + 1; q < L; q++) {
+                const int32_t y = sK[q];
+                if ((y >> B) != row) break;
+                a = a + sV[y & ((1 << B) - 1)];
+            }
+            const int at = base + __popcll(hm & ((1ull << lane) - 1ull));
+            trow[at] = row + lo;
+            tval[at] = a;
+        }
+        base += __popcll(hm);
+    }
+    wave_fence();  // the words are reused for the next column
+    return base;
+}
+
+// One wavefront per column; BIG: the columns of more than kSmallColumn triples,
+// else the others.  A column's distinct rows and sums go to trow / tval from its
+// first place on, their number to cnt.
+template <bool BIG>
+__global__ __launch_bounds__(64) void k_columns(const int32_t *__restrict__ I, const double *__restrict__ V, int64_t m,
+                                                int64_t n, const uint64_t *__restrict__ place,
+                                                const uint2 *__restrict__ runs, int32_t *__restrict__ cnt,
+                                                int32_t *__restrict__ trow, double *__restrict__ tval,
+                                                unsigned int *__restrict__ state) {
+    __shared__ __align__(16) int32_t lds[4 * (BIG ? kMaxColumn : kSmallColumn)];
+    const unsigned before = *state;
+    if ((before & kTooWide) || (BIG && !(before & kBigColumn))) return;
+    const int lane = threadIdx.x;
+    unsigned int st = 0;
+    for (int64_t c = blockIdx.x; c < n; c += gridDim.x) {
+        const uint64_t a = place[c], b = place[c + 1];
+        const int L = (int)((uint32_t)b - (uint32_t)a), nr = (int)((b >> 32) - (a >> 32));
+        if (BIG != (L > kSmallColumn)) continue;
+        const uint2 *ru = runs + (a >> 32);
+        int32_t *tr = trow + (uint32_t)a;
+        double *tv = tval + (uint32_t)a;
+        int k = 0;
+        if constexpr (BIG)
+            k = L <= 512 ? sort_column<8, 10>(I, V, m, ru, nr, L, lane, lds, tr, tv, st)
+                         : sort_column<16, 10>(I, V, m, ru, nr, L, lane, lds, tr, tv, st);
+        else if (L > 0)
+            k = L <= 64    ? sort_column<1, 8>(I, V, m, ru, nr, L, lane, lds, tr, tv, st)
+                : L <= 128 ? sort_column<2, 8>(I, V, m, ru, nr, L, lane, lds, tr, tv, st)
+                           : sort_column<4, 8>(I, V, m, ru, nr, L, lane, lds, tr, tv, st);
+        if (lane == 0) cnt[c] = k;
+    }
+    if (st && lane == 0) atomicOr(state, st);
+}
+
+// the columns' entries, packed
+__global__ __launch_bounds__(256) void k_columns_pack(const uint64_t *__restrict__ place, int64_t n, const int64_t *__restrict__ colptr,
+                                                      const int32_t *__restrict__ trow, const double *__restrict__ tval,
+                                                      int32_t *__restrict__ rowval, double *__restrict__ nzval) {
+    const int lane = threadIdx.x & 63;
+    for (int64_t c = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6; c < n;
+         c += ((int64_t)gridDim.x * blockDim.x) >> 6) {
+        const int64_t src = (uint32_t)place[c], dst = colptr[c], k = colptr[c + 1] - dst;
+        for (int64_t i = lane; i < k; i += 64) {
+            rowval[dst + i] = trow[src + i];
+            nzval[dst + i] = tval[src + i];
+        }
+    }
+}
+
 }  // namespace
+
+void fill_i64(hipStream_t s, int64_t *p, int64_t n, int64_t v) {
+    hipLaunchKernelGGL(k_fill_i64, dim3(grid_for(n, 256)), dim3(256), 0, s, p, n, v);
+    FEASM_HIP(hipGetLastError());
+}
+
+static void fill_i32(hipStream_t s, int32_t *p, int64_t n, int32_t v) {
+    hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(n, 256)), dim3(256), 0, s, p, n, v);
+    FEASM_HIP(hipGetLastError());
+}
+
+// The shorter way; null when the triples are not in runs, or a column is too
+// long or too wide for the wavefront sort.  Throws FEASM_EDOF for an index out
+// of range, as the general way does.
+static feasm_matrix *sparse_by_columns(feasm_ctx *ctx, int64_t nt, const int32_t *I, const int32_t *J, const double *V,
+                                       int64_t m, int64_t n) {
+    hipStream_t s = ctx->stream;
+    DevPtr small = dev_alloc(256);  // the column range flag, and the state word of k_columns
+    unsigned int *flags = dp<unsigned int>(small);
+    DevPtr ccnt = dev_alloc((n + 1) * 8), place = dev_alloc((n + 1) * 8);
+    fill_i64(s, reinterpret_cast<int64_t *>(flags), 2, 0);
+    fill_i64(s, dp<int64_t>(ccnt), n + 1, 0);
+    const unsigned gt = grid_for(nt, 256, 1u << 14);
+    hipLaunchKernelGGL(k_run_count, dim3(gt), dim3(256), 0, s, J, nt, n, dp<unsigned long long>(ccnt), flags);
+    FEASM_HIP(hipGetLastError());
+    // the run total stays below 2^31 and the triples below 2^32, so the two
+    // words are scanned as one number
+    exclusive_scan_i64(ctx, dp<int64_t>(ccnt), dp<int64_t>(place), n + 1);
+    uint64_t total = 0;
+    unsigned int bad = 0;
+    const ReadBack rb1[2] = {{&total, dp<uint64_t>(place) + n, sizeof(total)}, {&bad, flags, sizeof(bad)}};
+    read_back(s, rb1, 2);
+    FEASM_REQUIRE(bad == 0, FEASM_EDOF, "sparse: row or column index out of range");
+    const int64_t nruns = (int64_t)(total >> 32);
+    if (nt < kMinRun * nruns) return nullptr;
+    DevPtr runs = dev_alloc(nruns * sizeof(uint2));
+    hipLaunchKernelGGL(k_run_fill, dim3(gt), dim3(256), 0, s, J, nt, dp<uint64_t>(place),
+                       dp<unsigned long long>(ccnt), dp<uint2>(runs));
+    FEASM_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_col_check, dim3(grid_for(n, 256)), dim3(256), 0, s, dp<uint64_t>(place), n, flags + 1);
+    DevPtr cnt = dev_alloc((n + 1) * 4), trow = dev_alloc(nt * 4), tval = dev_alloc(nt * 8);
+    fill_i32(s, dp<int32_t>(cnt) + n, 1, 0);
+    const auto columns = [&](auto kern, unsigned most) {
+        hipLaunchKernelGGL(kern, dim3(grid_for(n, 1, most)), dim3(64), 0, s, I, V, m, n, dp<uint64_t>(place),
+                           dp<uint2>(runs), dp<int32_t>(cnt), dp<int32_t>(trow), dp<double>(tval), flags + 1);
+        FEASM_HIP(hipGetLastError());
+    };
+    columns(k_columns<false>, 1u << 17);
+    columns(k_columns<true>, 1u << 11);  // what the LDS of 256 CUs holds; most matrices have no such column
+    std::unique_ptr<feasm_matrix> M(new feasm_matrix);
+    M->ctx = ctx;
+    M->m = m;
+    M->n = n;
+    M->colptr = dev_alloc((n + 1) * sizeof(int64_t));
+    exclusive_scan_i32_to_i64(ctx, dp<int32_t>(cnt), dp<int64_t>(M->colptr), n + 1);
+    unsigned int state = 0;
+    const ReadBack rb2[2] = {{&M->nnz, dp<int64_t>(M->colptr) + n, sizeof(int64_t)}, {&state, flags + 1, sizeof(state)}};
+    read_back(s, rb2, 2);
+    if (state & kTooWide) return nullptr;
+    FEASM_REQUIRE(!(state & kBadRow), FEASM_EDOF, "sparse: row or column index out of range");
+    M->rowval = dev_alloc(std::max<int64_t>(M->nnz, 1) * sizeof(int32_t));
+    M->nzval = dev_alloc(std::max<int64_t>(M->nnz, 1) * sizeof(double));
+    hipLaunchKernelGGL(k_columns_pack, dim3(grid_for(n, 4)), dim3(256), 0, s, dp<uint64_t>(place), n,
+                       dp<int64_t>(M->colptr), dp<int32_t>(trow), dp<double>(tval), dp<int32_t>(M->rowval),
+                       dp<double>(M->nzval));
+    FEASM_HIP(hipGetLastError());
+    FEASM_HIP(hipStreamSynchronize(s));
+    return M.release();
+}
 
 int bits_for(uint64_t v) {
     int b = 0;
@@ -144,11 +456,6 @@ void sparse_phase_b(hipStream_t s, int64_t nt, const double *V, int64_t m, int64
     FEASM_HIP(hipGetLastError());
 }
 
-void fill_i64(hipStream_t s, int64_t *p, int64_t n, int64_t v) {
-    hipLaunchKernelGGL(k_fill_i64, dim3(grid_for(n, 256)), dim3(256), 0, s, p, n, v);
-    FEASM_HIP(hipGetLastError());
-}
-
 void check_sparse_args(int64_t nt, int64_t m, int64_t n) {
     FEASM_REQUIRE(nt >= 0 && m >= 0 && n >= 0, FEASM_EINVAL, "negative size");
     FEASM_REQUIRE(nt < (1ll << 32), FEASM_EUNSUPPORTED, "more than 2^32 triples");
@@ -160,6 +467,8 @@ feasm_matrix *sparse_device(feasm_ctx *ctx, int64_t nt, const int32_t *I, const 
                             int64_t m, int64_t n) {
     check_sparse_args(nt, m, n);
     hipStream_t s = ctx->stream;
+    if (nt > 0)
+        if (feasm_matrix *M = sparse_by_columns(ctx, nt, I, J, V, m, n)) return M;
     std::unique_ptr<feasm_matrix> M(new feasm_matrix);
     M->ctx = ctx;
     M->m = m;

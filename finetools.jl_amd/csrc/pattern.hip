@@ -17,6 +17,7 @@
 //      dof(node, k) = node*ndn + k (numberdofs! with no EBCs,
 //      src/FieldModule.jl:356-377), rows sorted within each column.
 #include "common.hpp"
+#include "wavesort.hpp"
 
 #include <rocprim/rocprim.hpp>
 
@@ -124,44 +125,6 @@ __global__ void k_n2e_sort(const int64_t *__restrict__ ptr, uint32_t *__restrict
 // runs.  Count pass (adj_ptr == nullptr) writes deg[c]; fill pass writes
 // adj[adj_ptr[c] ...].
 constexpr int kMaxCand = 2048;  // candidates of one node: incident elements x npe
-
-// Ascending bitonic sort of 64 E values held by one wavefront in
-// registers: lane l holds entries l + 64 m.  Partners less than 64 apart
-// are exchanged with lane shuffles, partners 64 or more apart sit in two
-// registers of the same lane.
-template <int E>
-__device__ __forceinline__ void wave_sort(int32_t (&x)[E], int lane) {
-#pragma unroll
-    for (int k = 2; k <= 64 * E; k <<= 1)
-#pragma unroll
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            if (j >= 64) {
-                const int jj = j >> 6;
-#pragma unroll
-                for (int m = 0; m < E; m++) {
-                    const int mp1 = m ^ 1, mp2 = m ^ 2;
-                    const int mp = jj == 1 ? mp1 : mp2;
-                    if (mp > m) {
-                        const bool up = ((lane + 64 * m) & k) == 0;
-                        // both partners named with compile-time indices
-                        int32_t &a = x[m];
-                        int32_t &b = (jj == 1) ? x[mp1 < E ? mp1 : m] : x[mp2 < E ? mp2 : m];
-                        const int32_t lo = min(a, b), hi = max(a, b);
-                        a = up ? lo : hi;
-                        b = up ? hi : lo;
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int m = 0; m < E; m++) {
-                    const int i = lane + 64 * m;
-                    const int32_t y = lane_xor(x[m], j, lane);
-                    const bool take_min = ((i & k) == 0) == ((i & j) == 0);
-                    x[m] = take_min ? min(x[m], y) : max(x[m], y);
-                }
-            }
-        }
-}
 
 // The distinct values v = x >> S of a wave-sorted register list of L keys
 // x (the pads after them): their number; each value written to out[pos] and
