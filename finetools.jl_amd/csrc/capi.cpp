@@ -146,11 +146,7 @@ void *ensure_stage(feasm_mesh *m, int form, int precision) {
 }  // namespace
 
 TileShape feasm::mesh_tile_shape(feasm_mesh *m, int nqp, int form, int precision) {
-    TileShape shape = tile_shape_for(m->ctx, m->npe, nqp, form, precision);
-    if (m->tile_nodes > 0) shape.max_nodes = std::min(255, m->tile_nodes);
-    if (m->tile_kib > 0) shape.budget = std::min(shape.budget, (size_t)m->tile_kib * 1024);
-    if (m->tile_threads == 256 || m->tile_threads == 512 || m->tile_threads == 1024) shape.threads = m->tile_threads;
-    return shape;
+    return tile_shape_for(m->ctx, m->npe, nqp, form, precision, m->tile_nodes, m->tile_kib, m->tile_threads);
 }
 
 void feasm::numeric_into_ctx(feasm_ctx *ctx, feasm_mesh *m, const FormParams &fp, int rule, int order,

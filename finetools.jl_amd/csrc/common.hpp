@@ -100,6 +100,8 @@ struct QTable {
     std::vector<double> N, dN, w;
 };
 QTable make_qtable(int etype, int rule, int order);  // tables.cpp
+// the point of the reference's two-point Gauss rule (src/IntegRuleModule.jl:211)
+constexpr double kGauss2 = 0.577350269189626;
 
 // Device copy of a QTable, one contiguous buffer: [N | dN | w].
 struct DevQTable {

@@ -242,11 +242,10 @@ struct Staged {
 };
 // chunks prefetched per thread (measured: the FP64 and DOT kernels gain from
 // a second chunk on the larger T10 blobs and nothing from a third; the
-// mixed-precision gradient kernels are faster with one, and so is FP64 scalar
-// diffusion, where the compiler spilled a second chunk around every task)
+// mixed-precision gradient kernels are faster with one)
 template <typename R, int FORM>
 constexpr int staged_chunks() {
-    return ((sizeof(R) == 4 && FORM != FEASM_FORM_DOT) || FORM == FEASM_FORM_DIFFUSION_ISO) ? 1 : 2;
+    return (sizeof(R) == 4 && FORM != FEASM_FORM_DOT) ? 1 : 2;
 }
 
 // A tile header.  With `hdr` a __restrict__ kernel argument (nothing the
@@ -597,10 +596,12 @@ __device__ __forceinline__ TileRange xcd_range(int64_t ntiles) {
 }
 
 template <int NPE, int NQP, int FORM, int NDN, typename R>
-__global__ __launch_bounds__(kMaxThreads) void k_fused(TileShape shape, TileJob job,
+__global__ __launch_bounds__(kMaxThreads) void k_fused(TileShape shape_, TileJob job,
                                                     const TileHdr *__restrict__ hdr, int64_t ntiles,
                                                     FusedParams kp) {
     extern __shared__ __align__(16) unsigned char smem[];
+    TileShape shape = shape_;
+    shape.packed = false;  // known here, so that the layout has no branch for it
     const TileRange rg = xcd_range(ntiles);
     if (rg.begin >= rg.end) return;
     constexpr int DS = NPE * 3;  // TileShape::dstride()
@@ -656,6 +657,294 @@ __global__ __launch_bounds__(kMaxThreads) void k_fused(TileShape shape, TileJob 
     }
 }
 
+// ---- H8 FP64 diffusion (scalar or 3 x 3 coefficient): packed element matrices
+//
+// One number per node pair, so a halo element's whole symmetric matrix (36
+// doubles) takes less LDS than its gradients (192) and a block's sum reads one
+// double per element instead of two nodes' gradients at every point.
+// Phase 1: two lanes per halo element form the matrix in registers, half of the
+// points each, and add their halves.  Phase 2: as in the general kernel, the sums in ascending
+// element order.  Two workgroups of 256 threads per CU, so that one's phase 1
+// (vector arithmetic) runs beside the other's loads, sums and stores.  H8
+// 71x53x47: the general kernel, bound by its LDS reads, 152 us; this one 61 us.
+
+constexpr int kPackedThreads = 256, kPackedKiB = 80, kPackedChunks = 4;
+
+// The metric of one point for diffusion, G = J w inv(J) (coefficient) inv(J)',
+// as G11 G12 G13 G22 G23 G33, from the columns of the Jacobian (derivatives of
+// x along the three directions).
+template <int FORM>
+__device__ __forceinline__ void point_metric(const double (&j1)[3], const double (&j2)[3], const double (&j3)[3],
+                                             double w, const double *coef, double (&G)[6]) {
+    // the rows of the adjugate: cross products of the columns
+    const double r1[3] = {j2[1] * j3[2] - j2[2] * j3[1], j2[2] * j3[0] - j2[0] * j3[2], j2[0] * j3[1] - j2[1] * j3[0]};
+    const double r2[3] = {j3[1] * j1[2] - j3[2] * j1[1], j3[2] * j1[0] - j3[0] * j1[2], j3[0] * j1[1] - j3[1] * j1[0]};
+    const double r3[3] = {j1[1] * j2[2] - j1[2] * j2[1], j1[2] * j2[0] - j1[0] * j2[2], j1[0] * j2[1] - j1[1] * j2[0]};
+    const double det = j1[0] * r1[0] + j1[1] * r1[1] + j1[2] * r1[2];
+    double s = w / det;  // det w / det^2
+    double f1[3], f2[3], f3[3];
+    if constexpr (FORM == FEASM_FORM_DIFFUSION_ISO) {
+        s *= coef[0];
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            f1[k] = s * r1[k];
+            f2[k] = s * r2[k];
+            f3[k] = s * r3[k];
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            f1[k] = s * (coef[3 * k] * r1[0] + coef[3 * k + 1] * r1[1] + coef[3 * k + 2] * r1[2]);
+            f2[k] = s * (coef[3 * k] * r2[0] + coef[3 * k + 1] * r2[1] + coef[3 * k + 2] * r2[2]);
+            f3[k] = s * (coef[3 * k] * r3[0] + coef[3 * k + 1] * r3[1] + coef[3 * k + 2] * r3[2]);
+        }
+    }
+    G[0] = r1[0] * f1[0] + r1[1] * f1[1] + r1[2] * f1[2];
+    G[1] = r1[0] * f2[0] + r1[1] * f2[1] + r1[2] * f2[2];
+    G[2] = r1[0] * f3[0] + r1[1] * f3[1] + r1[2] * f3[2];
+    G[3] = r2[0] * f2[0] + r2[1] * f2[1] + r2[2] * f2[2];
+    G[4] = r2[0] * f3[0] + r2[1] * f3[1] + r2[2] * f3[2];
+    G[5] = r3[0] * f3[0] + r3[1] * f3[1] + r3[2] * f3[2];
+}
+
+// H8 with GaussRule(3, 2): the four points of one xi half (point number 4 xi +
+// 2 eta + zeta), summed over the points direction by direction.  With n(c, p)
+// the 1D basis value of corner side c at point p (lo or hi below), node a =
+// (i, j, k) has dN_a = (s_i n_j n_k, s_j n_i n_k, s_k n_i n_j) / 2 (s = -1 or
+// 1), so the metric's six components are contracted with products of 1D values
+// one direction at a time and each pair adds a few of the results: about 700
+// operations for the 36 pairs, against 1250 for gradients and their dot
+// products.  S: packed upper triangle in the local node order.
+template <int FORM>
+__device__ __forceinline__ void h8_half(const double2 *__restrict__ sXY, const double *__restrict__ sZ,
+                                        const int (&n)[8], bool odd, double w, const double *coef, double (&S)[36]) {
+    // local node of corner (i, j, k)
+    constexpr int node[2][2][2] = {{{0, 4}, {3, 7}}, {{1, 5}, {2, 6}}};
+    constexpr double lo = 0.5 * (1.0 - kGauss2), hi = 0.5 * (1.0 + kGauss2);
+    // n[c][p]: side c at point p
+    constexpr double nb[2][2] = {{hi, lo}, {lo, hi}};
+    const double x0 = odd ? lo : hi, x1 = odd ? hi : lo;  // n_0, n_1 at this half's xi
+    // differences of the coordinates first (exact to rounding; a point far
+    // from the origin costs no digits): D along xi on the (eta, zeta) corners,
+    // E along eta at this xi on the zeta sides, F along zeta on the eta sides
+    // (all halved)
+    double X[2][2][2][3];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const int a = n[node[i][j][k]];
+                const double2 p = sXY[a];
+                X[i][j][k][0] = p.x;
+                X[i][j][k][1] = p.y;
+                X[i][j][k][2] = sZ[a];
+            }
+    const double w0 = 0.5 * x0, w1 = 0.5 * x1;
+    double D[2][2][3], E[2][3], F[2][3];
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            D[j][0][c] = 0.5 * (X[1][j][0][c] - X[0][j][0][c]);
+            D[j][1][c] = 0.5 * (X[1][j][1][c] - X[0][j][1][c]);
+            E[j][c] = w0 * (X[0][1][j][c] - X[0][0][j][c]) + w1 * (X[1][1][j][c] - X[1][0][j][c]);
+            F[j][c] = w0 * (X[0][j][1][c] - X[0][j][0][c]) + w1 * (X[1][j][1][c] - X[1][j][0][c]);
+        }
+    double J2[2][3], J3[2][3];  // d/deta at zeta point z, d/dzeta at eta point e
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            J2[p][c] = nb[0][p] * E[0][c] + nb[1][p] * E[1][c];
+            J3[p][c] = nb[0][p] * F[0][c] + nb[1][p] * F[1][c];
+        }
+    // contractions: over eta (e) inside, then zeta (z)
+    double A11[3][3], A22[3], A33[3], A12[2][3], A13[3][2], A23[2][2];  // [eta index][zeta index]; pairs 00 01 11
+    constexpr double pp[3][2] = {{hi * hi, lo * lo}, {hi * lo, hi * lo}, {lo * lo, hi * hi}};  // n_c n_c' at point p
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        A22[i] = A33[i] = 0.0;
+#pragma unroll
+        for (int j = 0; j < 3; j++) A11[i][j] = 0.0;
+#pragma unroll
+        for (int j = 0; j < 2; j++) A12[j][i] = A13[i][j] = 0.0;
+    }
+    A23[0][0] = A23[0][1] = A23[1][0] = A23[1][1] = 0.0;
+#pragma unroll
+    for (int z = 0; z < 2; z++) {
+        double G[2][6];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            double J1[3];
+#pragma unroll
+            for (int c = 0; c < 3; c++)
+                J1[c] = nb[0][e] * (nb[0][z] * D[0][0][c] + nb[1][z] * D[0][1][c]) +
+                        nb[1][e] * (nb[0][z] * D[1][0][c] + nb[1][z] * D[1][1][c]);
+            point_metric<FORM>(J1, J2[z], J3[e], w, coef, G[e]);
+        }
+        const double t22 = G[0][3] + G[1][3];
+        double t11[3], t13[3], t33[3], t12[2], t23[2];
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            t11[i] = pp[i][0] * G[0][0] + pp[i][1] * G[1][0];
+            t13[i] = pp[i][0] * G[0][2] + pp[i][1] * G[1][2];
+            t33[i] = pp[i][0] * G[0][5] + pp[i][1] * G[1][5];
+        }
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            t12[j] = nb[j][0] * G[0][1] + nb[j][1] * G[1][1];
+            t23[j] = nb[j][0] * G[0][4] + nb[j][1] * G[1][4];
+        }
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            A22[i] += pp[i][z] * t22;
+            A33[i] += t33[i];
+#pragma unroll
+            for (int j = 0; j < 3; j++) A11[i][j] += pp[j][z] * t11[i];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                A12[j][i] += pp[i][z] * t12[j];
+                A13[i][j] += nb[j][z] * t13[i];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int k = 0; k < 2; k++) A23[j][k] += nb[k][z] * t23[j];
+    }
+    // pairs of (eta, zeta) corners (j, k), (l, m): T the xi xi part, B the eta and
+    // zeta parts, U[jk][lm] the cross part with xi derived on the jk side
+    double U[4][4];
+#pragma unroll
+    for (int p = 0; p < 4; p++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int j = p >> 1, k = p & 1, l = q >> 1, m = q & 1;
+            const double a = A12[j][k + m], b = A13[j + l][k];
+            U[p][q] = (l ? a : -a) + (m ? b : -b);
+        }
+    const double q0 = 0.25 * x0 * x0, q1 = 0.25 * x1 * x1, q01 = 0.25 * x0 * x1, h0 = 0.25 * x0, h1 = 0.25 * x1;
+#pragma unroll
+    for (int p = 0; p < 4; p++)
+#pragma unroll
+        for (int q = p; q < 4; q++) {
+            const int j = p >> 1, k = p & 1, l = q >> 1, m = q & 1;
+            const double T = 0.25 * A11[j + l][k + m];
+            const double a22 = A22[k + m], a33 = A33[j + l];
+            const double c1 = A23[l][k], c2 = A23[j][m];  // d/deta on jk with d/dzeta on lm, and the other way
+            const double B = (j == l ? a22 : -a22) + (k == m ? a33 : -a33) + (j == m ? c1 : -c1) + (k == l ? c2 : -c2);
+            const double V = U[p][q] + U[q][p];
+            const auto put = [&](int x, int y, double v) { S[x > y ? x * (x + 1) / 2 + y : y * (y + 1) / 2 + x] = v; };
+            put(node[0][j][k], node[0][l][m], T + q0 * B - h0 * V);
+            put(node[1][j][k], node[1][l][m], T + q1 * B + h1 * V);
+            put(node[0][j][k], node[1][l][m], q01 * B - T + (h0 * U[q][p] - h1 * U[p][q]));
+            if (p != q) put(node[1][j][k], node[0][l][m], q01 * B - T + (h0 * U[p][q] - h1 * U[q][p]));
+        }
+}
+
+template <int FORM, bool LDSCOEF, typename BeforeStores>
+__device__ __forceinline__ void packed_tile(const TileShape &shape, const TileJob &job, const FusedParams &kp,
+                                            const TileHdr &hd, unsigned char *smem, const BeforeStores &before_stores) {
+    constexpr int NPE = 8, NP = 36, PS = NP | 1;  // TileShape::packed_stride()
+    const int tid = threadIdx.x;
+    const TileShape::Layout L = shape.layout(hd.H, hd.P, hd.NH, hd.K, hd.NT, hd.NI);
+    const double *coef = LDSCOEF ? reinterpret_cast<const double *>(smem) + 8 * 8 * 4 : kp.fp.coef;
+    const uint64_t *sTask = reinterpret_cast<const uint64_t *>(smem + L.task);
+    const uint16_t *sItem = reinterpret_cast<const uint16_t *>(smem + L.item);
+    const double2 *sXY = reinterpret_cast<const double2 *>(smem + L.X);
+    const double *sZ = reinterpret_cast<const double *>(smem + L.X) + 2 * hd.NH;
+    const int64_t *sCb = reinterpret_cast<const int64_t *>(smem + L.cbase);
+    double *sS = reinterpret_cast<double *>(smem + L.U);
+
+    // two lanes per element, each half of the points; i < 2 H for both or none
+    const bool odd = tid & 1;
+    for (int i = tid; i < 2 * hd.H; i += kPackedThreads) {
+        const int h = i >> 1;
+        const uint16_t *cn = reinterpret_cast<const uint16_t *>(smem + L.lconn) + h * NPE;
+        int n[NPE];
+#pragma unroll
+        for (int a = 0; a < NPE; a++) n[a] = cn[a];
+        double S[NP];
+        h8_half<FORM>(sXY, sZ, n, odd, 1.0, coef, S);  // every weight of the rule is 1
+        // each lane adds the other's half of the points for its half of the
+        // pairs (quad_perm 1,0,3,2: the neighbour's value)
+        constexpr int HALF = NP / 2;
+#pragma unroll
+        for (int p = 0; p < HALF; p++) {
+            const double keep = odd ? S[p + HALF] : S[p], send = odd ? S[p] : S[p + HALF];
+            const int2 w = __builtin_bit_cast(int2, send);
+            const int2 x = make_int2(__builtin_amdgcn_mov_dpp(w.x, 0xB1, 0xf, 0xf, false),
+                                     __builtin_amdgcn_mov_dpp(w.y, 0xB1, 0xf, 0xf, false));
+            const double sum = keep + __builtin_bit_cast(double, x);
+            sS[h * PS + p + (odd ? HALF : 0)] = sum;
+        }
+    }
+    __syncthreads();
+    before_stores();
+
+    double *__restrict__ nzval = job.nzval;
+    for (int t = tid; t < hd.NT; t += kPackedThreads) {
+        const uint64_t rec = sTask[t];
+        if ((uint32_t)rec == kNullTask) continue;
+        const int k = (int)((rec >> 16) & 255u);
+        const uint16_t *items = sItem + (uint32_t)((rec >> 32) & 0xffffu);
+        // items, then their numbers, four at a time; summed in item order
+        double acc = 0.0;
+        for (int j = 0; j < k; j += 4) {
+            uint32_t it[4];
+            double x[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) it[u] = items[min(j + u, k - 1)];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const uint32_t ac = (it[u] >> 4) & 15u, ar = it[u] & 15u, lo = min(ac, ar), hi = max(ac, ar);
+                x[u] = sS[(it[u] >> 8) * PS + (__umul24(hi, hi + 1) >> 1) + lo];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) acc = j + u < k ? acc + x[u] : acc;
+        }
+        nzval[sCb[rec & 255u] + ((rec >> 8) & 255u)] = acc;
+        const uint32_t pr = (uint32_t)(rec >> 48);
+        if (pr != kNoPair) nzval[sCb[pr & 255u] + (pr >> 8)] = acc;  // the transposed block
+    }
+}
+
+template <int NPE, int NQP, int FORM, int NDN, typename R>
+__global__ __launch_bounds__(kPackedThreads, 2) void k_packed(TileShape shape_, TileJob job,
+                                                           const TileHdr *__restrict__ hdr, int64_t ntiles,
+                                                           FusedParams kp) {
+    static_assert(NPE == 8 && NQP == 8 && NDN == 1 && sizeof(R) == 8);
+    extern __shared__ __align__(16) unsigned char smem[];
+    TileShape shape = shape_;
+    shape.packed = true;
+    const TileRange rg = xcd_range(ntiles);
+    if (rg.begin >= rg.end) return;
+    double *sD = reinterpret_cast<double *>(smem) + NQP * NPE * 4;
+    int *sNeg = reinterpret_cast<int *>(sD + 36);
+    int64_t t1 = rg.begin + rg.step;
+    TileHdr hd = load_hdr(hdr, rg.begin);
+    TileHdr hn = load_hdr(hdr, t1 < rg.end ? t1 : rg.begin);
+    Staged<false, kPackedChunks> st;
+    stage_issue(job, hd, nullptr, st);
+    st.ready();
+    for (;;) {
+        const bool more = t1 < rg.end;
+        const int64_t t2 = t1 + rg.step;
+        const TileHdr h2 = load_hdr(hdr, t2 < rg.end ? t2 : rg.begin);
+        stage_store(job, hd, st, shape.layout(hd.H, hd.P, hd.NH, hd.K, hd.NT, hd.NI), smem, sD, sNeg);
+        __syncthreads();
+        stage_issue(job, more ? hn : hd, nullptr, st);  // waited for before this tile's stores
+        packed_tile<FORM, false>(shape, job, kp, hd, smem, [&]() { st.ready(); });
+        if (!more) break;
+        __syncthreads();
+        t1 = t2;
+        hd = hn;
+        hn = h2;
+    }
+}
+
 // One entry per mesh of a batched launch.
 struct BatchEntry {
     TileJob job;
@@ -672,8 +961,10 @@ template <int NPE, int NQP, int FORM, int NDN, typename R>
 __global__ __launch_bounds__(kMaxThreads) void k_fused_batch(const BatchEntry *__restrict__ entries,
                                                           const int32_t *__restrict__ tile_entry,
                                                           const TileHdr *__restrict__ hdr, int64_t ntiles,
-                                                          TileShape shape) {
+                                                          TileShape shape_) {
     extern __shared__ __align__(16) unsigned char smem[];
+    TileShape shape = shape_;
+    shape.packed = false;  // known here, so that the layout has no branch for it
     const TileRange rg = xcd_range(ntiles);
     if (rg.begin >= rg.end) return;
     constexpr int DS = NPE * 3;  // TileShape::dstride()
@@ -728,6 +1019,50 @@ __global__ __launch_bounds__(kMaxThreads) void k_fused_batch(const BatchEntry *_
     }
 }
 
+// k_packed over the global tile list of a batched launch.
+template <int NPE, int NQP, int FORM, int NDN, typename R>
+__global__ __launch_bounds__(kPackedThreads, 2) void k_packed_batch(const BatchEntry *__restrict__ entries,
+                                                                 const int32_t *__restrict__ tile_entry,
+                                                                 const TileHdr *__restrict__ hdr, int64_t ntiles,
+                                                                 TileShape shape_) {
+    static_assert(NPE == 8 && NQP == 8 && NDN == 1 && sizeof(R) == 8);
+    extern __shared__ __align__(16) unsigned char smem[];
+    TileShape shape = shape_;
+    shape.packed = true;
+    const TileRange rg = xcd_range(ntiles);
+    if (rg.begin >= rg.end) return;
+    double *sD = reinterpret_cast<double *>(smem) + NQP * NPE * 4;
+    int *sNeg = reinterpret_cast<int *>(sD + 36);
+    int64_t t1 = rg.begin + rg.step;
+    TileHdr hd = load_hdr(hdr, rg.begin);
+    const BatchEntry *E = entries + tile_entry[rg.begin];
+    const int64_t i1 = t1 < rg.end ? t1 : rg.begin;
+    TileHdr hn = load_hdr(hdr, i1);
+    const BatchEntry *En = entries + tile_entry[i1];
+    Staged<true, kPackedChunks> st;
+    stage_issue(E->job, hd, E->kp.fp.coef, st);
+    st.ready();
+    for (;;) {
+        const bool more = t1 < rg.end;
+        const int64_t t2 = t1 + rg.step, i2 = t2 < rg.end ? t2 : rg.begin;
+        const TileHdr h2 = load_hdr(hdr, i2);
+        const BatchEntry *E2 = entries + tile_entry[i2];
+        stage_store(E->job, hd, st, shape.layout(hd.H, hd.P, hd.NH, hd.K, hd.NT, hd.NI), smem, sD, sNeg);
+        __syncthreads();
+        const TileHdr &hb = more ? hn : hd;
+        const BatchEntry *Eb = more ? En : E;
+        stage_issue(Eb->job, hb, Eb->kp.fp.coef, st);
+        packed_tile<FORM, true>(shape, E->job, E->kp, hd, smem, [&]() { st.ready(); });
+        if (!more) break;
+        __syncthreads();
+        t1 = t2;
+        hd = hn;
+        E = En;
+        hn = h2;
+        En = E2;
+    }
+}
+
 TileJob make_job(const feasm_mesh *m, const TileSet &t, double *nzval) {
     TileJob j;
     j.hdr = static_cast<const TileHdr *>(t.hdr->p);
@@ -754,7 +1089,13 @@ unsigned persistent_grid(feasm_ctx *ctx, size_t budget, int64_t ntiles) {
 template <int NPE, int NQP, int FORM, int NDN, typename R>
 void go(feasm_ctx *ctx, const feasm_mesh *m, const Pattern &p, const TileSet &t, const FusedParams &kp,
         double *nzval) {
-    auto kern = k_fused<NPE, NQP, FORM, NDN, R>;
+    constexpr bool PACKED = NPE == 8 && sizeof(R) == 8 && (FORM == FEASM_FORM_DIFFUSION_ISO || FORM == FEASM_FORM_DIFFUSION_MAT);
+    auto kern = [] {
+        if constexpr (PACKED)
+            return k_packed<NPE, NQP, FORM, NDN, R>;
+        else
+            return k_fused<NPE, NQP, FORM, NDN, R>;
+    }();
     const int budget = (int)t.shape.budget;
     FEASM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, budget));
     const unsigned grid = persistent_grid(ctx, t.shape.budget, t.ntiles);
@@ -792,7 +1133,13 @@ void dispatch(feasm_ctx *ctx, const feasm_mesh *m, const Pattern &p, const TileS
 
 template <int NPE, int NQP, int FORM, int NDN, typename R>
 void go_batch(feasm_ctx *ctx, const BatchLaunch &b) {
-    auto kern = k_fused_batch<NPE, NQP, FORM, NDN, R>;
+    constexpr bool PACKED = NPE == 8 && sizeof(R) == 8 && (FORM == FEASM_FORM_DIFFUSION_ISO || FORM == FEASM_FORM_DIFFUSION_MAT);
+    auto kern = [] {
+        if constexpr (PACKED)
+            return k_packed_batch<NPE, NQP, FORM, NDN, R>;
+        else
+            return k_fused_batch<NPE, NQP, FORM, NDN, R>;
+    }();
     FEASM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b.budget));
     hipLaunchKernelGGL(kern, dim3(b.grid), dim3(b.threads), b.budget, ctx->stream,
                        static_cast<const BatchEntry *>(b.entries->p), dp<int32_t>(b.tile_entry),
@@ -910,20 +1257,26 @@ void refresh_tile_coords(feasm_mesh *m, TileSet &t) {
 
 bool fused_supported(int npe, int nqp) { return (npe == 8 && nqp == 8) || (npe == 10 && nqp == 4); }
 
-TileShape tile_shape_for(feasm_ctx *ctx, int npe, int nqp, int form, int precision) {
+TileShape tile_shape_for(feasm_ctx *ctx, int npe, int nqp, int form, int precision, int nodes, int kib, int threads) {
     TileShape s;
     s.npe = npe;
     s.nqp = nqp;
     s.rbytes = (precision == FEASM_MIXED) ? 4 : 8;
-    s.grad = (form != FEASM_FORM_DOT);
+    // H8 only: a T10's 55 pairs leave too few registers (measured 50 -> 65 us on 20x21x19)
+    s.packed = npe == 8 && precision == FEASM_FP64 && (form == FEASM_FORM_DIFFUSION_ISO || form == FEASM_FORM_DIFFUSION_MAT);
+    s.grad = (form != FEASM_FORM_DOT) && !s.packed;
     int lds = 0;
     FEASM_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, ctx->device));
-    s.budget = (size_t)std::min(lds, 160 * 1024);
+    s.budget = (size_t)std::min(lds, (s.packed ? kPackedKiB : 160) * 1024);
     // measured best on MI355X: DOT tiles (tiny records, not bound by LDS)
     // with 64 nodes list more block tasks than the workgroup has threads
     s.max_nodes = (form == FEASM_FORM_DOT) ? 32 : 64;
     s.max_halo = 255;
     s.threads = 1024;
+    if (nodes > 0) s.max_nodes = std::min(255, nodes);
+    if (kib > 0) s.budget = std::min(s.budget, (size_t)kib * 1024);
+    if (threads == 256 || threads == 512 || threads == 1024) s.threads = threads;
+    if (s.packed) s.threads = kPackedThreads;  // an element per thread: wider workgroups would idle
     return s;
 }
 

@@ -10,8 +10,11 @@ __host__ __device__ inline size_t align16(size_t x) { return (x + 15) & ~size_t(
 // same function sizes the tiles on the host and carves LDS on the device.
 struct TileShape {
     int npe = 8, nqp = 8;
-    int rbytes = 8;    // sizeof of the element arithmetic type
-    bool grad = true;  // forms that need spatial gradients (all but DOT)
+    int rbytes = 8;  // sizeof of the element arithmetic type
+    bool grad = true;  // gradient records in LDS (all forms but DOT and the packed ones)
+    // H8 FP64 diffusion: a halo element's record is its packed symmetric matrix,
+    // one number per node pair (packed_stride doubles)
+    bool packed = false;
     int max_nodes = 64, max_halo = 255;
     int threads = 256;  // workgroup size of the fused kernel (256, 512 or 1024)
     size_t budget = 0;  // bytes of LDS available to one workgroup
@@ -23,6 +26,8 @@ struct TileShape {
     // chunks per record.  Consecutive records are one chunk further apart, so
     // that they start in different LDS banks.  (nqp a multiple of 2G.)
     __host__ __device__ int uchunks() const { return nqp * npe * 3 * rbytes / 16 + 1; }
+    // an odd stride spreads the lanes' records over the LDS banks
+    __host__ __device__ int packed_stride() const { return (npe * (npe + 1) / 2) | 1; }
     // the record stride in elements of the arithmetic type
     __host__ __device__ int ustride() const { return uchunks() * 16 / rbytes; }
 
@@ -59,9 +64,9 @@ struct TileShape {
         L.X = o;  // halo-node coordinates, the blob's last part
         o = align16(o + (size_t)NH * 3 * 8);
         L.U = o;  // end of the blob
-        o = align16(o + (grad ? (size_t)H * ustride() * rbytes : 0));
+        o = align16(o + (packed ? (size_t)H * packed_stride() * 8 : grad ? (size_t)H * ustride() * rbytes : 0));
         L.sgn = o;  // grad forms: one byte per (element, point), 1 where J w < 0; DOT: J w
-        o = align16(o + (grad ? (size_t)H * nqp : (size_t)H * nqp * rbytes));
+        o = align16(o + (packed ? 0 : grad ? (size_t)H * nqp : (size_t)H * nqp * rbytes));
         L.total = o;
         return L;
     }
@@ -71,8 +76,8 @@ struct TileShape {
     int64_t key() const {
         return ((((int64_t)(npe * 64 + nqp) * 16 + rbytes * 2 + (grad ? 1 : 0)) * 256 + max_nodes) * 4096 +
                 (int64_t)(budget / 1024)) *
-                   2048 +
-               threads;
+                   4096 +
+               2 * threads + (packed ? 1 : 0);
     }
 };
 
@@ -247,7 +252,8 @@ void prepare_batch_launch(feasm_ctx *ctx, BatchLaunch &b, const std::vector<Batc
 // kernel map to their own id)
 int fused_kernel_form(const FormParams &fp);
 void launch_batch(feasm_ctx *ctx, const BatchLaunch &b);
-TileShape tile_shape_for(feasm_ctx *ctx, int npe, int nqp, int form, int precision);
+// (nodes, kib and threads as in feasm_mesh_set_tile_params, 0 the default)
+TileShape tile_shape_for(feasm_ctx *ctx, int npe, int nqp, int form, int precision, int nodes, int kib, int threads);
 void launch_fused(feasm_ctx *ctx, const feasm_mesh *m, const Pattern &p, const TileSet &t, const DevQTable &qt,
                   const FormParams &fp, int precision, double *nzval);
 

@@ -14,7 +14,7 @@ namespace {
 bool gauss_1d(int order, std::vector<double> &p, std::vector<double> &w) {
     switch (order) {
         case 1: p = {0.0}; w = {2.0}; return true;
-        case 2: p = {-0.577350269189626, 0.577350269189626}; w = {1.0, 1.0}; return true;
+        case 2: p = {-kGauss2, kGauss2}; w = {1.0, 1.0}; return true;
         case 3:
             p = {-0.774596669241483, 0.0, 0.774596669241483};
             w = {0.5555555555555556, 0.8888888888888889, 0.5555555555555556};
