@@ -143,6 +143,7 @@ struct feasm_ctx {
     // reusable scratch for library temporaries (sort/scan storage)
     feasm::DevPtr scratch;
     void *scratch_get(size_t bytes);
+    feasm::DevPtr tile_queue;  // the fused launches' tile queue (fused.hip), on `stream` only
 };
 
 // releases the context when the last reference goes (capi.cpp)

@@ -254,6 +254,39 @@ constexpr int staged_chunks() {
 // memory wait is needed for it.
 __device__ __forceinline__ TileHdr load_hdr(const TileHdr *__restrict__ hdr, int64_t t) { return hdr[t]; }
 
+// A tile header (and in a batched launch the tile's entry) on its way, as words
+// in the lanes of each wavefront: a vector load like the blob's, waited for
+// together with it.  (A scalar load still pending makes every wait for an LDS
+// read wait for it too, and the walk's next header is a new cache line each
+// time.)
+struct StagedHdr {
+    static constexpr int kWords = sizeof(TileHdr) / 4;
+    uint32_t w;
+    __device__ __forceinline__ void issue(const TileHdr *__restrict__ hdr, const int32_t *__restrict__ entry,
+                                          int64_t t) {
+        const int lane = threadIdx.x & 63;
+        const uint32_t *p = reinterpret_cast<const uint32_t *>(hdr + t) + min(lane, kWords - 1);
+        if (entry && lane >= kWords) p = reinterpret_cast<const uint32_t *>(entry + t);
+        w = *p;
+    }
+    __device__ __forceinline__ void ready() const { asm volatile("" ::"v"(w)); }
+    __device__ __forceinline__ uint32_t word(int i) const { return (uint32_t)__builtin_amdgcn_readlane((int)w, i); }
+    __device__ __forceinline__ int32_t entry() const { return (int32_t)word(kWords); }
+    __device__ __forceinline__ TileHdr get() const {
+        TileHdr h;
+        h.P = (int32_t)word(0);
+        h.H = (int32_t)word(1);
+        h.NH = (int32_t)word(2);
+        h.NT = (int32_t)word(3);
+        h.K = (int32_t)word(4);
+        h.NI = (int32_t)word(5);
+        h.x0 = (int32_t)word(6);
+        h.nbytes = (int32_t)word(7);
+        h.blob = (int64_t)((uint64_t)word(8) | ((uint64_t)word(9) << 32));
+        return h;
+    }
+};
+
 template <bool COEF, int NC>
 __device__ __forceinline__ void stage_issue(const TileJob &job, const TileHdr &hd, const double *coef,
                                             Staged<COEF, NC> &st) {
@@ -582,31 +615,81 @@ __device__ __forceinline__ void load_tables(const FusedParams &kp, unsigned char
 }
 
 // XCD-aware persistent walk: consecutive workgroups land on different XCDs,
-// so each XCD takes a contiguous range of the (Morton-ordered) tile list and
-// its workgroups stride through it.
-struct TileRange {
-    int64_t begin, end, step;
+// so each XCD takes a contiguous range of the (Morton-ordered) tile list.  The
+// workgroups stride through the first kAhead tiles each; the rest of a range
+// (queue given: at least kAhead tiles per workgroup) is handed out one tile at
+// a time, and a workgroup whose range has run out goes on with the next one's:
+// tiles differ in time (T10: by a quarter of the mean), and with a fixed stride
+// the last workgroup ended 20 % (T10), 5 % (H8) after the mean.  Measured: H8
+// elasticity, 1M elements 1010 -> 984 us, T10 elasticity, 178k elements 233 ->
+// 216; with fewer than kAhead tiles a workgroup there is nothing to hand out.
+//
+// A workgroup runs tile t, loads the blob of t1, reads the header of t2 and
+// claims the tile after it.  One lane claims: the atomic is issued before phase
+// 1 and its result goes to the other wavefronts through LDS.
+constexpr int kAhead = 3;
+constexpr int kQueuePad = 32;  // words between counters: a cache line each
+struct TileWalk {
+    uint32_t *queue;  // 8 counters, one per XCD's range, and the finished workgroups; null: fixed stride
+    int64_t ntiles;
+    int xcd, slot, slots;
+    int32_t v;         // claiming lane: ranges found empty (fixed stride: tiles claimed)
+    uint32_t claimed;  // claiming lane: the atomic's result
+    __device__ __forceinline__ TileWalk(uint32_t *q, int64_t n)
+        : queue(q), ntiles(n), xcd(blockIdx.x % 8), slot(blockIdx.x / 8), slots(gridDim.x / 8),
+          v(q ? 0 : kAhead - 1), claimed(0) {}
+    __device__ __forceinline__ static bool claimer() { return threadIdx.x == blockDim.x - 64; }
+    __device__ __forceinline__ int64_t range(int x) const { return ntiles * x / 8; }
+    // the workgroup's i-th tile by the stride, -1 if its range has no such tile
+    __device__ __forceinline__ int32_t strided(int i) const {
+        const int64_t t = range(xcd) + slot + (int64_t)i * slots;
+        return t < range(xcd + 1) ? (int32_t)t : -1;
+    }
+    __device__ __forceinline__ void start(int *next) const {
+        if (claimer()) *next = strided(kAhead - 1);
+    }
+    __device__ __forceinline__ void claim() {
+        if (claimer() && queue && v < 8) claimed = atomicAdd(queue + kQueuePad * ((xcd + v) & 7), 1u);
+    }
+    __device__ __forceinline__ void resolve(int *next) {
+        if (!claimer()) return;
+        int32_t t = -1;
+        if (!queue) {
+            t = strided(++v);
+        } else {
+            while (v < 8) {
+                const int x = (xcd + v) & 7;
+                const int64_t i = range(x) + (int64_t)kAhead * slots + claimed;
+                if (i < range(x + 1)) {
+                    t = (int32_t)i;
+                    break;
+                }
+                if (++v < 8) {
+                    claimed = atomicAdd(queue + kQueuePad * ((xcd + v) & 7), 1u);
+                } else if (atomicAdd(queue + kQueuePad * 8, 1u) == gridDim.x - 1) {
+                    // every workgroup has made its last claim: ready for the next launch
+                    for (int k = 0; k <= 8; k++) atomicExch(queue + kQueuePad * k, 0u);
+                }
+            }
+        }
+        *next = t;
+    }
 };
-__device__ __forceinline__ TileRange xcd_range(int64_t ntiles) {
-    const int64_t per = (ntiles + 7) / 8;
-    const int64_t xcd = blockIdx.x % 8, slot = blockIdx.x / 8, nslots = gridDim.x / 8;
-    const int64_t b = xcd * per;
-    const int64_t e = (b + per < ntiles) ? b + per : ntiles;
-    return TileRange{b + slot, e, nslots};
-}
 
 template <int NPE, int NQP, int FORM, int NDN, typename R>
 __global__ __launch_bounds__(kMaxThreads) void k_fused(TileShape shape_, TileJob job,
                                                     const TileHdr *__restrict__ hdr, int64_t ntiles,
-                                                    FusedParams kp) {
+                                                    FusedParams kp, uint32_t *queue) {
     extern __shared__ __align__(16) unsigned char smem[];
     TileShape shape = shape_;
     shape.packed = false;  // known here, so that the layout has no branch for it
-    const TileRange rg = xcd_range(ntiles);
-    if (rg.begin >= rg.end) return;
+    TileWalk walk(queue, ntiles);
+    const int32_t t0 = walk.strided(0);
+    if (t0 < 0) return;
     constexpr int DS = NPE * 3;  // TileShape::dstride()
     double *sD = reinterpret_cast<double *>(smem) + NQP * NPE + NQP * DS;
-    int *sNeg = reinterpret_cast<int *>(sD + 36);
+    int *sNeg = reinterpret_cast<int *>(sD + 36), *sNext = sNeg + 1;
+    walk.start(sNext);
     load_tables<NPE, NQP>(kp, smem);
     for (int i = threadIdx.x; i < 36; i += blockDim.x) sD[i] = kp.fp.coef[i];  // one material per launch
     // Tile t runs while the blob of tile t1 (the next one) is loaded and
@@ -618,42 +701,43 @@ __global__ __launch_bounds__(kMaxThreads) void k_fused(TileShape shape_, TileJob
     // they issue it after phase 1 and wait for it (and the stores) at the
     // next tile (measured faster for them).
     constexpr bool EARLY = (FORM != FEASM_FORM_DOT);
-    int64_t t1 = rg.begin + rg.step;
-    TileHdr hd = load_hdr(hdr, rg.begin);
-    TileHdr hn = load_hdr(hdr, t1 < rg.end ? t1 : rg.begin);
+    int32_t t1 = walk.strided(1);
+    TileHdr hd = load_hdr(hdr, t0);
+    TileHdr hn = load_hdr(hdr, max(t1, 0));
     // (the loads are unconditional, from valid tiles, so that no register
     // copy of a pending load forces an early wait)
     Staged<false, staged_chunks<R, FORM>()> st;
     stage_issue(job, hd, nullptr, st);
     st.ready();
     for (;;) {
-        const bool more = t1 < rg.end;
-        const int64_t t2 = t1 + rg.step;
-        const int64_t i2 = t2 < rg.end ? t2 : rg.begin;
-        // the gradient forms read the header of tile t2 while the blob goes
-        // to LDS: the barrier's wait covers it, and no scalar load is left
-        // pending in the phases (that would turn every wait for an LDS read
-        // into a wait for all of them); the store-bound DOT forms measured
-        // faster with the read after the barrier
-        TileHdr h2;
-        if constexpr (EARLY) h2 = load_hdr(hdr, i2);
+        const bool more = t1 >= 0;
+        StagedHdr sh;  // the header of tile t2
         stage_store(job, hd, st, shape.layout(hd.H, hd.P, hd.NH, hd.K, hd.NT, hd.NI), smem, sD, sNeg);
         __syncthreads();
-        if constexpr (!EARLY) h2 = load_hdr(hdr, i2);
+        const int32_t t2 = __builtin_amdgcn_readfirstlane(*sNext);
         const TileHdr &hb = more ? hn : hd;
-        if constexpr (EARLY) stage_issue(job, hb, nullptr, st);
+        const auto issue = [&]() {
+            sh.issue(hdr, nullptr, max(t2, 0));
+            stage_issue(job, hb, nullptr, st);
+        };
+        walk.claim();
+        if constexpr (EARLY) issue();
         tile_compute<NPE, NQP, FORM, NDN, R, false>(
             shape, job, kp, hd, smem,
             [&]() {
-                if constexpr (!EARLY) stage_issue(job, hb, nullptr, st);
+                if constexpr (!EARLY) issue();
             },
             [&]() {
-                if constexpr (EARLY) st.ready();
+                if constexpr (EARLY) {
+                    sh.ready();
+                    st.ready();
+                }
+                walk.resolve(sNext);
             });
         if (!more) break;
         t1 = t2;
         hd = hn;
-        hn = h2;
+        hn = sh.get();
     }
 }
 
@@ -914,34 +998,42 @@ __device__ __forceinline__ void packed_tile(const TileShape &shape, const TileJo
 template <int NPE, int NQP, int FORM, int NDN, typename R>
 __global__ __launch_bounds__(kPackedThreads, 2) void k_packed(TileShape shape_, TileJob job,
                                                            const TileHdr *__restrict__ hdr, int64_t ntiles,
-                                                           FusedParams kp) {
+                                                           FusedParams kp, uint32_t *queue) {
     static_assert(NPE == 8 && NQP == 8 && NDN == 1 && sizeof(R) == 8);
     extern __shared__ __align__(16) unsigned char smem[];
     TileShape shape = shape_;
     shape.packed = true;
-    const TileRange rg = xcd_range(ntiles);
-    if (rg.begin >= rg.end) return;
+    TileWalk walk(queue, ntiles);
+    const int32_t t0 = walk.strided(0);
+    if (t0 < 0) return;
     double *sD = reinterpret_cast<double *>(smem) + NQP * NPE * 4;
-    int *sNeg = reinterpret_cast<int *>(sD + 36);
-    int64_t t1 = rg.begin + rg.step;
-    TileHdr hd = load_hdr(hdr, rg.begin);
-    TileHdr hn = load_hdr(hdr, t1 < rg.end ? t1 : rg.begin);
+    int *sNeg = reinterpret_cast<int *>(sD + 36), *sNext = sNeg + 1;
+    walk.start(sNext);
+    int32_t t1 = walk.strided(1);
+    TileHdr hd = load_hdr(hdr, t0);
+    TileHdr hn = load_hdr(hdr, max(t1, 0));
     Staged<false, kPackedChunks> st;
     stage_issue(job, hd, nullptr, st);
     st.ready();
     for (;;) {
-        const bool more = t1 < rg.end;
-        const int64_t t2 = t1 + rg.step;
-        const TileHdr h2 = load_hdr(hdr, t2 < rg.end ? t2 : rg.begin);
+        const bool more = t1 >= 0;
+        StagedHdr sh;  // the header of tile t2
         stage_store(job, hd, st, shape.layout(hd.H, hd.P, hd.NH, hd.K, hd.NT, hd.NI), smem, sD, sNeg);
         __syncthreads();
+        const int32_t t2 = __builtin_amdgcn_readfirstlane(*sNext);
+        walk.claim();
+        sh.issue(hdr, nullptr, max(t2, 0));
         stage_issue(job, more ? hn : hd, nullptr, st);  // waited for before this tile's stores
-        packed_tile<FORM, false>(shape, job, kp, hd, smem, [&]() { st.ready(); });
+        packed_tile<FORM, false>(shape, job, kp, hd, smem, [&]() {
+            sh.ready();
+            st.ready();
+            walk.resolve(sNext);
+        });
         if (!more) break;
         __syncthreads();
         t1 = t2;
         hd = hn;
-        hn = h2;
+        hn = sh.get();
     }
 }
 
@@ -961,61 +1053,61 @@ template <int NPE, int NQP, int FORM, int NDN, typename R>
 __global__ __launch_bounds__(kMaxThreads) void k_fused_batch(const BatchEntry *__restrict__ entries,
                                                           const int32_t *__restrict__ tile_entry,
                                                           const TileHdr *__restrict__ hdr, int64_t ntiles,
-                                                          TileShape shape_) {
+                                                          TileShape shape_, uint32_t *queue) {
     extern __shared__ __align__(16) unsigned char smem[];
     TileShape shape = shape_;
     shape.packed = false;  // known here, so that the layout has no branch for it
-    const TileRange rg = xcd_range(ntiles);
-    if (rg.begin >= rg.end) return;
+    TileWalk walk(queue, ntiles);
+    const int32_t t0 = walk.strided(0);
+    if (t0 < 0) return;
     constexpr int DS = NPE * 3;  // TileShape::dstride()
     double *sD = reinterpret_cast<double *>(smem) + NQP * NPE + NQP * DS;
-    int *sNeg = reinterpret_cast<int *>(sD + 36);
-    load_tables<NPE, NQP>(entries[tile_entry[rg.begin]].kp, smem);
+    int *sNeg = reinterpret_cast<int *>(sD + 36), *sNext = sNeg + 1;
+    walk.start(sNext);
+    load_tables<NPE, NQP>(entries[tile_entry[t0]].kp, smem);
     // the tile walk and its loads as in k_fused; every tile also brings its
     // mesh's coefficients
     constexpr bool EARLY = (FORM != FEASM_FORM_DOT);
-    int64_t t1 = rg.begin + rg.step;
-    TileHdr hd = load_hdr(hdr, rg.begin);
-    const BatchEntry *E = entries + tile_entry[rg.begin];
-    const int64_t i1 = t1 < rg.end ? t1 : rg.begin;
-    TileHdr hn = load_hdr(hdr, i1);
-    const BatchEntry *En = entries + tile_entry[i1];
+    int32_t t1 = walk.strided(1);
+    TileHdr hd = load_hdr(hdr, t0);
+    const BatchEntry *E = entries + tile_entry[t0];
+    TileHdr hn = load_hdr(hdr, max(t1, 0));
+    const BatchEntry *En = entries + tile_entry[max(t1, 0)];
     Staged<true, staged_chunks<R, FORM>()> st;
     stage_issue(E->job, hd, E->kp.fp.coef, st);
     st.ready();
     for (;;) {
-        const bool more = t1 < rg.end;
-        const int64_t t2 = t1 + rg.step;
-        const int64_t i2 = t2 < rg.end ? t2 : rg.begin;
-        TileHdr h2;
-        const BatchEntry *E2 = nullptr;
-        if constexpr (EARLY) {
-            h2 = load_hdr(hdr, i2);
-            E2 = entries + tile_entry[i2];
-        }
+        const bool more = t1 >= 0;
+        StagedHdr sh;  // the header and entry of tile t2
         stage_store(E->job, hd, st, shape.layout(hd.H, hd.P, hd.NH, hd.K, hd.NT, hd.NI), smem, sD, sNeg);
         __syncthreads();
-        if constexpr (!EARLY) {
-            h2 = load_hdr(hdr, i2);
-            E2 = entries + tile_entry[i2];
-        }
+        const int32_t t2 = __builtin_amdgcn_readfirstlane(*sNext);
         const TileHdr &hb = more ? hn : hd;
         const BatchEntry *Eb = more ? En : E;
-        if constexpr (EARLY) stage_issue(Eb->job, hb, Eb->kp.fp.coef, st);
+        const auto issue = [&]() {
+            sh.issue(hdr, tile_entry, max(t2, 0));
+            stage_issue(Eb->job, hb, Eb->kp.fp.coef, st);
+        };
+        walk.claim();
+        if constexpr (EARLY) issue();
         tile_compute<NPE, NQP, FORM, NDN, R, true>(
             shape, E->job, E->kp, hd, smem,
             [&]() {
-                if constexpr (!EARLY) stage_issue(Eb->job, hb, Eb->kp.fp.coef, st);
+                if constexpr (!EARLY) issue();
             },
             [&]() {
-                if constexpr (EARLY) st.ready();
+                if constexpr (EARLY) {
+                    sh.ready();
+                    st.ready();
+                }
+                walk.resolve(sNext);
             });
         if (!more) break;
         t1 = t2;
         hd = hn;
         E = En;
-        hn = h2;
-        En = E2;
+        hn = sh.get();
+        En = entries + sh.entry();
     }
 }
 
@@ -1024,42 +1116,48 @@ template <int NPE, int NQP, int FORM, int NDN, typename R>
 __global__ __launch_bounds__(kPackedThreads, 2) void k_packed_batch(const BatchEntry *__restrict__ entries,
                                                                  const int32_t *__restrict__ tile_entry,
                                                                  const TileHdr *__restrict__ hdr, int64_t ntiles,
-                                                                 TileShape shape_) {
+                                                                 TileShape shape_, uint32_t *queue) {
     static_assert(NPE == 8 && NQP == 8 && NDN == 1 && sizeof(R) == 8);
     extern __shared__ __align__(16) unsigned char smem[];
     TileShape shape = shape_;
     shape.packed = true;
-    const TileRange rg = xcd_range(ntiles);
-    if (rg.begin >= rg.end) return;
+    TileWalk walk(queue, ntiles);
+    const int32_t t0 = walk.strided(0);
+    if (t0 < 0) return;
     double *sD = reinterpret_cast<double *>(smem) + NQP * NPE * 4;
-    int *sNeg = reinterpret_cast<int *>(sD + 36);
-    int64_t t1 = rg.begin + rg.step;
-    TileHdr hd = load_hdr(hdr, rg.begin);
-    const BatchEntry *E = entries + tile_entry[rg.begin];
-    const int64_t i1 = t1 < rg.end ? t1 : rg.begin;
-    TileHdr hn = load_hdr(hdr, i1);
-    const BatchEntry *En = entries + tile_entry[i1];
+    int *sNeg = reinterpret_cast<int *>(sD + 36), *sNext = sNeg + 1;
+    walk.start(sNext);
+    int32_t t1 = walk.strided(1);
+    TileHdr hd = load_hdr(hdr, t0);
+    const BatchEntry *E = entries + tile_entry[t0];
+    TileHdr hn = load_hdr(hdr, max(t1, 0));
+    const BatchEntry *En = entries + tile_entry[max(t1, 0)];
     Staged<true, kPackedChunks> st;
     stage_issue(E->job, hd, E->kp.fp.coef, st);
     st.ready();
     for (;;) {
-        const bool more = t1 < rg.end;
-        const int64_t t2 = t1 + rg.step, i2 = t2 < rg.end ? t2 : rg.begin;
-        const TileHdr h2 = load_hdr(hdr, i2);
-        const BatchEntry *E2 = entries + tile_entry[i2];
+        const bool more = t1 >= 0;
+        StagedHdr sh;  // the header and entry of tile t2
         stage_store(E->job, hd, st, shape.layout(hd.H, hd.P, hd.NH, hd.K, hd.NT, hd.NI), smem, sD, sNeg);
         __syncthreads();
+        const int32_t t2 = __builtin_amdgcn_readfirstlane(*sNext);
         const TileHdr &hb = more ? hn : hd;
         const BatchEntry *Eb = more ? En : E;
+        walk.claim();
+        sh.issue(hdr, tile_entry, max(t2, 0));
         stage_issue(Eb->job, hb, Eb->kp.fp.coef, st);
-        packed_tile<FORM, true>(shape, E->job, E->kp, hd, smem, [&]() { st.ready(); });
+        packed_tile<FORM, true>(shape, E->job, E->kp, hd, smem, [&]() {
+            sh.ready();
+            st.ready();
+            walk.resolve(sNext);
+        });
         if (!more) break;
         __syncthreads();
         t1 = t2;
         hd = hn;
         E = En;
-        hn = h2;
-        En = E2;
+        hn = sh.get();
+        En = entries + sh.entry();
     }
 }
 
@@ -1086,6 +1184,22 @@ unsigned persistent_grid(feasm_ctx *ctx, size_t budget, int64_t ntiles) {
     return (unsigned)std::min(grid, std::max<int64_t>(need, 8));
 }
 
+// A launch leaves its queue cleared for the next one, so launches that share
+// one must run one after the other: those on the context's stream do.  A launch
+// recorded into a graph may be replayed on another stream, beside the next
+// one: it gets none and walks with the fixed stride.
+constexpr size_t kQueueBytes = sizeof(uint32_t) * kQueuePad * 9;
+uint32_t *ctx_tile_queue(feasm_ctx *ctx) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    FEASM_HIP(hipStreamIsCapturing(ctx->stream, &cs));
+    if (cs != hipStreamCaptureStatusNone) return nullptr;
+    if (!ctx->tile_queue) {
+        ctx->tile_queue = dev_alloc(kQueueBytes);
+        FEASM_HIP(hipMemsetAsync(ctx->tile_queue->p, 0, kQueueBytes, ctx->stream));
+    }
+    return dp<uint32_t>(ctx->tile_queue);
+}
+
 template <int NPE, int NQP, int FORM, int NDN, typename R>
 void go(feasm_ctx *ctx, const feasm_mesh *m, const Pattern &p, const TileSet &t, const FusedParams &kp,
         double *nzval) {
@@ -1100,8 +1214,9 @@ void go(feasm_ctx *ctx, const feasm_mesh *m, const Pattern &p, const TileSet &t,
     FEASM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, budget));
     const unsigned grid = persistent_grid(ctx, t.shape.budget, t.ntiles);
     TileJob job = make_job(m, t, nzval);
+    uint32_t *queue = t.ntiles >= (int64_t)kAhead * grid ? ctx_tile_queue(ctx) : nullptr;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(t.shape.threads), budget, ctx->stream, t.shape, job, job.hdr, t.ntiles,
-                       kp);
+                       kp, queue);
     FEASM_HIP(hipGetLastError());
 }
 
@@ -1143,7 +1258,8 @@ void go_batch(feasm_ctx *ctx, const BatchLaunch &b) {
     FEASM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b.budget));
     hipLaunchKernelGGL(kern, dim3(b.grid), dim3(b.threads), b.budget, ctx->stream,
                        static_cast<const BatchEntry *>(b.entries->p), dp<int32_t>(b.tile_entry),
-                       static_cast<const TileHdr *>(b.hdr->p), b.ntiles, b.shape);
+                       static_cast<const TileHdr *>(b.hdr->p), b.ntiles, b.shape,
+                       b.queue ? dp<uint32_t>(b.queue) : nullptr);
     FEASM_HIP(hipGetLastError());
 }
 
@@ -1185,6 +1301,10 @@ void prepare_batch_launch(feasm_ctx *ctx, BatchLaunch &b, const std::vector<Batc
         FEASM_HIP(hipMemcpy(static_cast<TileHdr *>(b.hdr->p) + host[i].tile0, items[i].tiles->hdr->p,
                             (size_t)items[i].tiles->ntiles * sizeof(TileHdr), hipMemcpyDeviceToDevice));
     b.grid = persistent_grid(ctx, b.budget, b.ntiles);
+    if (b.ntiles >= (int64_t)kAhead * b.grid) {
+        b.queue = dev_alloc(kQueueBytes);
+        FEASM_HIP(hipMemset(b.queue->p, 0, kQueueBytes));
+    }
 }
 
 namespace {

@@ -245,6 +245,9 @@ struct BatchLaunch {
     size_t budget = 0;
     unsigned grid = 0;
     DevPtr entries, tile_entry, hdr;  // hdr: the tiles' headers, mesh after mesh
+    // the launch's own tile queue (none when there are few tiles): its runs,
+    // and the replays of its graph, write the same matrices one after the other
+    DevPtr queue;
     TileShape shape;  // the meshes' tile layout (npe, nqp, rbytes and grad agree)
 };
 void prepare_batch_launch(feasm_ctx *ctx, BatchLaunch &b, const std::vector<BatchMesh> &items);
