@@ -102,6 +102,8 @@ struct QTable {
 QTable make_qtable(int etype, int rule, int order);  // tables.cpp
 // the point of the reference's two-point Gauss rule (src/IntegRuleModule.jl:211)
 constexpr double kGauss2 = 0.577350269189626;
+// coordinates of its four-point tetrahedron rule (src/IntegRuleModule.jl:488-493)
+constexpr double kTet4Lo = 0.13819660, kTet4Hi = 0.58541020;
 
 // Device copy of a QTable, one contiguous buffer: [N | dN | w].
 struct DevQTable {

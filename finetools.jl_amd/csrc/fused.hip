@@ -317,6 +317,172 @@ __device__ __forceinline__ void stage_store(const TileJob &job, const TileHdr &h
     if (tid == 0) *sNeg = 0;
 }
 
+// Phase 1 in FP64: the lanes of an element's points share its coordinates.
+// The 8 points of the H8 Gauss rule and the 4 of the T10 rule lie each beside a
+// corner of their own, so the element looks the same from every point once its
+// corners are named from there: corner m of point q is corner q ^ m (H8:
+// reflected, one bit per direction; T10: permuted, always evenly).  Lane q reads
+// its own corner (T10: and that corner's edges), the sums over the others are
+// lane exchanges, and the basis values are the same constants in every lane.
+// Phase 1 waits for LDS: a thread that sums over all nodes makes 48 (H8) or 40
+// (T10) reads, half of them of scattered coordinates; this one makes 2 or 8.  It
+// takes 3500 instead of 7200 of an H8 tile's cycles (T10: 3400 for 8500); H8
+// elasticity, 1M elements 985 -> 936 us, T10, 178k elements 217 -> 212.  The
+// FP32 kernels read the tables: their values would not stay the same.
+
+// the value of lane (lane ^ M), M < 8, in a group of 8 whose lanes all run
+template <int M>
+__device__ __forceinline__ double lane_swap(double v) {
+    const auto word = [](int x) {
+        if constexpr (M >= 4) x = __builtin_amdgcn_mov_dpp(x, 0x141, 0xF, 0xF, false);  // row_half_mirror: lane ^ 7
+        constexpr int q = M >= 4 ? M ^ 7 : M;
+        if constexpr (q == 1) x = __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, false);  // quad_perm [1,0,3,2]
+        if constexpr (q == 2) x = __builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, false);  // quad_perm [2,3,0,1]
+        if constexpr (q == 3) x = __builtin_amdgcn_mov_dpp(x, 0x1B, 0xF, 0xF, false);  // quad_perm [3,2,1,0]
+        return x;
+    };
+    return __hiloint2double(word(__double2hiint(v)), word(__double2loint(v)));
+}
+
+__device__ __forceinline__ double det3(const double (&a)[3], const double (&b)[3], const double (&c)[3]) {
+    return a[0] * (b[1] * c[2] - b[2] * c[1]) + a[1] * (b[2] * c[0] - b[0] * c[2]) + a[2] * (b[0] * c[1] - b[1] * c[0]);
+}
+
+struct H8Point {
+    static constexpr int kNodes = 8, kPoints = 8;
+    static constexpr double lo = 0.5 * (1.0 - kGauss2), hi = 0.5 * (1.0 + kGauss2);
+    int q;
+    // local node of corner c = 4 i + 2 j + k (bit 1: the + side)
+    __device__ __forceinline__ static int node(int c) { return (int)(0x62517340u >> (4 * c)) & 7; }
+    // columns of the Jacobian along each direction, from this corner towards
+    // the other (2 J times -1 on the + side); returns det J
+    __device__ __forceinline__ double jacobian(const uint16_t *cn, const double2 *sXY, const double *sZ,
+                                               double (&j1)[3], double (&j2)[3], double (&j3)[3], double &det) {
+        const int n = (int)cn[node(q)];
+        const double2 xy = sXY[n];
+        const double x[3] = {xy.x, xy.y, sZ[n]};
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const double xi = lane_swap<4>(x[c]);
+            const double d = xi - x[c], v = hi * x[c] + lo * xi;  // derivative and value along xi
+            const double dj = lane_swap<2>(d), vj = lane_swap<2>(v);
+            const double dv = hi * d + lo * dj, vd = vj - v, vv = hi * v + lo * vj;  // and along eta
+            j1[c] = hi * dv + lo * lane_swap<1>(dv);
+            j2[c] = hi * vd + lo * lane_swap<1>(vd);
+            j3[c] = lane_swap<1>(vv) - vv;
+        }
+        det = det3(j1, j2, j3);
+        return (__popc(q) & 1) ? -0.125 * det : 0.125 * det;
+    }
+    // put(a, u) for every node a: its gradient in terms of the inverse's rows
+    template <typename Put>
+    __device__ __forceinline__ void gradients(const double (&r1)[3], const double (&r2)[3], const double (&r3)[3],
+                                              const Put &put) const {
+#pragma unroll
+        for (int m = 0; m < 8; m++) {
+            const double n1 = (m & 4) ? lo : hi, n2 = (m & 2) ? lo : hi, n3 = (m & 1) ? lo : hi;
+            const double d1 = (m & 4) ? n2 * n3 : -n2 * n3, d2 = (m & 2) ? n1 * n3 : -n1 * n3,
+                         d3 = (m & 1) ? n1 * n2 : -n1 * n2;
+            double u[3];
+#pragma unroll
+            for (int c = 0; c < 3; c++) u[c] = d1 * r1[c] + d2 * r2[c] + d3 * r3[c];
+            put(node(q ^ m), u);
+        }
+    }
+};
+
+struct T10Point {
+    static constexpr int kNodes = 10, kPoints = 4;
+    static constexpr double lo = kTet4Lo, hi = kTet4Hi;
+    int q, e[3];  // e: the edges from corner q to the corners q ^ 1, q ^ 2, q ^ 3
+    // columns of the Jacobian: the derivatives along the barycentric
+    // coordinates of the corners q ^ 1, q ^ 2, q ^ 3, less corner q's
+    __device__ __forceinline__ double jacobian(const uint16_t *cn, const double2 *sXY, const double *sZ,
+                                               double (&j1)[3], double (&j2)[3], double (&j3)[3], double &det) {
+        e[0] = (q & 2) ? 9 : 4;
+        e[1] = (q & 1) ? 8 : 6;
+        e[2] = (q == 1 || q == 2) ? 5 : 7;
+        const int n = (int)cn[q], n1 = (int)cn[e[0]], n2 = (int)cn[e[1]], n3 = (int)cn[e[2]];
+        const double2 p = sXY[n], p1 = sXY[n1], p2 = sXY[n2], p3 = sXY[n3];
+        const double x[3] = {p.x, p.y, sZ[n]}, x1[3] = {p1.x, p1.y, sZ[n1]}, x2[3] = {p2.x, p2.y, sZ[n2]},
+                     x3[3] = {p3.x, p3.y, sZ[n3]};
+        // along corner c: E_c + 4 (hi - lo) x(edge c q), E_c the lane's own
+        // corner at lo; along q itself E_q + 4 (hi - lo) x_q
+        constexpr double g = 4.0 * (hi - lo);
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const double E = (4.0 * lo - 1.0) * x[c] + 4.0 * lo * ((x1[c] + x2[c]) + x3[c]);
+            j1[c] = (lane_swap<1>(E) - E) + g * (x1[c] - x[c]);
+            j2[c] = (lane_swap<2>(E) - E) + g * (x2[c] - x[c]);
+            j3[c] = (lane_swap<3>(E) - E) + g * (x3[c] - x[c]);
+        }
+        det = det3(j1, j2, j3);
+        return det;
+    }
+    template <typename Put>
+    __device__ __forceinline__ void gradients(const double (&r1)[3], const double (&r2)[3], const double (&r3)[3],
+                                              const Put &put) const {
+        double t[3];
+#pragma unroll
+        for (int c = 0; c < 3; c++) t[c] = -((r1[c] + r2[c]) + r3[c]);  // corner q's own coordinate
+        const auto corner = [&](int a, double s, const double (&v)[3]) {
+            const double u[3] = {s * v[0], s * v[1], s * v[2]};
+            put(a, u);
+        };
+        const auto edge = [&](int a, double s, const double (&v)[3], const double (&w)[3]) {
+            const double u[3] = {s * v[0] + 4.0 * lo * w[0], s * v[1] + 4.0 * lo * w[1], s * v[2] + 4.0 * lo * w[2]};
+            put(a, u);
+        };
+        corner(q, 4.0 * hi - 1.0, t);
+        corner(q ^ 1, 4.0 * lo - 1.0, r1);
+        corner(q ^ 2, 4.0 * lo - 1.0, r2);
+        corner(q ^ 3, 4.0 * lo - 1.0, r3);
+        edge(e[0], 4.0 * hi, r1, t);
+        edge(e[1], 4.0 * hi, r2, t);
+        edge(e[2], 4.0 * hi, r3, t);
+        // the edges that do not meet corner q, each opposite one that does
+        edge(13 - e[0], 4.0 * lo, r2, r3);
+        edge(14 - e[1], 4.0 * lo, r1, r3);
+        edge(12 - e[2], 4.0 * lo, r1, r2);
+    }
+};
+
+template <typename P, int FORM>
+__device__ __forceinline__ void point_fp64(int h, int q, const uint16_t *sLc, const double *sX, int NH,
+                                           const double *sWq, const double *coef, double *sU, uint8_t *sSg, double *sW,
+                                           int *sNeg) {
+    constexpr int NPE = P::kNodes, NQP = P::kPoints;
+    P pt;
+    pt.q = q;
+    double j1[3], j2[3], j3[3], det;
+    const double detJ = pt.jacobian(sLc + h * NPE, reinterpret_cast<const double2 *>(sX), sX + 2 * NH, j1, j2, j3, det);
+    const double wj = (FORM == FEASM_FORM_DIFFUSION_ISO) ? (coef[0] * detJ) * sWq[q] : detJ * sWq[q];
+    if constexpr (FORM == FEASM_FORM_DOT) {
+        sW[h * NQP + q] = wj;
+    } else {
+        sSg[h * NQP + q] = (wj < 0.0) ? 1 : 0;
+        if (wj < 0.0) atomicOr(sNeg, 1);
+        // the inverse scaled by sqrt(|J w|) once: its rows are the cross
+        // products of the columns
+        const double s = (1.0 / det) * sqrt(fabs(wj));
+        const double r1[3] = {(j2[1] * j3[2] - j2[2] * j3[1]) * s, (j2[2] * j3[0] - j2[0] * j3[2]) * s,
+                              (j2[0] * j3[1] - j2[1] * j3[0]) * s};
+        const double r2[3] = {(j3[1] * j1[2] - j3[2] * j1[1]) * s, (j3[2] * j1[0] - j3[0] * j1[2]) * s,
+                              (j3[0] * j1[1] - j3[1] * j1[0]) * s};
+        const double r3[3] = {(j1[1] * j2[2] - j1[2] * j2[1]) * s, (j1[2] * j2[0] - j1[0] * j2[2]) * s,
+                              (j1[0] * j2[1] - j1[1] * j2[0]) * s};
+        // the element's record of 16-byte chunks (TileShape::uchunks): (u0, u1)
+        // of point q in xy chunk q, u2 in z chunk q / 2
+        double2 *const rec = reinterpret_cast<double2 *>(sU) + (size_t)h * (NPE * NQP * 3 / 2 + 1);
+        double2 *const xy = rec + q * NPE;
+        double *const zz = reinterpret_cast<double *>(rec + NQP * NPE + (q >> 1) * NPE) + (q & 1);
+        pt.gradients(r1, r2, r3, [&](int a, const double (&u)[3]) {
+            xy[a] = make_double2(u[0], u[1]);
+            zz[2 * a] = u[2];
+        });
+    }
+}
+
 // One tile, phases 1 and 2, with its image already in LDS.  `after_phase1`
 // runs between the phases; `before_stores` in phase 2, before the first
 // global store of every thread.  LDSCOEF: the scalar material coefficients
@@ -356,6 +522,13 @@ __device__ __forceinline__ void tile_compute(const TileShape &shape, const TileJ
     // ---- phase 1: Jacobians, inverses and scaled gradients
     for (int task = tid; task < H * NQP; task += kThreads) {
         const int h = task / NQP, q = task % NQP;
+        if constexpr (sizeof(R) == 8) {
+            using P = typename std::conditional<NPE == 8, H8Point, T10Point>::type;
+            static_assert(P::kNodes == NPE && P::kPoints == NQP, "one lane per corner");
+            point_fp64<P, FORM>(h, q, sLc, sX, NH, sWq, coef, reinterpret_cast<double *>(sU), sSg,
+                                reinterpret_cast<double *>(sW), sNeg);
+            continue;
+        }
         const uint16_t *cn = sLc + h * NPE;
         // coordinates: (x, y) pairs then z values; gradient table: (d0, d1)
         // pairs then d2 values; nodes visited in an order rotated by the
@@ -366,11 +539,6 @@ __device__ __forceinline__ void tile_compute(const TileShape &shape, const TileJ
         const double2 *dxy = reinterpret_cast<const double2 *>(sDN) + q * NPE;
         const double *dz = sDN + 2 * NQP * NPE + q * NPE;
         double J[9];
-        // FP64: the point's gradient table, read once (the stores of the
-        // scaled gradients below could alias it, so a second read would be
-        // reloaded); measured no faster for FP32, whose kernels keep the reload
-        constexpr bool TQ = sizeof(R) == 8;
-        double tq[TQ ? 3 * NPE : 1];
 #pragma unroll
         for (int i = 0; i < 9; i++) J[i] = 0.0;
 #pragma unroll
@@ -381,11 +549,6 @@ __device__ __forceinline__ void tile_compute(const TileShape &shape, const TileJ
             const double x0 = xy.x, x1 = xy.y, x2 = sZ[n];
             const double2 dd = dxy[a];
             const double d0 = dd.x, d1 = dd.y, d2 = dz[a];
-            if constexpr (TQ) {
-                tq[3 * i] = d0;
-                tq[3 * i + 1] = d1;
-                tq[3 * i + 2] = d2;
-            }
             J[0] += x0 * d0; J[1] += x0 * d1; J[2] += x0 * d2;
             J[3] += x1 * d0; J[4] += x1 * d1; J[5] += x1 * d2;
             J[6] += x2 * d0; J[7] += x2 * d1; J[8] += x2 * d2;
@@ -421,17 +584,8 @@ __device__ __forceinline__ void tile_compute(const TileShape &shape, const TileJ
 #pragma unroll
             for (int i = 0; i < NPE; i++) {
                 const int a = (i + q) % NPE;
-                R d0, d1, d2;
-                if constexpr (TQ) {
-                    d0 = tq[3 * i];
-                    d1 = tq[3 * i + 1];
-                    d2 = tq[3 * i + 2];
-                } else {
-                    const double2 dd = dxy[a];
-                    d0 = (R)dd.x;
-                    d1 = (R)dd.y;
-                    d2 = (R)dz[a];
-                }
+                const double2 dd = dxy[a];
+                const R d0 = (R)dd.x, d1 = (R)dd.y, d2 = (R)dz[a];
                 const R u0 = d0 * ivr[0] + d1 * ivr[3] + d2 * ivr[6];
                 const R u1 = d0 * ivr[1] + d1 * ivr[4] + d2 * ivr[7];
                 const R u2 = d0 * ivr[2] + d1 * ivr[5] + d2 * ivr[8];

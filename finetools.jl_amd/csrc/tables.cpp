@@ -48,7 +48,7 @@ void rule_points(int rule, int order, std::vector<double> &pc, std::vector<doubl
         pc = {0.25, 0.25, 0.25};
         w = {1.0 / 6.0};
     } else if (order == 4) {
-        const double lo = 0.13819660, hi = 0.58541020;
+        const double lo = kTet4Lo, hi = kTet4Hi;
         pc = {lo, lo, lo, hi, lo, lo, lo, hi, lo, lo, lo, hi};
         w.assign(4, 0.041666666666666666667);
     } else if (order == 5) {
