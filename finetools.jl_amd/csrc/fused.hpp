@@ -108,6 +108,27 @@ constexpr uint16_t kNoPair = 0xffff;
 // room for them)
 constexpr int kPadTasks = 320;
 
+// Order of a tile's block tasks (k elements each, K the most): the symmetric
+// diagonal blocks first, then the others, the longest first in each kind.
+__host__ __device__ inline int task_order(int k, bool sym, int K) { return (sym ? 0 : K + 1) + (K - k); }
+// The chunks of 64 tasks that run as one wavefront: [0, nsym) and [nsym, nt)
+// are cut up separately (nsym = 0 where the kernel has no shorter sum for the
+// symmetric blocks).  A wavefront that held both kinds ran both sums in turn:
+// 8 symmetric and 4 other elements of H8 in 9900 cycles, the longest of the
+// tile by 2600, with half its lanes idle in each (apart: T10 elasticity 212 ->
+// 202 us, H8 936 -> 930, a batch of mixed-precision meshes 221 -> 216).
+struct TaskChunk {
+    int begin, end;
+};
+__host__ __device__ inline int task_chunks(int nsym, int nt) { return (nsym + 63) / 64 + (nt - nsym + 63) / 64; }
+__host__ __device__ inline TaskChunk task_chunk(int ch, int nsym, int nt) {
+    const int ns = (nsym + 63) / 64, b = ch < ns ? ch * 64 : nsym + (ch - ns) * 64, lim = ch < ns ? nsym : nt;
+    return {b, b + 64 < lim ? b + 64 : lim};
+}
+// a wavefront's time by its longest task, in elements: the material and store
+// work counts as two
+__host__ __device__ inline double task_cost(int k, bool sym) { return (sym ? 0.5 : 1.0) * k + 2.0; }
+
 struct TileSet {
     TileShape shape;
     int64_t ntiles = 0, nhalo = 0, ntasks = 0, nitems = 0, blob_bytes = 0;

@@ -334,14 +334,14 @@ void make_tile(const HostMesh &h, const int32_t *owned, int P, const TileShape &
         for (int j = 0; T.sym && j < T.k; j++)
             if (((its[T.off + j] >> 4) & 15u) != (its[T.off + j] & 15u)) T.sym = false;
     }
-    // longest first; among equal counts the symmetric diagonal blocks first,
-    // so that they fill wavefronts of their own (a stable counting sort on
-    // (k, sym): the order of std::stable_sort by that key)
+    // longest first, the symmetric diagonal blocks before all others (see
+    // task_order; a stable counting sort: the order of std::stable_sort by
+    // that key)
     int K = 0;
     for (const Task &T : tasks) K = std::max(K, T.k);
     FEASM_REQUIRE(K <= 255, FEASM_EUNSUPPORTED, "a node block is shared by more than 255 elements");
     {
-        auto bucket = [K](const Task &T) { return 2 * (K - T.k) + (T.sym ? 0 : 1); };
+        auto bucket = [K](const Task &T) { return task_order(T.k, T.sym, K); };
         std::vector<int> start(2 * K + 3, 0);
         for (const Task &T : tasks) start[bucket(T) + 1]++;
         for (size_t b = 1; b < start.size(); b++) start[b] += start[b - 1];
@@ -351,19 +351,24 @@ void make_tile(const HostMesh &h, const int32_t *owned, int P, const TileShape &
     }
     o.K = K;
     // Wavefront schedule: 64 consecutive tasks run as one wavefront, and the
-    // wavefronts of a workgroup go to the 4 SIMDs in turn.  Chunks of 64
-    // tasks of equal element count (costed by that count plus the material
-    // and store work) are dealt to the SIMDs longest first, each to the least
-    // loaded one; chunk slots a SIMD does not use are filled with null tasks.
+    // wavefronts of a workgroup go to the 4 SIMDs in turn.  Chunks of up to 64
+    // tasks of one kind (see task_chunk; costed by task_cost of the longest)
+    // are dealt to the SIMDs in order, each to the least loaded one; chunk
+    // slots a SIMD does not use are filled with null tasks.
     constexpr int W = 64, NS = 4;
+    const int nt = (int)tasks.size();
+    int nsym = 0;
+    for (const Task &T : tasks) nsym += T.sym;
+    if (!shape.grad) nsym = 0;
+    const int nch = task_chunks(nsym, nt);
     std::vector<std::vector<int>> queue(NS);
     {
         std::vector<double> load(NS, 0.0);
-        for (size_t c0 = 0; c0 < tasks.size(); c0 += W) {
-            const double cost = (double)tasks[c0].k + 2.0;
+        for (int ch = 0; ch < nch; ch++) {
+            const Task &T = tasks[task_chunk(ch, nsym, nt).begin];
             const int q = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-            queue[q].push_back((int)c0);
-            load[q] += cost;
+            queue[q].push_back(ch);
+            load[q] += task_cost(T.k, T.sym);
         }
     }
     size_t rounds = 0;
@@ -371,7 +376,7 @@ void make_tile(const HostMesh &h, const int32_t *owned, int P, const TileShape &
     if (rounds * NS * W > tasks.size() + kPadTasks) {  // too much padding: plain order
         for (auto &q : queue) q.clear();
         int i = 0;
-        for (size_t c0 = 0; c0 < tasks.size(); c0 += W, i++) queue[i % NS].push_back((int)c0);
+        for (; i < nch; i++) queue[i % NS].push_back(i);
         rounds = 0;
         for (auto &q : queue) rounds = std::max(rounds, q.size());
     }
@@ -385,10 +390,11 @@ void make_tile(const HostMesh &h, const int32_t *owned, int P, const TileShape &
     o.item.reserve(its.size());
     for (size_t rr = 0; rr < rounds; rr++)
         for (int q = 0; q < NS; q++) {
-            const int c0 = rr < queue[q].size() ? queue[q][rr] : -1;
+            TaskChunk ck{0, 0};
+            if (rr < queue[q].size()) ck = task_chunk(queue[q][rr], nsym, nt);
             for (int l = 0; l < W; l++) {
-                const size_t t = (size_t)c0 + l;
-                if (c0 < 0 || t >= tasks.size()) {
+                const int t = ck.begin + l;
+                if (t >= ck.end) {
                     o.task.push_back(kNullTask);
                     o.toff.push_back(0);
                     o.tpair.push_back(kNoPair);

@@ -521,7 +521,7 @@ __host__ __device__ inline BuildLds build_lds(const BuildCaps &c, int npe) {
     BuildLds B;
     size_t o = 0;
     const size_t ns = (size_t)c.ntu + kSlotsExtra;  // schedule slots
-    const size_t nch = (size_t)c.ntu / 64 + 2;       // chunks of 64 tasks
+    const size_t nch = (size_t)c.ntu / 64 + 3;       // chunks of up to 64 tasks
     const size_t nsg = nch + 8;                      // slot groups
     B.word = bl_take(o, (size_t)c.ntu * 4);
     B.tpair = bl_take(o, (size_t)c.ntu * 2);
@@ -581,7 +581,7 @@ __device__ int merge_halo(const uint32_t *keys, const uint16_t *nptr, int ja, in
 // the stable-sort key of a kept task: longest first, the symmetric diagonal
 // blocks first among equal counts
 __device__ __forceinline__ int task_bucket(uint32_t w, int K) {
-    return 2 * (K - (int)((w >> 16) & 255u)) + (((w >> 26) & 1u) ? 0 : 1);
+    return task_order((int)((w >> 16) & 255u), (w >> 26) & 1u, K);
 }
 
 constexpr uint32_t kDropBit = 1u << 27;  // builder-internal: computed by the transposed block's task
@@ -791,6 +791,8 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
     }
     __syncthreads();
     const int NTk = (int)block_excl_scan(bcount, nb, L.part);
+    const int nsym = shape.grad ? (int)bcount[K + 1] : 0;
+    __syncthreads();
     // each bucket's tasks in task order, one wavefront per bucket
     for (int b = wave; b < nb; b += kTB / 64) {
         uint32_t pos = bcount[b];
@@ -806,20 +808,22 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
     __syncthreads();
     mark(4);
 
-    // wavefront schedule: chunks of 64 sorted tasks dealt to the 4 SIMDs,
-    // the costliest first, each to the least loaded (first on ties); plain
-    // order when that needs more than kPadTasks null tasks
-    const int nch = (NTk + 63) / 64;
+    // wavefront schedule: the chunks dealt to the 4 SIMDs in order, each to
+    // the least loaded (first on ties); plain order when that needs more than
+    // kPadTasks null tasks
+    const int nch = task_chunks(nsym, NTk);
     for (int ch = tid; ch < nch; ch += kTB) {
+        const TaskChunk ck = task_chunk(ch, nsym, NTk);
         uint32_t sum = 0;
-        for (int i = ch * 64; i < min(NTk, ch * 64 + 64); i++) sum += (word[sorted[i]] >> 16) & 255u;
+        for (int i = ck.begin; i < ck.end; i++) sum += (word[sorted[i]] >> 16) & 255u;
         csum[ch] = sum;
     }
     if (tid == 0) {
         double load[4] = {0.0, 0.0, 0.0, 0.0};
         int qn[4] = {0, 0, 0, 0};
         for (int ch = 0; ch < nch; ch++) {
-            const double cost = (double)((word[sorted[ch * 64]] >> 16) & 255u) + 2.0;
+            const uint32_t w = word[sorted[task_chunk(ch, nsym, NTk).begin]];
+            const double cost = task_cost((int)((w >> 16) & 255u), (w >> 26) & 1u);
             int q = 0;
             for (int i = 1; i < 4; i++)
                 if (load[i] < load[q]) q = i;
@@ -842,7 +846,8 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
     __syncthreads();
     for (int ch = tid; ch < nch; ch += kTB) {
         qtab[cq[ch]] = ch;
-        atomicMax(&sh_NT, cq[ch] * 64 + min(64, NTk - ch * 64));
+        const TaskChunk ck = task_chunk(ch, nsym, NTk);
+        atomicMax(&sh_NT, cq[ch] * 64 + ck.end - ck.begin);
     }
     __syncthreads();
     if (tid == 0) {  // item offsets of the slot groups
@@ -876,8 +881,10 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
     // task records and items, one slot group per wavefront
     for (int sg = wave; sg < nsg; sg += kTB / 64) {
         const int ch = qtab[sg];
-        const int idx = ch * 64 + lane;
-        const bool valid = ch >= 0 && idx < NTk;
+        TaskChunk ck{0, 0};
+        if (ch >= 0) ck = task_chunk(ch, nsym, NTk);
+        const int idx = ck.begin + lane;
+        const bool valid = idx < ck.end;
         const int u = valid ? sorted[idx] : 0;
         const uint32_t w = valid ? word[u] : 0u;
         const uint32_t k = (w >> 16) & 255u;
