@@ -64,15 +64,18 @@ enum : unsigned {
 };
 
 // LDS of one box evaluation (sorting buffer, halo lists, owned nodes)
-struct EvalLds {
-    uint32_t buf[kMaxBoxCand];
-    int32_t hn[kMaxHaloNodes + 2];
+struct EvalCore {
     int32_t halo[256];
     int32_t owned[256];
     uint32_t coff[260];
     uint32_t part[kTB + 1];
     int sk;
     unsigned long long snt;
+};
+// ... with the sorting buffer and the halo nodes of any box
+struct EvalLds : EvalCore {
+    uint32_t buf[kMaxBoxCand];
+    int32_t hn[kMaxHaloNodes + 2];
 };
 
 // ---- workgroup primitives (blockDim.x == kTB)
@@ -272,7 +275,7 @@ __device__ __forceinline__ int lower_bound_i32(const int32_t *a, int n, int32_t 
 // halo elements and, when H fits, the sorted halo nodes.  All threads of the
 // workgroup call it and get the same answer.
 __device__ bool eval_box(const MeshView &mv, const int32_t *order, int64_t s0, int P, const TileShape &shape,
-                         EvalLds &L, BoxSizes &bs) {
+                         EvalCore &L, uint32_t *buf, int32_t *hn, BoxSizes &bs) {
     const int t = threadIdx.x;
     if (t == 0) {
         L.sk = 0;
@@ -303,25 +306,25 @@ __device__ bool eval_box(const MeshView &mv, const int32_t *order, int64_t s0, i
         const int64_t q0 = mv.n2e_ptr[v];
         const int d = (int)(mv.n2e_ptr[v + 1] - q0);
         const uint32_t o = L.coff[t];
-        for (int j = 0; j < d; j++) L.buf[o + j] = mv.n2e[q0 + j] >> 4;
+        for (int j = 0; j < d; j++) buf[o + j] = mv.n2e[q0 + j] >> 4;
     }
     int n2 = 2;
     while (n2 < (int)cand) n2 <<= 1;
-    for (int i = (int)cand + t; i < n2; i += kTB) L.buf[i] = 0xffffffffu;
+    for (int i = (int)cand + t; i < n2; i += kTB) buf[i] = 0xffffffffu;
     __syncthreads();
-    block_sort(L.buf, n2);
+    block_sort(buf, n2);
     const int hmax = min(shape.max_halo, 255);
-    const int H = block_unique(L.buf, (int)cand, L.halo, hmax, L.part);
+    const int H = block_unique(buf, (int)cand, L.halo, hmax, L.part);
     bs.H = H;
     if (H > hmax) return false;
     const int nc = H * mv.npe;
-    for (int i = t; i < nc; i += kTB) L.buf[i] = (uint32_t)mv.conn[(int64_t)L.halo[i / mv.npe] * mv.npe + i % mv.npe];
+    for (int i = t; i < nc; i += kTB) buf[i] = (uint32_t)mv.conn[(int64_t)L.halo[i / mv.npe] * mv.npe + i % mv.npe];
     n2 = 2;
     while (n2 < nc) n2 <<= 1;
-    for (int i = nc + t; i < n2; i += kTB) L.buf[i] = 0xffffffffu;
+    for (int i = nc + t; i < n2; i += kTB) buf[i] = 0xffffffffu;
     __syncthreads();
-    block_sort(L.buf, n2);
-    bs.NH = block_unique(L.buf, nc, L.hn, kMaxHaloNodes, L.part);
+    block_sort(buf, n2);
+    bs.NH = block_unique(buf, nc, hn, kMaxHaloNodes, L.part);
     return box_fits(shape, bs);
 }
 
@@ -399,7 +402,7 @@ __global__ __launch_bounds__(kTB) void k_part_level(const int64_t *in, int64_t *
         const int64_t P = s1 - s0;
         bool fits = false;
         BoxSizes bs;
-        if (P <= box_max_nodes(shape)) fits = eval_box(mv, order, s0, (int)P, shape, L, bs);
+        if (P <= box_max_nodes(shape)) fits = eval_box(mv, order, s0, (int)P, shape, L, L.buf, L.hn, bs);
         if (threadIdx.x == 0) {
             if (fits) {
                 start[s0] = 1;
@@ -439,7 +442,7 @@ __global__ void k_tile_starts(const uint8_t *start, const int32_t *inc, int64_t 
 // per tile: halo-node count and slot size (for the scans), maxima for the
 // build kernel's LDS
 struct PrepStats {
-    unsigned long long ntu_max, niu_max, k_max;
+    unsigned long long ntu_max, niu_max, k_max, h_max, nh_max, p_max;
 };
 
 // largest of v over the workgroup (256 threads), added to *out with one atomic
@@ -467,7 +470,7 @@ __device__ void block_sum_to(unsigned long long v, unsigned long long *out, unsi
 __global__ __launch_bounds__(256) void k_tile_prep(const int64_t *ts, int64_t ntiles, const int64_t *info,
                                                    TileShape shape, int64_t *nh, int64_t *slot, PrepStats *st) {
     __shared__ unsigned long long sh[256];
-    unsigned long long ntu = 0, niu = 0, km = 0;
+    unsigned long long ntu = 0, niu = 0, km = 0, hm = 0, nhm = 0, pm = 0;
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t <= ntiles; t += (int64_t)gridDim.x * blockDim.x) {
         if (t == ntiles) {
             nh[t] = 0;
@@ -483,10 +486,16 @@ __global__ __launch_bounds__(256) void k_tile_prep(const int64_t *ts, int64_t nt
         ntu = max(ntu, (unsigned long long)f[3]);
         niu = max(niu, (unsigned long long)f[4]);
         km = max(km, (unsigned long long)f[2]);
+        hm = max(hm, (unsigned long long)f[0]);
+        nhm = max(nhm, (unsigned long long)f[1]);
+        pm = max(pm, (unsigned long long)P);
     }
     block_max_to(ntu, &st->ntu_max, sh);
     block_max_to(niu, &st->niu_max, sh);
     block_max_to(km, &st->k_max, sh);
+    block_max_to(hm, &st->h_max, sh);
+    block_max_to(nhm, &st->nh_max, sh);
+    block_max_to(pm, &st->p_max, sh);
 }
 
 // ---- 3. one tile
@@ -495,20 +504,21 @@ __global__ __launch_bounds__(256) void k_tile_prep(const int64_t *ts, int64_t nt
 struct BuildCaps {
     int ntu;     // unfolded block tasks
     int niu;     // unfolded items
+    int h, nc, nh;  // halo elements, their nodes, the distinct ones
+    int k;          // elements of one node
+    int buf;     // words of the sorting buffer
     int nsets;   // bank-spread read sets (< 4096: the read entries are 16-bit)
     int spread;  // H8 FP64 bank-spread numbering
 };
 
 constexpr int kSlotsExtra = kPadTasks + 256;  // schedule slots beyond the tasks
 
-// Dynamic LDS of the build kernel.  The task arrays (word .. rows) are dead
-// once the records and items are written: the bank spread's load counters
-// reuse them, and its read entries reuse the evaluation's sort buffer when
-// they fit there.
+// Dynamic LDS of the build kernel.  The sorting buffer and the task arrays
+// (word .. rows) are dead once the records and items are written: the bank
+// spread's slots, then its load counters, and its read entries go there.
 struct BuildLds {
-    size_t word, tpair, sorted, rows, load, bcount, cq, csum, qtab, ibase, lconn, ownc, items, sinfo, gk, occcnt,
-        occfill, occ, perm, order, slotl, total;
-    bool occ_in_buf;
+    size_t buf, hn, word, tpair, sorted, rows, load, bcount, cq, csum, qtab, ibase, lconn, ownc, items, sinfo, gk,
+        occcnt, occfill, occ, perm, order, slotl, total;
 };
 
 __host__ __device__ inline size_t bl_take(size_t &o, size_t bytes) {
@@ -517,38 +527,42 @@ __host__ __device__ inline size_t bl_take(size_t &o, size_t bytes) {
     return r;
 }
 
-__host__ __device__ inline BuildLds build_lds(const BuildCaps &c, int npe) {
+__host__ __device__ inline BuildLds build_lds(const BuildCaps &c) {
     BuildLds B;
     size_t o = 0;
     const size_t ns = (size_t)c.ntu + kSlotsExtra;  // schedule slots
     const size_t nch = (size_t)c.ntu / 64 + 3;       // chunks of up to 64 tasks
     const size_t nsg = nch + 8;                      // slot groups
+    B.buf = bl_take(o, (size_t)c.buf * 4);
     B.word = bl_take(o, (size_t)c.ntu * 4);
     B.tpair = bl_take(o, (size_t)c.ntu * 2);
     B.sorted = bl_take(o, (size_t)c.ntu * 2);
     B.rows = bl_take(o, (size_t)c.ntu * 2);
-    B.load = B.word;
-    if (c.spread && (size_t)c.nsets * 16 > o) o = align16((size_t)c.nsets * 16);
-    B.bcount = bl_take(o, 513 * 4);
+    B.sinfo = B.load = B.occ = 0;
+    if (c.spread) {
+        size_t u = 0;
+        bl_take(u, std::max(ns * 4, (size_t)c.nsets * 16));
+        B.occ = bl_take(u, (size_t)c.niu * 2 * 2);
+        o = std::max(o, u);
+    }
+    B.hn = bl_take(o, (size_t)c.nh * 4);
+    B.bcount = bl_take(o, (size_t)(2 * c.k + 3) * 4);
     B.cq = bl_take(o, nch * 4);
     B.csum = bl_take(o, nch * 4);
     B.qtab = bl_take(o, nsg * 4);
     B.ibase = bl_take(o, (nsg + 1) * 4);
-    B.lconn = bl_take(o, (size_t)255 * npe * 2);
-    B.ownc = bl_take(o, (size_t)255 * npe * 2);
-    B.occ_in_buf = (size_t)c.niu * 2 * 2 <= (size_t)kMaxBoxCand * 4;
+    B.lconn = bl_take(o, (size_t)c.nc * 2);
+    B.ownc = bl_take(o, (size_t)c.nh * 2);
     if (c.spread) {
         B.items = bl_take(o, (size_t)c.niu * 2);
-        B.sinfo = bl_take(o, ns * 4);
         B.gk = bl_take(o, (ns / 16 + 2) * 4);
-        B.occcnt = bl_take(o, 257 * 4);
-        B.occfill = bl_take(o, 257 * 4);
-        B.occ = B.occ_in_buf ? 0 : bl_take(o, (size_t)c.niu * 2 * 2);
-        B.perm = bl_take(o, 256 * 4);
-        B.order = bl_take(o, 256 * 4);
-        B.slotl = bl_take(o, (256 + 32) * 4);
+        B.occcnt = bl_take(o, (size_t)(c.h + 1) * 4);
+        B.occfill = bl_take(o, (size_t)(c.h + 1) * 4);
+        B.perm = bl_take(o, (size_t)c.h * 4);
+        B.order = bl_take(o, (size_t)c.h * 4);
+        B.slotl = bl_take(o, (size_t)(c.h + 16) * 4);
     } else {
-        B.items = B.sinfo = B.gk = B.occcnt = B.occfill = B.occ = B.perm = B.order = B.slotl = 0;
+        B.items = B.gk = B.occcnt = B.occfill = B.perm = B.order = B.slotl = 0;
     }
     B.total = o;
     return B;
@@ -627,12 +641,14 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
                                                     const int64_t *slot_off, TileShape shape, BuildCaps caps,
                                                     unsigned char *slots, int32_t *hnodes, int32_t *tout,
                                                     unsigned *err, unsigned long long *tim) {
-    __shared__ __align__(16) EvalLds L;
+    __shared__ __align__(16) EvalCore L;
     __shared__ uint16_t ownj[256];  // halo-node index of each owned column (0xffff: no element)
     __shared__ int sh_fail, sh_K, sh_nch, sh_nsg, sh_NT;
     __shared__ uint32_t sh_NI;
     extern __shared__ __align__(16) unsigned char dyn[];
-    const BuildLds B = build_lds(caps, mv.npe);
+    const BuildLds B = build_lds(caps);
+    uint32_t *const buf = reinterpret_cast<uint32_t *>(dyn + B.buf);
+    int32_t *const hn = reinterpret_cast<int32_t *>(dyn + B.hn);
     uint32_t *word = reinterpret_cast<uint32_t *>(dyn + B.word);
     uint16_t *tpair = reinterpret_cast<uint16_t *>(dyn + B.tpair);
     uint16_t *sorted = reinterpret_cast<uint16_t *>(dyn + B.sorted);
@@ -663,10 +679,10 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
 
     // halo lists (the same evaluation the partition made)
     BoxSizes bs;
-    const bool fits = eval_box(mv, order, s0, P, shape, L, bs);
+    const bool fits = eval_box(mv, order, s0, P, shape, L, buf, hn, bs);
     const int64_t *f = info + kInfo * s0;
     if (!fits || bs.H != f[0] || bs.NH != f[1] || bs.NT != f[3] || bs.NI != f[4] || bs.NT > caps.ntu ||
-        bs.NI > caps.niu) {
+        bs.NI > caps.niu || bs.NH > caps.nh || bs.H > caps.h || bs.K > caps.k) {
         if (tid == 0) atomicOr(err, kErrSizes);
         return;
     }
@@ -674,16 +690,16 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
     const int H = (int)bs.H, NH = (int)bs.NH, NTu = (int)bs.NT;
     const int nc = H * npe;
     for (int i = tid; i < NH; i += kTB) {
-        hnodes[x0[t] + i] = L.hn[i];
+        hnodes[x0[t] + i] = hn[i];
         ownc[i] = -1;
     }
     for (int i = tid; i < nc; i += kTB) {
         const int32_t v = mv.conn[(int64_t)L.halo[i / npe] * npe + i % npe];
-        lconn[i] = (uint16_t)lower_bound_i32(L.hn, NH, v);
+        lconn[i] = (uint16_t)lower_bound_i32(hn, NH, v);
     }
     if (tid < P) {
-        const int j = lower_bound_i32(L.hn, NH, L.owned[tid]);
-        ownj[tid] = (j < NH && L.hn[j] == L.owned[tid]) ? (uint16_t)j : (uint16_t)0xffff;
+        const int j = lower_bound_i32(hn, NH, L.owned[tid]);
+        ownj[tid] = (j < NH && hn[j] == L.owned[tid]) ? (uint16_t)j : (uint16_t)0xffff;
     }
     if (tid == 0) {
         sh_fail = 0;
@@ -691,7 +707,7 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
     }
     __syncthreads();
     // node incidence lists (merge_halo)
-    uint32_t *keys = L.buf;
+    uint32_t *keys = buf;
     for (int i = tid; i < nc; i += kTB) keys[i] = ((uint32_t)lconn[i] << 16) | ((uint32_t)(i / npe) << 4) | (uint32_t)(i % npe);
     int n2 = 2;
     while (n2 < nc) n2 <<= 1;
@@ -722,8 +738,8 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
     for (int u = tid; u < NTu; u += kTB) {
         const int c = column_of(L.coff, P, u), r = u - (int)L.coff[c];
         const int32_t m = mv.adj[mv.adj_ptr[L.owned[c]] + r];
-        const int j = lower_bound_i32(L.hn, NH, m);
-        if (j >= NH || L.hn[j] != m) {  // a block the tile's elements do not reach
+        const int j = lower_bound_i32(hn, NH, m);
+        if (j >= NH || hn[j] != m) {  // a block the tile's elements do not reach
             atomicOr(err, kErrEmptyBlock);
             sh_fail = 1;
         }
@@ -876,7 +892,6 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
     uint64_t *rec = reinterpret_cast<uint64_t *>(blob + (Lay.task - Lay.cbase));
     uint16_t *gitem = reinterpret_cast<uint16_t *>(blob + (Lay.item - Lay.cbase));
     uint16_t *items = caps.spread ? reinterpret_cast<uint16_t *>(dyn + B.items) : gitem;
-    uint32_t *sinfo = caps.spread ? reinterpret_cast<uint32_t *>(dyn + B.sinfo) : nullptr;
 
     // task records and items, one slot group per wavefront
     for (int sg = wave; sg < nsg; sg += kTB / 64) {
@@ -898,7 +913,6 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
         if (s < NT) {
             rec[s] = valid ? ((uint64_t)(w & 0x07ffffffu) | ((uint64_t)toff << 32) | ((uint64_t)tpair[u] << 48))
                            : ((uint64_t)kNullTask | ((uint64_t)kNoPair << 48));
-            if (sinfo) sinfo[s] = valid ? (toff | (k << 16)) : 0xffffffffu;
         }
         if (valid) {
             const int c = (int)(w & 255u);
@@ -915,9 +929,16 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
         // read sets per (group of 16 slots, item step j, side), each
         // element's reads, then the greedy class choice, most-read first.
         uint32_t *gk = reinterpret_cast<uint32_t *>(dyn + B.gk);
+        uint32_t *sinfo = reinterpret_cast<uint32_t *>(dyn + B.sinfo);  // first item | items << 16, or none
+        for (int sl = tid; sl < NT; sl += kTB) {
+            const uint64_t w = rec[sl];
+            sinfo[sl] = (uint32_t)w == kNullTask ? 0xffffffffu
+                                                 : ((uint32_t)(w >> 32) & 0xffffu) | ((uint32_t)w & 0xff0000u);
+        }
+        __syncthreads();
         uint32_t *occcnt = reinterpret_cast<uint32_t *>(dyn + B.occcnt);
         uint32_t *occfill = reinterpret_cast<uint32_t *>(dyn + B.occfill);
-        uint16_t *occ = B.occ_in_buf ? reinterpret_cast<uint16_t *>(L.buf) : reinterpret_cast<uint16_t *>(dyn + B.occ);
+        uint16_t *occ = reinterpret_cast<uint16_t *>(dyn + B.occ);
         uint8_t *load = reinterpret_cast<uint8_t *>(dyn + B.load);
         int32_t *perm = reinterpret_cast<int32_t *>(dyn + B.perm);
         int32_t *eorder = reinterpret_cast<int32_t *>(dyn + B.order);
@@ -936,7 +957,6 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
             if (tid == 0) atomicOr(err, kErrSets);
             return;
         }
-        for (int i = tid; i < nsets * 16; i += kTB) load[i] = 0;
         // The reads of each set: one quarter-wavefront per group of 16 slots,
         // lane l for slot 16 g + l, one set after the other; a read counts
         // once per set (at its first slot).  Pass 0 counts each element's
@@ -982,6 +1002,7 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
             }
             __syncthreads();
         }
+        for (int i = tid; i < nsets * 16; i += kTB) load[i] = 0;  // the slots are dead
         // elements by read count, descending, stable; slots per residue class
         const int uc = shape.uchunks();
         if (tid < 16) slotl[tid] = 0;
@@ -1101,7 +1122,7 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
     }
     double *X = reinterpret_cast<double *>(blob + (Lay.X - Lay.cbase));
     for (int i = tid; i < NH; i += kTB) {
-        const int64_t n = L.hn[i];
+        const int64_t n = hn[i];
         X[2 * i] = xyz[3 * n];
         X[2 * i + 1] = xyz[3 * n + 1];
         X[2 * NH + i] = xyz[3 * n + 2];
@@ -1358,13 +1379,28 @@ std::shared_ptr<TileSet> build_tiles_device(feasm_mesh *m, const TileShape &shap
     caps.ntu = (int)ps.ntu_max;
     caps.niu = (int)ps.niu_max;
     caps.spread = (shape.grad && shape.rbytes == 8 && npe == 8) ? 1 : 0;
-    // sets of the bank spread: per chunk of 64 sorted tasks at most
-    // 2 * (K + (chunk items) / 16), the groups' first tasks
-    caps.nsets = caps.spread ? std::min(4095, 2 * ((caps.ntu / 64 + 2) * (int)ps.k_max + caps.niu / 16 + 16)) : 0;
-    const BuildLds B = build_lds(caps, npe);
+    // The sorting buffer holds the elements of the owned nodes or the nodes of
+    // the halo elements, padded to a power of two, or the sorted nodes and the
+    // lists' starts.  The LDS is sized by the largest tile: with room for any
+    // box two workgroups fit a CU (72 KiB, H8), now four do, and the kernel, which
+    // waits for LDS, takes 910 -> 590 us for the 2303 tiles of 58k elements.
+    caps.h = (int)ps.h_max;
+    caps.k = (int)ps.k_max;
+    caps.nc = caps.h * npe;
+    caps.nh = (int)ps.nh_max + 2;
+    int words = kTB;
+    while (words < std::max<int64_t>(caps.nc, std::min<int64_t>((int64_t)(ps.p_max * ps.k_max), kMaxBoxCand))) words <<= 1;
+    words = std::max(words, caps.nc + caps.nh / 2 + 2);
+    caps.buf = words;
+    // sets of the bank spread: two per group of 16 tasks and element of its
+    // longest task; the tasks of a kind (symmetric or not) are sorted by their
+    // elements, so that a group's longest is no longer than any of the group
+    // before: at most K + (items) / 16 a kind
+    caps.nsets = caps.spread ? std::min(4095, 2 * (2 * caps.k + caps.niu / 16 + 2)) : 0;
+    const BuildLds B = build_lds(caps);
     int maxlds = 0;
     FEASM_HIP(hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, ctx->device));
-    FEASM_REQUIRE(B.total + sizeof(EvalLds) + 64 <= (size_t)maxlds, FEASM_EUNSUPPORTED,
+    FEASM_REQUIRE(B.total + sizeof(EvalCore) + 1024 <= (size_t)maxlds, FEASM_EUNSUPPORTED,
                   "tiles too large for the device tile builder");
     T->hnodes = dev_alloc(std::max<int64_t>(tot[0], 1) * 4);
     DevPtr slots = tmp(std::max<int64_t>(tot[1], 16));
@@ -1437,7 +1473,7 @@ std::shared_ptr<TileSet> build_tiles_device(feasm_mesh *m, const TileShape &shap
     T->max_k = (int)st.max_k;
     if (clk.on)
         std::fprintf(stderr, "device tiles: %lld tiles, %d levels, build LDS %zu + %zu bytes\n", (long long)ntiles,
-                     levels, B.total, sizeof(EvalLds));
+                     levels, B.total, sizeof(EvalCore));
     return T;
 }
 
