@@ -53,6 +53,9 @@ struct ScopedThreadFence {
     ScopedThreadFence(int device, hipStream_t s);
     ~ScopedThreadFence();
 };
+// the calling thread's pinned host buffer, of at least `bytes`; the next call
+// (read_back's too) hands it out again
+void *pinned_buffer(size_t bytes);
 // copies bytes from device memory after the work queued on s, through a
 // pinned buffer of the calling thread (a copy into pageable memory goes
 // through the runtime's staging path, tens of microseconds a call)
@@ -306,6 +309,8 @@ std::shared_ptr<Pattern> build_pattern(feasm_mesh *m, int ndn, bool with_contrib
 // the DOF-level CSC of the mesh's own (distinct, not node-major) numbering
 std::shared_ptr<GeneralPattern> build_general_pattern(feasm_mesh *m);
 // every entry of the device connectivity d_conn[0..n) lies in [0, nnodes)
+// d[i] = i on the context's stream (pattern.hip)
+void fill_iota(feasm_ctx *ctx, int32_t *d, int64_t n);
 bool conn_in_range(feasm_ctx *ctx, const int32_t *d_conn, int64_t n, int64_t nnodes);
 void build_contributions(feasm_mesh *m, Pattern &p);
 

@@ -538,6 +538,17 @@ void exclusive_scan_i64(feasm_ctx *ctx, const int64_t *in, int64_t *out, int64_t
         rocprim::exclusive_scan(tmp, bytes, in, out, (int64_t)0, (size_t)n, rocprim::plus<int64_t>(), ctx->stream));
 }
 
+__global__ void k_iota(int32_t *__restrict__ d, int64_t n) {
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        d[i] = (int32_t)i;
+}
+
+void fill_iota(feasm_ctx *ctx, int32_t *d, int64_t n) {
+    if (n == 0) return;
+    hipLaunchKernelGGL(k_iota, dim3(grid_for(n, 256, 4096)), dim3(256), 0, ctx->stream, d, n);
+    FEASM_HIP(hipGetLastError());
+}
+
 bool conn_in_range(feasm_ctx *ctx, const int32_t *d_conn, int64_t n, int64_t nnodes) {
     if (n == 0) return true;
     DevPtr flag = dev_alloc(sizeof(unsigned int));

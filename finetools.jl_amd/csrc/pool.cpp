@@ -285,7 +285,7 @@ ScopedThreadFence::~ScopedThreadFence() {
 }
 
 namespace {
-// pinned host buffers of read_back, one per host thread; a thread's buffer
+// pinned host buffers of pinned_buffer, one per host thread; a thread's buffer
 // goes back to a free list when the thread ends (never freed: the HIP runtime
 // may be gone when the last threads end)
 struct Pinned {
@@ -305,14 +305,7 @@ struct PinnedHolder {
 thread_local PinnedHolder t_pinned;
 }  // namespace
 
-void read_back(hipStream_t s, void *host, const void *dev, size_t bytes) {
-    const ReadBack one{host, dev, bytes};
-    read_back(s, &one, 1);
-}
-
-void read_back(hipStream_t s, const ReadBack *parts, int n) {
-    size_t bytes = 0;
-    for (int i = 0; i < n; i++) bytes += (parts[i].bytes + 15) & ~size_t(15);
+void *pinned_buffer(size_t bytes) {
     Pinned &b = t_pinned.b;
     if (b.bytes < bytes) {
         Pinned nb;
@@ -325,20 +318,32 @@ void read_back(hipStream_t s, const ReadBack *parts, int n) {
                     break;
                 }
             if (b.p) g_pinned_free.push_back(b);  // too small for this thread now; another may use it
+            b = Pinned();
         }
         if (!nb.p) {
+            FEASM_HIP(hipHostMalloc(&nb.p, std::max<size_t>(bytes, 4096), hipHostMallocDefault));
             nb.bytes = std::max<size_t>(bytes, 4096);
-            FEASM_HIP(hipHostMalloc(&nb.p, nb.bytes, hipHostMallocDefault));
         }
         b = nb;
     }
-    unsigned char *q = static_cast<unsigned char *>(b.p);
+    return b.p;
+}
+
+void read_back(hipStream_t s, void *host, const void *dev, size_t bytes) {
+    const ReadBack one{host, dev, bytes};
+    read_back(s, &one, 1);
+}
+
+void read_back(hipStream_t s, const ReadBack *parts, int n) {
+    size_t bytes = 0;
+    for (int i = 0; i < n; i++) bytes += (parts[i].bytes + 15) & ~size_t(15);
+    unsigned char *const buf = static_cast<unsigned char *>(pinned_buffer(bytes)), *q = buf;
     for (int i = 0; i < n; i++) {
         if (parts[i].bytes) FEASM_HIP(hipMemcpyAsync(q, parts[i].dev, parts[i].bytes, hipMemcpyDeviceToHost, s));
         q += (parts[i].bytes + 15) & ~size_t(15);
     }
     FEASM_HIP(hipStreamSynchronize(s));
-    q = static_cast<unsigned char *>(b.p);
+    q = buf;
     for (int i = 0; i < n; i++) {
         if (parts[i].bytes) std::memcpy(parts[i].host, q, parts[i].bytes);
         q += (parts[i].bytes + 15) & ~size_t(15);

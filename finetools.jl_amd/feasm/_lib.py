@@ -37,6 +37,7 @@ SIGNATURES = {
     "feasm_probe_gram": (I32, [P, I32, I64, I32, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_double),
                                P, I64]),
     "feasm_mesh_create": (I32, [P, I32, I64, I32, P, I64, P, PP]),
+    "feasm_mesh_create_rowmajor": (I32, [P, I32, I64, I32, P, I64, P, PP]),
     "feasm_mesh_create_device": (I32, [P, I32, I64, I32, P, I64, P, PP]),
     "feasm_mesh_destroy": (I32, [P]),
     "feasm_mesh_set_xyz": (I32, [P, P]),

@@ -124,6 +124,9 @@ int feasm_probe_gram(feasm_ctx *ctx, int variant, int64_t nelem, int reps, doubl
  * 34-44): copies conn (1-based) and xyz to the device. */
 int feasm_mesh_create(feasm_ctx *ctx, int elem_type, int64_t nelem, int npe, const int64_t *conn,
                       int64_t nnodes, const double *xyz_colmajor, feasm_mesh **out);
+/* Same, with the coordinates row-major (nnodes x 3). */
+int feasm_mesh_create_rowmajor(feasm_ctx *ctx, int elem_type, int64_t nelem, int npe, const int64_t *conn,
+                               int64_t nnodes, const double *xyz, feasm_mesh **out);
 /* Same, from device memory already resident in HBM: conn0 int32 0-based
  * row-major (nelem x npe), xyz row-major (nnodes x 3).  The mesh copies them;
  * an entry of conn0 outside [0, nnodes) is FEASM_EINVAL, as on the host path. */
