@@ -771,27 +771,28 @@ __device__ __forceinline__ void load_tables(const FusedParams &kp, unsigned char
 // XCD-aware persistent walk: consecutive workgroups land on different XCDs,
 // so each XCD takes a contiguous range of the (Morton-ordered) tile list.  The
 // workgroups stride through the first kAhead tiles each; the rest of a range
-// (queue given: at least kAhead tiles per workgroup) is handed out one tile at
-// a time, and a workgroup whose range has run out goes on with the next one's:
+// (QUEUE: at least kAhead tiles per workgroup) is handed out one tile at a
+// time, and a workgroup whose range has run out goes on with the next one's:
 // tiles differ in time (T10: by a quarter of the mean), and with a fixed stride
 // the last workgroup ended 20 % (T10), 5 % (H8) after the mean.  Measured: H8
 // elasticity, 1M elements 1010 -> 984 us, T10 elasticity, 178k elements 233 ->
-// 216; with fewer than kAhead tiles a workgroup there is nothing to hand out.
+// 216.  With fewer tiles there is nothing to hand out, and the stride alone
+// (scalar header loads, no claims) is 0.4 us shorter in launches of 8 to 18 us.
 //
 // A workgroup runs tile t, loads the blob of t1, reads the header of t2 and
 // claims the tile after it.  One lane claims: the atomic is issued before phase
 // 1 and its result goes to the other wavefronts through LDS.
 constexpr int kAhead = 3;
 constexpr int kQueuePad = 32;  // words between counters: a cache line each
+template <bool QUEUE>
 struct TileWalk {
-    uint32_t *queue;  // 8 counters, one per XCD's range, and the finished workgroups; null: fixed stride
+    uint32_t *queue;  // 8 counters, one per XCD's range, and the finished workgroups
     int64_t ntiles;
     int xcd, slot, slots;
-    int32_t v;         // claiming lane: ranges found empty (fixed stride: tiles claimed)
-    uint32_t claimed;  // claiming lane: the atomic's result
+    int32_t v = 0;         // claiming lane: ranges found empty
+    uint32_t claimed = 0;  // claiming lane: the atomic's result
     __device__ __forceinline__ TileWalk(uint32_t *q, int64_t n)
-        : queue(q), ntiles(n), xcd(blockIdx.x % 8), slot(blockIdx.x / 8), slots(gridDim.x / 8),
-          v(q ? 0 : kAhead - 1), claimed(0) {}
+        : queue(q), ntiles(n), xcd(blockIdx.x % 8), slot(blockIdx.x / 8), slots(gridDim.x / 8) {}
     __device__ __forceinline__ static bool claimer() { return threadIdx.x == blockDim.x - 64; }
     __device__ __forceinline__ int64_t range(int x) const { return ntiles * x / 8; }
     // the workgroup's i-th tile by the stride, -1 if its range has no such tile
@@ -799,45 +800,45 @@ struct TileWalk {
         const int64_t t = range(xcd) + slot + (int64_t)i * slots;
         return t < range(xcd + 1) ? (int32_t)t : -1;
     }
+    // the tile after t by the stride, -1 after the last
+    __device__ __forceinline__ int32_t after(int32_t t) const {
+        return t >= 0 && (int64_t)t + slots < range(xcd + 1) ? t + slots : -1;
+    }
     __device__ __forceinline__ void start(int *next) const {
-        if (claimer()) *next = strided(kAhead - 1);
+        if (QUEUE && claimer()) *next = strided(kAhead - 1);
     }
     __device__ __forceinline__ void claim() {
-        if (claimer() && queue && v < 8) claimed = atomicAdd(queue + kQueuePad * ((xcd + v) & 7), 1u);
+        if (claimer() && v < 8) claimed = atomicAdd(queue + kQueuePad * ((xcd + v) & 7), 1u);
     }
     __device__ __forceinline__ void resolve(int *next) {
         if (!claimer()) return;
         int32_t t = -1;
-        if (!queue) {
-            t = strided(++v);
-        } else {
-            while (v < 8) {
-                const int x = (xcd + v) & 7;
-                const int64_t i = range(x) + (int64_t)kAhead * slots + claimed;
-                if (i < range(x + 1)) {
-                    t = (int32_t)i;
-                    break;
-                }
-                if (++v < 8) {
-                    claimed = atomicAdd(queue + kQueuePad * ((xcd + v) & 7), 1u);
-                } else if (atomicAdd(queue + kQueuePad * 8, 1u) == gridDim.x - 1) {
-                    // every workgroup has made its last claim: ready for the next launch
-                    for (int k = 0; k <= 8; k++) atomicExch(queue + kQueuePad * k, 0u);
-                }
+        while (v < 8) {
+            const int x = (xcd + v) & 7;
+            const int64_t i = range(x) + (int64_t)kAhead * slots + claimed;
+            if (i < range(x + 1)) {
+                t = (int32_t)i;
+                break;
+            }
+            if (++v < 8) {
+                claimed = atomicAdd(queue + kQueuePad * ((xcd + v) & 7), 1u);
+            } else if (atomicAdd(queue + kQueuePad * 8, 1u) == gridDim.x - 1) {
+                // every workgroup has made its last claim: ready for the next launch
+                for (int k = 0; k <= 8; k++) atomicExch(queue + kQueuePad * k, 0u);
             }
         }
         *next = t;
     }
 };
 
-template <int NPE, int NQP, int FORM, int NDN, typename R>
+template <int NPE, int NQP, int FORM, int NDN, typename R, bool QUEUE>
 __global__ __launch_bounds__(kMaxThreads) void k_fused(TileShape shape_, TileJob job,
                                                     const TileHdr *__restrict__ hdr, int64_t ntiles,
                                                     FusedParams kp, uint32_t *queue) {
     extern __shared__ __align__(16) unsigned char smem[];
     TileShape shape = shape_;
     shape.packed = false;  // known here, so that the layout has no branch for it
-    TileWalk walk(queue, ntiles);
+    TileWalk<QUEUE> walk(queue, ntiles);
     const int32_t t0 = walk.strided(0);
     if (t0 < 0) return;
     constexpr int DS = NPE * 3;  // TileShape::dstride()
@@ -865,16 +866,26 @@ __global__ __launch_bounds__(kMaxThreads) void k_fused(TileShape shape_, TileJob
     st.ready();
     for (;;) {
         const bool more = t1 >= 0;
-        StagedHdr sh;  // the header of tile t2
+        int32_t t2 = QUEUE ? -1 : walk.after(t1);
+        TileHdr h2;    // the header of tile t2
+        StagedHdr sh;  // (QUEUE: on its way)
+        // without the queue the gradient forms read it while the blob goes to
+        // LDS: the barrier's wait covers it, and no scalar load is left
+        // pending in the phases; the store-bound DOT forms measured faster
+        // with the read after the barrier
+        if constexpr (!QUEUE && EARLY) h2 = load_hdr(hdr, t2 >= 0 ? t2 : t0);
         stage_store(job, hd, st, shape.layout(hd.H, hd.P, hd.NH, hd.K, hd.NT, hd.NI), smem, sD, sNeg);
         __syncthreads();
-        const int32_t t2 = __builtin_amdgcn_readfirstlane(*sNext);
+        if constexpr (!QUEUE && !EARLY) h2 = load_hdr(hdr, t2 >= 0 ? t2 : t0);
+        if constexpr (QUEUE) {
+            t2 = __builtin_amdgcn_readfirstlane(*sNext);
+            walk.claim();
+        }
         const TileHdr &hb = more ? hn : hd;
         const auto issue = [&]() {
-            sh.issue(hdr, nullptr, max(t2, 0));
+            if constexpr (QUEUE) sh.issue(hdr, nullptr, max(t2, 0));
             stage_issue(job, hb, nullptr, st);
         };
-        walk.claim();
         if constexpr (EARLY) issue();
         tile_compute<NPE, NQP, FORM, NDN, R, false>(
             shape, job, kp, hd, smem,
@@ -883,15 +894,18 @@ __global__ __launch_bounds__(kMaxThreads) void k_fused(TileShape shape_, TileJob
             },
             [&]() {
                 if constexpr (EARLY) {
-                    sh.ready();
+                    if constexpr (QUEUE) sh.ready();
                     st.ready();
                 }
-                walk.resolve(sNext);
+                if constexpr (QUEUE) walk.resolve(sNext);
             });
         if (!more) break;
         t1 = t2;
         hd = hn;
-        hn = sh.get();
+        if constexpr (QUEUE)
+            hn = sh.get();
+        else
+            hn = h2;
     }
 }
 
@@ -1149,7 +1163,7 @@ __device__ __forceinline__ void packed_tile(const TileShape &shape, const TileJo
     }
 }
 
-template <int NPE, int NQP, int FORM, int NDN, typename R>
+template <int NPE, int NQP, int FORM, int NDN, typename R, bool QUEUE>
 __global__ __launch_bounds__(kPackedThreads, 2) void k_packed(TileShape shape_, TileJob job,
                                                            const TileHdr *__restrict__ hdr, int64_t ntiles,
                                                            FusedParams kp, uint32_t *queue) {
@@ -1157,7 +1171,7 @@ __global__ __launch_bounds__(kPackedThreads, 2) void k_packed(TileShape shape_, 
     extern __shared__ __align__(16) unsigned char smem[];
     TileShape shape = shape_;
     shape.packed = true;
-    TileWalk walk(queue, ntiles);
+    TileWalk<QUEUE> walk(queue, ntiles);
     const int32_t t0 = walk.strided(0);
     if (t0 < 0) return;
     double *sD = reinterpret_cast<double *>(smem) + NQP * NPE * 4;
@@ -1171,23 +1185,31 @@ __global__ __launch_bounds__(kPackedThreads, 2) void k_packed(TileShape shape_, 
     st.ready();
     for (;;) {
         const bool more = t1 >= 0;
-        StagedHdr sh;  // the header of tile t2
+        int32_t t2 = QUEUE ? -1 : walk.after(t1);
+        TileHdr h2;  // the header of tile t2, as in k_fused
+        StagedHdr sh;
+        if constexpr (!QUEUE) h2 = load_hdr(hdr, t2 >= 0 ? t2 : t0);
         stage_store(job, hd, st, shape.layout(hd.H, hd.P, hd.NH, hd.K, hd.NT, hd.NI), smem, sD, sNeg);
         __syncthreads();
-        const int32_t t2 = __builtin_amdgcn_readfirstlane(*sNext);
-        walk.claim();
-        sh.issue(hdr, nullptr, max(t2, 0));
+        if constexpr (QUEUE) {
+            t2 = __builtin_amdgcn_readfirstlane(*sNext);
+            walk.claim();
+            sh.issue(hdr, nullptr, max(t2, 0));
+        }
         stage_issue(job, more ? hn : hd, nullptr, st);  // waited for before this tile's stores
         packed_tile<FORM, false>(shape, job, kp, hd, smem, [&]() {
-            sh.ready();
+            if constexpr (QUEUE) sh.ready();
             st.ready();
-            walk.resolve(sNext);
+            if constexpr (QUEUE) walk.resolve(sNext);
         });
         if (!more) break;
         __syncthreads();
         t1 = t2;
         hd = hn;
-        hn = sh.get();
+        if constexpr (QUEUE)
+            hn = sh.get();
+        else
+            hn = h2;
     }
 }
 
@@ -1203,7 +1225,7 @@ struct BatchEntry {
 // meshes' tiles, mesh after mesh); every tile carries its mesh's
 // coefficients and arrays.  One launch covers the meshes of one element
 // type, rule, arithmetic and form.
-template <int NPE, int NQP, int FORM, int NDN, typename R>
+template <int NPE, int NQP, int FORM, int NDN, typename R, bool QUEUE>
 __global__ __launch_bounds__(kMaxThreads) void k_fused_batch(const BatchEntry *__restrict__ entries,
                                                           const int32_t *__restrict__ tile_entry,
                                                           const TileHdr *__restrict__ hdr, int64_t ntiles,
@@ -1211,7 +1233,7 @@ __global__ __launch_bounds__(kMaxThreads) void k_fused_batch(const BatchEntry *_
     extern __shared__ __align__(16) unsigned char smem[];
     TileShape shape = shape_;
     shape.packed = false;  // known here, so that the layout has no branch for it
-    TileWalk walk(queue, ntiles);
+    TileWalk<QUEUE> walk(queue, ntiles);
     const int32_t t0 = walk.strided(0);
     if (t0 < 0) return;
     constexpr int DS = NPE * 3;  // TileShape::dstride()
@@ -1232,17 +1254,30 @@ __global__ __launch_bounds__(kMaxThreads) void k_fused_batch(const BatchEntry *_
     st.ready();
     for (;;) {
         const bool more = t1 >= 0;
-        StagedHdr sh;  // the header and entry of tile t2
+        int32_t t2 = QUEUE ? -1 : walk.after(t1);
+        TileHdr h2;  // the header and entry of tile t2, as in k_fused
+        const BatchEntry *E2 = nullptr;
+        StagedHdr sh;
+        if constexpr (!QUEUE && EARLY) {
+            h2 = load_hdr(hdr, t2 >= 0 ? t2 : t0);
+            E2 = entries + tile_entry[t2 >= 0 ? t2 : t0];
+        }
         stage_store(E->job, hd, st, shape.layout(hd.H, hd.P, hd.NH, hd.K, hd.NT, hd.NI), smem, sD, sNeg);
         __syncthreads();
-        const int32_t t2 = __builtin_amdgcn_readfirstlane(*sNext);
+        if constexpr (!QUEUE && !EARLY) {
+            h2 = load_hdr(hdr, t2 >= 0 ? t2 : t0);
+            E2 = entries + tile_entry[t2 >= 0 ? t2 : t0];
+        }
+        if constexpr (QUEUE) {
+            t2 = __builtin_amdgcn_readfirstlane(*sNext);
+            walk.claim();
+        }
         const TileHdr &hb = more ? hn : hd;
         const BatchEntry *Eb = more ? En : E;
         const auto issue = [&]() {
-            sh.issue(hdr, tile_entry, max(t2, 0));
+            if constexpr (QUEUE) sh.issue(hdr, tile_entry, max(t2, 0));
             stage_issue(Eb->job, hb, Eb->kp.fp.coef, st);
         };
-        walk.claim();
         if constexpr (EARLY) issue();
         tile_compute<NPE, NQP, FORM, NDN, R, true>(
             shape, E->job, E->kp, hd, smem,
@@ -1251,22 +1286,27 @@ __global__ __launch_bounds__(kMaxThreads) void k_fused_batch(const BatchEntry *_
             },
             [&]() {
                 if constexpr (EARLY) {
-                    sh.ready();
+                    if constexpr (QUEUE) sh.ready();
                     st.ready();
                 }
-                walk.resolve(sNext);
+                if constexpr (QUEUE) walk.resolve(sNext);
             });
         if (!more) break;
         t1 = t2;
         hd = hn;
         E = En;
-        hn = sh.get();
-        En = entries + sh.entry();
+        if constexpr (QUEUE) {
+            hn = sh.get();
+            En = entries + sh.entry();
+        } else {
+            hn = h2;
+            En = E2;
+        }
     }
 }
 
 // k_packed over the global tile list of a batched launch.
-template <int NPE, int NQP, int FORM, int NDN, typename R>
+template <int NPE, int NQP, int FORM, int NDN, typename R, bool QUEUE>
 __global__ __launch_bounds__(kPackedThreads, 2) void k_packed_batch(const BatchEntry *__restrict__ entries,
                                                                  const int32_t *__restrict__ tile_entry,
                                                                  const TileHdr *__restrict__ hdr, int64_t ntiles,
@@ -1275,7 +1315,7 @@ __global__ __launch_bounds__(kPackedThreads, 2) void k_packed_batch(const BatchE
     extern __shared__ __align__(16) unsigned char smem[];
     TileShape shape = shape_;
     shape.packed = true;
-    TileWalk walk(queue, ntiles);
+    TileWalk<QUEUE> walk(queue, ntiles);
     const int32_t t0 = walk.strided(0);
     if (t0 < 0) return;
     double *sD = reinterpret_cast<double *>(smem) + NQP * NPE * 4;
@@ -1291,27 +1331,41 @@ __global__ __launch_bounds__(kPackedThreads, 2) void k_packed_batch(const BatchE
     st.ready();
     for (;;) {
         const bool more = t1 >= 0;
-        StagedHdr sh;  // the header and entry of tile t2
+        int32_t t2 = QUEUE ? -1 : walk.after(t1);
+        TileHdr h2;  // the header and entry of tile t2, as in k_fused
+        const BatchEntry *E2 = nullptr;
+        StagedHdr sh;
+        if constexpr (!QUEUE) {
+            h2 = load_hdr(hdr, t2 >= 0 ? t2 : t0);
+            E2 = entries + tile_entry[t2 >= 0 ? t2 : t0];
+        }
         stage_store(E->job, hd, st, shape.layout(hd.H, hd.P, hd.NH, hd.K, hd.NT, hd.NI), smem, sD, sNeg);
         __syncthreads();
-        const int32_t t2 = __builtin_amdgcn_readfirstlane(*sNext);
         const TileHdr &hb = more ? hn : hd;
         const BatchEntry *Eb = more ? En : E;
-        walk.claim();
-        sh.issue(hdr, tile_entry, max(t2, 0));
+        if constexpr (QUEUE) {
+            t2 = __builtin_amdgcn_readfirstlane(*sNext);
+            walk.claim();
+            sh.issue(hdr, tile_entry, max(t2, 0));
+        }
         stage_issue(Eb->job, hb, Eb->kp.fp.coef, st);
         packed_tile<FORM, true>(shape, E->job, E->kp, hd, smem, [&]() {
-            sh.ready();
+            if constexpr (QUEUE) sh.ready();
             st.ready();
-            walk.resolve(sNext);
+            if constexpr (QUEUE) walk.resolve(sNext);
         });
         if (!more) break;
         __syncthreads();
         t1 = t2;
         hd = hn;
         E = En;
-        hn = sh.get();
-        En = entries + sh.entry();
+        if constexpr (QUEUE) {
+            hn = sh.get();
+            En = entries + sh.entry();
+        } else {
+            hn = h2;
+            En = E2;
+        }
     }
 }
 
@@ -1358,17 +1412,17 @@ template <int NPE, int NQP, int FORM, int NDN, typename R>
 void go(feasm_ctx *ctx, const feasm_mesh *m, const Pattern &p, const TileSet &t, const FusedParams &kp,
         double *nzval) {
     constexpr bool PACKED = NPE == 8 && sizeof(R) == 8 && (FORM == FEASM_FORM_DIFFUSION_ISO || FORM == FEASM_FORM_DIFFUSION_MAT);
-    auto kern = [] {
+    const unsigned grid = persistent_grid(ctx, t.shape.budget, t.ntiles);
+    uint32_t *queue = t.ntiles >= (int64_t)kAhead * grid ? ctx_tile_queue(ctx) : nullptr;
+    auto kern = [&] {
         if constexpr (PACKED)
-            return k_packed<NPE, NQP, FORM, NDN, R>;
+            return queue ? k_packed<NPE, NQP, FORM, NDN, R, true> : k_packed<NPE, NQP, FORM, NDN, R, false>;
         else
-            return k_fused<NPE, NQP, FORM, NDN, R>;
+            return queue ? k_fused<NPE, NQP, FORM, NDN, R, true> : k_fused<NPE, NQP, FORM, NDN, R, false>;
     }();
     const int budget = (int)t.shape.budget;
     FEASM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, budget));
-    const unsigned grid = persistent_grid(ctx, t.shape.budget, t.ntiles);
     TileJob job = make_job(m, t, nzval);
-    uint32_t *queue = t.ntiles >= (int64_t)kAhead * grid ? ctx_tile_queue(ctx) : nullptr;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(t.shape.threads), budget, ctx->stream, t.shape, job, job.hdr, t.ntiles,
                        kp, queue);
     FEASM_HIP(hipGetLastError());
@@ -1403,11 +1457,11 @@ void dispatch(feasm_ctx *ctx, const feasm_mesh *m, const Pattern &p, const TileS
 template <int NPE, int NQP, int FORM, int NDN, typename R>
 void go_batch(feasm_ctx *ctx, const BatchLaunch &b) {
     constexpr bool PACKED = NPE == 8 && sizeof(R) == 8 && (FORM == FEASM_FORM_DIFFUSION_ISO || FORM == FEASM_FORM_DIFFUSION_MAT);
-    auto kern = [] {
+    auto kern = [&] {
         if constexpr (PACKED)
-            return k_packed_batch<NPE, NQP, FORM, NDN, R>;
+            return b.queue ? k_packed_batch<NPE, NQP, FORM, NDN, R, true> : k_packed_batch<NPE, NQP, FORM, NDN, R, false>;
         else
-            return k_fused_batch<NPE, NQP, FORM, NDN, R>;
+            return b.queue ? k_fused_batch<NPE, NQP, FORM, NDN, R, true> : k_fused_batch<NPE, NQP, FORM, NDN, R, false>;
     }();
     FEASM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b.budget));
     hipLaunchKernelGGL(kern, dim3(b.grid), dim3(b.threads), b.budget, ctx->stream,
