@@ -789,7 +789,7 @@ struct TileWalk {
     uint32_t *queue;  // 8 counters, one per XCD's range, and the finished workgroups
     int64_t ntiles;
     int xcd, slot, slots;
-    int32_t v = 0;         // claiming lane: ranges found empty
+    int32_t v = 0;         // claiming wavefront: ranges found empty
     uint32_t claimed = 0;  // claiming lane: the atomic's result
     __device__ __forceinline__ TileWalk(uint32_t *q, int64_t n)
         : queue(q), ntiles(n), xcd(blockIdx.x % 8), slot(blockIdx.x / 8), slots(gridDim.x / 8) {}
@@ -810,24 +810,32 @@ struct TileWalk {
     __device__ __forceinline__ void claim() {
         if (claimer() && v < 8) claimed = atomicAdd(queue + kQueuePad * ((xcd + v) & 7), 1u);
     }
+    // by the claiming wavefront together, so that only `claimed` takes a vector
+    // register (between the two calls)
     __device__ __forceinline__ void resolve(int *next) {
-        if (!claimer()) return;
+        if ((threadIdx.x >> 6) != (blockDim.x >> 6) - 1) return;
+        const auto add = [&](int k) {
+            uint32_t old = 0;
+            if (claimer()) old = atomicAdd(queue + kQueuePad * k, 1u);
+            return (uint32_t)__builtin_amdgcn_readfirstlane(old);
+        };
         int32_t t = -1;
+        uint32_t c = __builtin_amdgcn_readfirstlane(claimed);
         while (v < 8) {
             const int x = (xcd + v) & 7;
-            const int64_t i = range(x) + (int64_t)kAhead * slots + claimed;
+            const int64_t i = range(x) + (int64_t)kAhead * slots + c;
             if (i < range(x + 1)) {
                 t = (int32_t)i;
                 break;
             }
             if (++v < 8) {
-                claimed = atomicAdd(queue + kQueuePad * ((xcd + v) & 7), 1u);
-            } else if (atomicAdd(queue + kQueuePad * 8, 1u) == gridDim.x - 1) {
+                c = add((xcd + v) & 7);
+            } else if (add(8) == gridDim.x - 1 && claimer()) {
                 // every workgroup has made its last claim: ready for the next launch
                 for (int k = 0; k <= 8; k++) atomicExch(queue + kQueuePad * k, 0u);
             }
         }
-        *next = t;
+        if (claimer()) *next = t;
     }
 };
 
@@ -890,19 +898,27 @@ __global__ __launch_bounds__(kMaxThreads) void k_fused(TileShape shape_, TileJob
         tile_compute<NPE, NQP, FORM, NDN, R, false>(
             shape, job, kp, hd, smem,
             [&]() {
+                if constexpr (QUEUE && EARLY) {
+                    // done with before phase 2: the claim and the header held
+                    // in vector registers across it cost spills (H8 elasticity
+                    // with a general D, 64k elements: 97.6 us, so 87.8)
+                    walk.resolve(sNext);
+                    sh.ready();
+                    h2 = sh.get();
+                }
                 if constexpr (!EARLY) issue();
             },
             [&]() {
                 if constexpr (EARLY) {
-                    if constexpr (QUEUE) sh.ready();
                     st.ready();
+                } else if constexpr (QUEUE) {
+                    walk.resolve(sNext);  // (phase 1 is too short for the claim)
                 }
-                if constexpr (QUEUE) walk.resolve(sNext);
             });
         if (!more) break;
         t1 = t2;
         hd = hn;
-        if constexpr (QUEUE)
+        if constexpr (QUEUE && !EARLY)
             hn = sh.get();
         else
             hn = h2;
@@ -1282,14 +1298,16 @@ __global__ __launch_bounds__(kMaxThreads) void k_fused_batch(const BatchEntry *_
         tile_compute<NPE, NQP, FORM, NDN, R, true>(
             shape, E->job, E->kp, hd, smem,
             [&]() {
+                if constexpr (QUEUE && EARLY) walk.resolve(sNext);
                 if constexpr (!EARLY) issue();
             },
             [&]() {
                 if constexpr (EARLY) {
                     if constexpr (QUEUE) sh.ready();
                     st.ready();
+                } else if constexpr (QUEUE) {
+                    walk.resolve(sNext);  // (phase 1 is too short for the claim)
                 }
-                if constexpr (QUEUE) walk.resolve(sNext);
             });
         if (!more) break;
         t1 = t2;
