@@ -527,11 +527,12 @@ static void new_numbering(feasm_mesh *m, int ndn, DevPtr dofs, int64_t nalldofs,
 }
 
 // the node-major numbering 1..ndn*nnodes, written on the device (made on the
-// host and uploaded, 73k nodes of 3 components took 280 us, now 6)
+// host and uploaded, 73k nodes of 3 components took 280 us, now 15)
 static void set_dofs_nodemajor(feasm_mesh *m, int ndn) {
     const int64_t n = m->nnodes * ndn;
     DevPtr d = dev_alloc(std::max<size_t>(n * sizeof(int32_t), 4));
     fill_iota(m->ctx, dp<int32_t>(d), n);
+    FEASM_HIP(hipStreamSynchronize(m->ctx->stream));  // usable on any stream, as a copied one
     new_numbering(m, ndn, d, n, true);
 }
 

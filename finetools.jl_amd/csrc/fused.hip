@@ -1,16 +1,16 @@
 // Fused numeric assembly: element integration and the global summation in
 // one kernel, nothing staged in HBM.
 //
-// Each workgroup walks a contiguous range of tiles (a compact set of owned
-// column nodes plus the halo of elements incident to them, with the tile's
-// node blocks listed as tasks; see tiles.cpp).  Per tile:
+// Each workgroup walks tiles of its XCD's contiguous range (a tile: a compact
+// set of owned column nodes plus the halo of elements incident to them, with
+// the tile's node blocks listed as tasks; see tiles.cpp).  Per tile:
 //   0  the tile's LDS image (column pointers, task and item lists, halo
 //      connectivity; one contiguous blob laid out by TileShape::layout) and
 //      the coordinates of its halo nodes go to LDS.  These global loads are
 //      issued while the previous tile is in phase 2 and held in registers;
-//   1  one thread per (halo element, quadrature point): J = X' dN, det J by
-//      cofactors of row 1 and the adjugate inverse (src/FESetModule.jl:479-544)
-//      in FP64; the spatial gradients g_a = inv(J)' dN_a are stored scaled by
+//   1  one thread per (halo element, quadrature point): J = X' dN (in FP64
+//      kernels by exchanges between the element's points, point_fp64), det J
+//      and the adjugate inverse (src/FESetModule.jl:479-544) in FP64; the spatial gradients g_a = inv(J)' dN_a are stored scaled by
 //      sqrt(|J w|) (u_a = sqrt(|Jw|) g_a, with the sign of J w kept apart), so
 //      that an element's node-pair matrix is M_ab = sum_q s_q u_a u_b^T;
 //   2  one thread per CSC node block (m, c) of the tile's columns forms the

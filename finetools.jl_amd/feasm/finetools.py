@@ -656,7 +656,7 @@ def _run(femm, assembler, geom, u, form, coeff, return_device=False):
             mesh = femm._device_mesh(geom, u, nodemajor=True)
             full = mesh.bilform(form, kind, order, coeff, precision=assembler.precision)
             keep = ~u.fixed.ravel()
-        else:  # the field's own numbering (COO path), its leading block
+        else:  # the field's own numbering (general pattern), its leading block
             mesh = femm._device_mesh(geom, u)
             full = mesh.bilform(form, kind, order, coeff, precision=assembler.precision)
             keep = np.zeros(full.dims[1], bool)

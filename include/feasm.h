@@ -138,7 +138,8 @@ int feasm_mesh_set_xyz(feasm_mesh *mesh, const double *xyz_rowmajor);
 /* numberdofs!/gatherdofnums! (src/FieldModule.jl:304-377): dofnums nnodes x ndn
  * column-major, 1-based; nalldofs (src/FieldModule.jl:102).  When dofnums is
  * the node-major numbering (node-1)*ndn + comp, assembly uses the device
- * resident CSC pattern; otherwise it goes through the generic COO path. */
+ * resident CSC pattern; other numberings of distinct DOFs get a pattern ranked
+ * from the node blocks, and numberings that share DOFs the generic COO path. */
 int feasm_dofs_set(feasm_mesh *mesh, int ndn, const int64_t *dofnums_colmajor, int64_t nalldofs);
 /* Node-major numbering without passing the table (numberdofs! with no EBCs). */
 int feasm_dofs_set_nodemajor(feasm_mesh *mesh, int ndn);
@@ -160,8 +161,8 @@ int feasm_bilform(feasm_mesh *mesh, int form, int rule, int order, const double 
  * staging buffers already exist). */
 int feasm_bilform_into(feasm_mesh *mesh, int form, int rule, int order, const double *coeff, int ncoeff,
                        int precision, feasm_matrix *mat);
-/* Generic path used for non-node-major DOF numberings, and selectable for
- * testing: element kernels write COO triples in assemble!'s order, then the
+/* Generic path used for numberings that share DOFs between nodes, and
+ * selectable for testing: element kernels write COO triples in assemble!'s order, then the
  * device sparse() (radix sort + ordered duplicate summation). */
 int feasm_bilform_coo(feasm_mesh *mesh, int form, int rule, int order, const double *coeff, int ncoeff,
                       int precision, feasm_matrix **out);
@@ -172,7 +173,8 @@ int feasm_bilform_coo(feasm_mesh *mesh, int form, int rule, int order, const dou
  * pattern; values agree to rounding. */
 int feasm_mesh_set_numeric_path(feasm_mesh *mesh, int path);
 /* Tile parameters of the fused kernel for this mesh (0 = default):
- * owned nodes per tile (<= 255), LDS per workgroup in KiB, threads (256/512/1024). */
+ * owned nodes per tile (<= 255), LDS per workgroup in KiB, threads (256/512/1024;
+ * H8 FP64 scalar diffusion always runs 256). */
 int feasm_mesh_set_tile_params(feasm_mesh *mesh, int max_nodes, int budget_kib, int threads);
 /* Tiles built for the fused kernel so far (summed over forms/precisions). */
 int feasm_mesh_tile_info(feasm_mesh *mesh, int64_t *ntiles, int64_t *nhalo);
