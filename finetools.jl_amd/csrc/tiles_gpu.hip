@@ -440,9 +440,9 @@ __global__ void k_tile_starts(const uint8_t *start, const int32_t *inc, int64_t 
 }
 
 // per tile: halo-node count and slot size (for the scans), maxima for the
-// build kernel's LDS
+// build kernel's LDS; rep_max: the most times an element lists one node
 struct PrepStats {
-    unsigned long long ntu_max, niu_max, k_max, h_max, nh_max, p_max;
+    unsigned long long ntu_max, niu_max, k_max, h_max, nh_max, p_max, rep_max;
 };
 
 // largest of v over the workgroup (256 threads), added to *out with one atomic
@@ -468,9 +468,16 @@ __device__ void block_sum_to(unsigned long long v, unsigned long long *out, unsi
 }
 
 __global__ __launch_bounds__(256) void k_tile_prep(const int64_t *ts, int64_t ntiles, const int64_t *info,
-                                                   TileShape shape, int64_t *nh, int64_t *slot, PrepStats *st) {
+                                                   TileShape shape, const int32_t *conn, int64_t nelem, int npe,
+                                                   int64_t *nh, int64_t *slot, PrepStats *st) {
     __shared__ unsigned long long sh[256];
-    unsigned long long ntu = 0, niu = 0, km = 0, hm = 0, nhm = 0, pm = 0;
+    unsigned long long ntu = 0, niu = 0, km = 0, hm = 0, nhm = 0, pm = 0, rm = 1;
+    for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < nelem; e += (int64_t)gridDim.x * blockDim.x)
+        for (int a = 0; a < npe; a++) {
+            unsigned long long r = 1;
+            for (int b = a + 1; b < npe; b++) r += conn[e * npe + a] == conn[e * npe + b] ? 1 : 0;
+            rm = max(rm, r);
+        }
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t <= ntiles; t += (int64_t)gridDim.x * blockDim.x) {
         if (t == ntiles) {
             nh[t] = 0;
@@ -496,6 +503,7 @@ __global__ __launch_bounds__(256) void k_tile_prep(const int64_t *ts, int64_t nt
     block_max_to(hm, &st->h_max, sh);
     block_max_to(nhm, &st->nh_max, sh);
     block_max_to(pm, &st->p_max, sh);
+    block_max_to(rm, &st->rep_max, sh);
 }
 
 // ---- 3. one tile
@@ -505,7 +513,8 @@ struct BuildCaps {
     int ntu;     // unfolded block tasks
     int niu;     // unfolded items
     int h, nc, nh;  // halo elements, their nodes, the distinct ones
-    int k;          // elements of one node
+    int k;          // elements of one node (its incidences)
+    int kb;         // items of one node block
     int buf;     // words of the sorting buffer
     int nsets;   // bank-spread read sets (< 4096: the read entries are 16-bit)
     int spread;  // H8 FP64 bank-spread numbering
@@ -546,7 +555,7 @@ __host__ __device__ inline BuildLds build_lds(const BuildCaps &c) {
         o = std::max(o, u);
     }
     B.hn = bl_take(o, (size_t)c.nh * 4);
-    B.bcount = bl_take(o, (size_t)(2 * c.k + 3) * 4);
+    B.bcount = bl_take(o, (size_t)(2 * c.kb + 3) * 4);
     B.cq = bl_take(o, nch * 4);
     B.csum = bl_take(o, nch * 4);
     B.qtab = bl_take(o, nsg * 4);
@@ -796,6 +805,11 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
     if (sh_fail) return;
     mark(3);
     const int K = sh_K;
+
+    if (K > caps.kb) {
+        if (tid == 0) atomicOr(err, kErrSizes);
+        return;
+    }
 
     // stable counting sort of the kept tasks by task_bucket
     const int nb = 2 * K + 2;
@@ -1364,8 +1378,9 @@ std::shared_ptr<TileSet> build_tiles_device(feasm_mesh *m, const TileShape &shap
     DevPtr x0 = tmp((ntiles + 1) * 8), slot_off = tmp((ntiles + 1) * 8);
     DevPtr pst = tmp(sizeof(PrepStats));
     FEASM_HIP(hipMemsetAsync(pst->p, 0, sizeof(PrepStats), s));
-    hipLaunchKernelGGL(k_tile_prep, dim3(grid_for(ntiles + 1, 256, 1024)), dim3(256), 0, s, dp<int64_t>(ts), ntiles,
-                       dp<int64_t>(info), shape, dp<int64_t>(nh), dp<int64_t>(slot), dp<PrepStats>(pst));
+    hipLaunchKernelGGL(k_tile_prep, dim3(grid_for(std::max(ntiles + 1, m->nelem), 256, 1024)), dim3(256), 0, s,
+                       dp<int64_t>(ts), ntiles, dp<int64_t>(info), shape, mv.conn, m->nelem, npe, dp<int64_t>(nh),
+                       dp<int64_t>(slot), dp<PrepStats>(pst));
     FEASM_HIP(hipGetLastError());
     scan_excl<int64_t>(s, dp<int64_t>(nh), dp<int64_t>(x0), ntiles + 1, hold);
     scan_excl<int64_t>(s, dp<int64_t>(slot), dp<int64_t>(slot_off), ntiles + 1, hold);
@@ -1386,6 +1401,10 @@ std::shared_ptr<TileSet> build_tiles_device(feasm_mesh *m, const TileShape &shap
     // waits for LDS, takes 910 -> 590 us for the 2303 tiles of 68k elements.
     caps.h = (int)ps.h_max;
     caps.k = (int)ps.k_max;
+    // a block of the nodes n and m has (times an element lists n) * (times it
+    // lists m) items of each element: an element that lists a node r times
+    // (a collapsed hexahedron) has r incidences of it, and r * r items
+    caps.kb = (int)std::min<unsigned long long>(255, ps.k_max * ps.rep_max);
     caps.nc = caps.h * npe;
     caps.nh = (int)ps.nh_max + 2;
     int words = kTB;
