@@ -1411,11 +1411,12 @@ std::shared_ptr<TileSet> build_tiles_device(feasm_mesh *m, const TileShape &shap
     while (words < std::max<int64_t>(caps.nc, std::min<int64_t>((int64_t)(ps.p_max * ps.k_max), kMaxBoxCand))) words <<= 1;
     words = std::max(words, caps.nc + caps.nh / 2 + 2);
     caps.buf = words;
-    // sets of the bank spread: two per group of 16 tasks and element of its
-    // longest task; the tasks of a kind (symmetric or not) are sorted by their
-    // elements, so that a group's longest is no longer than any of the group
-    // before: at most K + (items) / 16 a kind
-    caps.nsets = caps.spread ? std::min(4095, 2 * (2 * caps.k + caps.niu / 16 + 2)) : 0;
+    // sets of the bank spread: two per group of 16 tasks and item of its
+    // longest task; the tasks of a kind are sorted by their items, so that a
+    // group's longest is no longer than any of the group before: at most the
+    // kind's longest (k for the symmetric tasks, which have one item of each
+    // element, kb for the others) + (items) / 16
+    caps.nsets = caps.spread ? std::min(4095, 2 * (caps.k + caps.kb + caps.niu / 16 + 2)) : 0;
     const BuildLds B = build_lds(caps);
     int maxlds = 0;
     FEASM_HIP(hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, ctx->device));
