@@ -1523,13 +1523,16 @@ void prepare_batch_launch(feasm_ctx *ctx, BatchLaunch &b, const std::vector<Batc
     b.hdr = dev_alloc(std::max<size_t>((size_t)b.ntiles * sizeof(TileHdr), 16));
     FEASM_HIP(hipMemcpy(b.entries->p, host.data(), host.size() * sizeof(BatchEntry), hipMemcpyHostToDevice));
     FEASM_HIP(hipMemcpy(b.tile_entry->p, tile_entry.data(), tile_entry.size() * 4, hipMemcpyHostToDevice));
+    // on the launches' own stream: device work on the null stream need not be
+    // done when the call returns, and the context's stream does not wait for it
     for (size_t i = 0; i < items.size(); i++)  // the meshes' headers, one after the other
-        FEASM_HIP(hipMemcpy(static_cast<TileHdr *>(b.hdr->p) + host[i].tile0, items[i].tiles->hdr->p,
-                            (size_t)items[i].tiles->ntiles * sizeof(TileHdr), hipMemcpyDeviceToDevice));
+        FEASM_HIP(hipMemcpyAsync(static_cast<TileHdr *>(b.hdr->p) + host[i].tile0, items[i].tiles->hdr->p,
+                                 (size_t)items[i].tiles->ntiles * sizeof(TileHdr), hipMemcpyDeviceToDevice,
+                                 ctx->stream));
     b.grid = persistent_grid(ctx, b.budget, b.ntiles);
     if (b.ntiles >= (int64_t)kAhead * b.grid) {
         b.queue = dev_alloc(kQueueBytes);
-        FEASM_HIP(hipMemset(b.queue->p, 0, kQueueBytes));
+        FEASM_HIP(hipMemsetAsync(b.queue->p, 0, kQueueBytes, ctx->stream));
     }
 }
 
