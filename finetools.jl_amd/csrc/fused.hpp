@@ -108,9 +108,14 @@ constexpr uint16_t kNoPair = 0xffff;
 // room for them)
 constexpr int kPadTasks = 320;
 
-// Order of a tile's block tasks (k elements each, K the most): the symmetric
-// diagonal blocks first, then the others, the longest first in each kind.
-__host__ __device__ inline int task_order(int k, bool sym, int K) { return (sym ? 0 : K + 1) + (K - k); }
+// Order of a tile's block tasks (k items each, K the most).  Where the kernel
+// has a shorter sum for the symmetric diagonal blocks (grad: the shapes with
+// gradient records) these come first, then the others, the longest first in each
+// kind; elsewhere a task's time is its items' whatever its kind, and the longest
+// come first, the symmetric ones before the others of equal length.
+__host__ __device__ inline int task_order(int k, bool sym, int K, bool grad) {
+    return grad ? (sym ? 0 : K + 1) + (K - k) : 2 * (K - k) + (sym ? 0 : 1);
+}
 // The chunks of 64 tasks that run as one wavefront: [0, nsym) and [nsym, nt)
 // are cut up separately (nsym = 0 where the kernel has no shorter sum for the
 // symmetric blocks).  A wavefront that held both kinds ran both sums in turn:
@@ -125,9 +130,9 @@ __host__ __device__ inline TaskChunk task_chunk(int ch, int nsym, int nt) {
     const int ns = (nsym + 63) / 64, b = ch < ns ? ch * 64 : nsym + (ch - ns) * 64, lim = ch < ns ? nsym : nt;
     return {b, b + 64 < lim ? b + 64 : lim};
 }
-// a wavefront's time by its longest task, in elements: the material and store
+// a wavefront's time by its longest task, in items: the material and store
 // work counts as two
-__host__ __device__ inline double task_cost(int k, bool sym) { return (sym ? 0.5 : 1.0) * k + 2.0; }
+__host__ __device__ inline double task_cost(int k, bool sym, bool grad) { return (grad && sym ? 0.5 : 1.0) * k + 2.0; }
 
 struct TileSet {
     TileShape shape;

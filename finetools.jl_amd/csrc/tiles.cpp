@@ -334,14 +334,13 @@ void make_tile(const HostMesh &h, const int32_t *owned, int P, const TileShape &
         for (int j = 0; T.sym && j < T.k; j++)
             if (((its[T.off + j] >> 4) & 15u) != (its[T.off + j] & 15u)) T.sym = false;
     }
-    // longest first, the symmetric diagonal blocks before all others (see
-    // task_order; a stable counting sort: the order of std::stable_sort by
+    // in task_order (a stable counting sort: the order of std::stable_sort by
     // that key)
     int K = 0;
     for (const Task &T : tasks) K = std::max(K, T.k);
     FEASM_REQUIRE(K <= 255, FEASM_EUNSUPPORTED, "a node block is shared by more than 255 elements");
     {
-        auto bucket = [K](const Task &T) { return task_order(T.k, T.sym, K); };
+        auto bucket = [K, &shape](const Task &T) { return task_order(T.k, T.sym, K, shape.grad); };
         std::vector<int> start(2 * K + 3, 0);
         for (const Task &T : tasks) start[bucket(T) + 1]++;
         for (size_t b = 1; b < start.size(); b++) start[b] += start[b - 1];
@@ -368,7 +367,7 @@ void make_tile(const HostMesh &h, const int32_t *owned, int P, const TileShape &
             const Task &T = tasks[task_chunk(ch, nsym, nt).begin];
             const int q = (int)(std::min_element(load.begin(), load.end()) - load.begin());
             queue[q].push_back(ch);
-            load[q] += task_cost(T.k, T.sym);
+            load[q] += task_cost(T.k, T.sym, shape.grad);
         }
     }
     size_t rounds = 0;

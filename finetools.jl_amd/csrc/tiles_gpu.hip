@@ -601,10 +601,9 @@ __device__ int merge_halo(const uint32_t *keys, const uint16_t *nptr, int ja, in
     return k;
 }
 
-// the stable-sort key of a kept task: longest first, the symmetric diagonal
-// blocks first among equal counts
-__device__ __forceinline__ int task_bucket(uint32_t w, int K) {
-    return task_order((int)((w >> 16) & 255u), (w >> 26) & 1u, K);
+// the stable-sort key of a kept task
+__device__ __forceinline__ int task_bucket(uint32_t w, int K, bool grad) {
+    return task_order((int)((w >> 16) & 255u), (w >> 26) & 1u, K, grad);
 }
 
 constexpr uint32_t kDropBit = 1u << 27;  // builder-internal: computed by the transposed block's task
@@ -817,7 +816,7 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
     __syncthreads();
     for (int u = tid; u < NTu; u += kTB) {
         const uint32_t w = word[u];
-        if (!(w & kDropBit)) atomicAdd(&bcount[task_bucket(w, K)], 1u);
+        if (!(w & kDropBit)) atomicAdd(&bcount[task_bucket(w, K, shape.grad)], 1u);
     }
     __syncthreads();
     const int NTk = (int)block_excl_scan(bcount, nb, L.part);
@@ -829,7 +828,7 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
         for (int base = 0; base < NTu; base += 64) {
             const int u = base + lane;
             const uint32_t w = u < NTu ? word[u] : kDropBit;
-            const bool hit = !(w & kDropBit) && task_bucket(w, K) == b;
+            const bool hit = !(w & kDropBit) && task_bucket(w, K, shape.grad) == b;
             const uint64_t mask = __ballot(hit);
             if (hit) sorted[pos + __popcll(mask & ((1ull << lane) - 1ull))] = (uint16_t)u;
             pos += (uint32_t)__popcll(mask);
@@ -853,7 +852,7 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
         int qn[4] = {0, 0, 0, 0};
         for (int ch = 0; ch < nch; ch++) {
             const uint32_t w = word[sorted[task_chunk(ch, nsym, NTk).begin]];
-            const double cost = task_cost((int)((w >> 16) & 255u), (w >> 26) & 1u);
+            const double cost = task_cost((int)((w >> 16) & 255u), (w >> 26) & 1u, shape.grad);
             int q = 0;
             for (int i = 1; i < 4; i++)
                 if (load[i] < load[q]) q = i;
