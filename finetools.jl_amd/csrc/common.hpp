@@ -374,8 +374,9 @@ int bits_for(uint64_t v);
 size_t sort_tmp_bytes(int64_t nt, unsigned end_bit, hipStream_t s);
 // keys + range check, stable sort, segment heads and numbers, one read-back:
 // returns nnz, throws FEASM_EDOF for an index outside [0,m) x [0,n)
+// (pinned: through the thread's pinned buffer, which may be allocated for it)
 int64_t sparse_phase_a(hipStream_t s, int64_t nt, const int32_t *I, const int32_t *J, int64_t m, int64_t n,
-                       unsigned end_bit, SparseWork &w);
+                       unsigned end_bit, SparseWork &w, bool pinned);
 // segment starts, ordered sums, column pointers
 void sparse_phase_b(hipStream_t s, int64_t nt, const double *V, int64_t m, int64_t n, int64_t nnz,
                     const SparseWork &w, int64_t *colptr, int32_t *rowval, double *nzval);

@@ -86,11 +86,6 @@ __global__ void k_colptr(const uint64_t *__restrict__ keys, const int64_t *__res
     }
 }
 
-__global__ void k_fill_i32(int32_t *__restrict__ p, int64_t n, int32_t v) {
-    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x)
-        p[t] = v;
-}
-
 // colptr of a matrix with no entries (a fill kernel rather than a memset)
 __global__ void k_fill_i64(int64_t *__restrict__ p, int64_t n, int64_t v) {
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x)
@@ -111,9 +106,39 @@ __global__ void k_fill_i64(int64_t *__restrict__ p, int64_t n, int64_t v) {
 constexpr int kSmallColumn = 256, kMaxColumn = 1024;  // triples of one column the wavefront sorts hold
 // mean run length from which this way pays: the lists take 8 bytes a run
 constexpr int64_t kMinRun = 4;
-// state bits: a row out of range; a column too long or its rows too far apart;
-// a column of more than kSmallColumn triples
-constexpr unsigned kBadRow = 1, kTooWide = 2, kBigColumn = 4;
+// state bits: a row or column out of range; a column too long or its rows too
+// far apart; a column of more than kSmallColumn triples; runs too short
+constexpr unsigned kBadRow = 1, kTooWide = 2, kBigColumn = 4, kBadColumn = 8, kShortRuns = 16;
+// states in which this way is given up: the kernels that follow return at once
+constexpr unsigned kGiveUp = kTooWide | kBadColumn | kShortRuns;
+constexpr int kSampleWindows = 256, kFarTriples = kMaxColumn;
+constexpr int64_t kMinTriples = 1 << 16;
+
+// What the triples look like, from up to kSampleWindows stretches of 64 spread
+// over them: out[0] the runs, out[1] the triples that have the column of the one
+// kFarTriples further on (columns too long for the wavefront sorts).
+__global__ __launch_bounds__(1024) void k_run_sample(const int32_t *__restrict__ J, int64_t nt,
+                                                     unsigned int *__restrict__ out) {
+    __shared__ unsigned int sum[2];
+    if (threadIdx.x < 2) sum[threadIdx.x] = 0;
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t all = (nt + 63) / 64, windows = min(all, (int64_t)kSampleWindows);
+    unsigned int runs = 0, far = 0;
+    for (int64_t k = wave; k < windows; k += 16) {
+        const int64_t t = all * k / windows * 64 + lane;
+        const int32_t j = t < nt ? J[t] : 0, f = t + kFarTriples < nt ? J[t + kFarTriples] : ~j;
+        const int32_t prev = __shfl_up(j, 1, 64);
+        runs += (unsigned)__popcll(__ballot(t < nt && (lane == 0 || prev != j)));
+        far += (unsigned)__popcll(__ballot(t < nt && f == j));
+    }
+    if (lane == 0) {
+        atomicAdd(&sum[0], runs);
+        atomicAdd(&sum[1], far);
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) out[threadIdx.x] = sum[threadIdx.x];
+}
 
 // the run that starts at this lane's triple: its length, 0 when none does
 __device__ __forceinline__ int run_at(int32_t j, bool in, int lane) {
@@ -124,11 +149,11 @@ __device__ __forceinline__ int run_at(int32_t j, bool in, int lane) {
     return above ? __ffsll((unsigned long long)above) : __popcll(all >> lane);
 }
 
-// per column: its runs (high word) and triples (low word); bad is set for a
+// per column: its runs (high word) and triples (low word); kBadColumn for a
 // column index outside [0, n)
 __global__ __launch_bounds__(256) void k_run_count(const int32_t *__restrict__ J, int64_t nt, int64_t n,
                                                    unsigned long long *__restrict__ cnt,
-                                                   unsigned int *__restrict__ bad) {
+                                                   unsigned int *__restrict__ state) {
     const int lane = threadIdx.x & 63;
     const int64_t step = (int64_t)gridDim.x * blockDim.x;
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t - lane < nt; t += step) {
@@ -139,7 +164,7 @@ __global__ __launch_bounds__(256) void k_run_count(const int32_t *__restrict__ J
             if (ok)
                 atomicAdd(&cnt[j], (1ull << 32) | (unsigned)len);
             else
-                atomicOr(bad, 1u);
+                atomicOr(state, kBadColumn);
         }
     }
 }
@@ -149,7 +174,9 @@ __global__ __launch_bounds__(256) void k_run_count(const int32_t *__restrict__ J
 // place in column order (low word).
 __global__ __launch_bounds__(256) void k_run_fill(const int32_t *__restrict__ J, int64_t nt,
                                                   const uint64_t *__restrict__ place,
-                                                  unsigned long long *__restrict__ cnt, uint2 *__restrict__ runs) {
+                                                  unsigned long long *__restrict__ cnt, uint2 *__restrict__ runs,
+                                                  const unsigned int *__restrict__ state) {
+    if (*state & kGiveUp) return;
     const int lane = threadIdx.x & 63;
     const int64_t step = (int64_t)gridDim.x * blockDim.x;
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t - lane < nt; t += step) {
@@ -162,9 +189,14 @@ __global__ __launch_bounds__(256) void k_run_fill(const int32_t *__restrict__ J,
     }
 }
 
-__global__ __launch_bounds__(256) void k_col_check(const uint64_t *__restrict__ place, int64_t n,
-                                                   unsigned int *__restrict__ state) {
+// (cnt: the end of the columns' entry counts, which the scan of them reads)
+__global__ __launch_bounds__(256) void k_col_check(const uint64_t *__restrict__ place, int64_t n, int64_t nt,
+                                                   int32_t *__restrict__ cnt, unsigned int *__restrict__ state) {
     unsigned st = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        cnt[n] = 0;
+        if ((int64_t)(place[n] >> 32) > nt / kMinRun) st = kShortRuns;
+    }
     for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x) {
         const uint32_t L = (uint32_t)place[c + 1] - (uint32_t)place[c];
         st |= (L > kMaxColumn ? kTooWide : 0u) | (L > kSmallColumn ? kBigColumn : 0u);
@@ -290,7 +322,7 @@ __global__ __launch_bounds__(64) void k_columns(const int32_t *__restrict__ I, c
                                                 unsigned int *__restrict__ state) {
     __shared__ __align__(16) int32_t lds[4 * (BIG ? kMaxColumn : kSmallColumn)];
     const unsigned before = *state;
-    if ((before & kTooWide) || (BIG && !(before & kBigColumn))) return;
+    if ((before & kGiveUp) || (BIG && !(before & kBigColumn))) return;
     const int lane = threadIdx.x;
     unsigned int st = 0;
     for (int64_t c = blockIdx.x; c < n; c += gridDim.x) {
@@ -335,45 +367,45 @@ void fill_i64(hipStream_t s, int64_t *p, int64_t n, int64_t v) {
     FEASM_HIP(hipGetLastError());
 }
 
-static void fill_i32(hipStream_t s, int32_t *p, int64_t n, int32_t v) {
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(n, 256)), dim3(256), 0, s, p, n, v);
-    FEASM_HIP(hipGetLastError());
-}
-
-// The shorter way; null when the triples are not in runs, or a column is too
-// long or too wide for the wavefront sort.  Throws FEASM_EDOF for an index out
+// The shorter way; null when the triples are few or not in runs, or a column is
+// too long or too wide for the wavefront sort.  Throws FEASM_EDOF for an index out
 // of range, as the general way does.
 static feasm_matrix *sparse_by_columns(feasm_ctx *ctx, int64_t nt, const int32_t *I, const int32_t *J, const double *V,
                                        int64_t m, int64_t n) {
+    // few triples: both ways are launches and waits, and the sort has fewer of
+    // them (H8 elasticity in runs: 37k triples 135 us by the sort, 146 this way; 72k
+    // 169, 127); but the sort fills the gaps of a wide matrix's column pointers one
+    // by one (37k triples of 20 M columns 501 ms, this way 2.5)
+    if (nt < kMinTriples && n <= nt) return nullptr;
     hipStream_t s = ctx->stream;
-    DevPtr small = dev_alloc(256);  // the column range flag, and the state word of k_columns
-    unsigned int *flags = dp<unsigned int>(small);
-    DevPtr ccnt = dev_alloc((n + 1) * 8), place = dev_alloc((n + 1) * 8);
-    fill_i64(s, reinterpret_cast<int64_t *>(flags), 2, 0);
-    fill_i64(s, dp<int64_t>(ccnt), n + 1, 0);
+    // A look at a few of the triples first: what this way does before it knows
+    // all the runs (an atomic a run, two passes over the columns) would cost
+    // triples in no order half of their sort again (11.3 M: 1030 us, 560 more).
+    unsigned int *sample = static_cast<unsigned int *>(pinned_buffer(2 * sizeof(unsigned int)));
+    hipLaunchKernelGGL(k_run_sample, dim3(1), dim3(1024), 0, s, J, nt, sample);
+    FEASM_HIP(hipGetLastError());
+    FEASM_HIP(hipStreamSynchronize(s));
+    const int64_t seen = std::min<int64_t>(nt, 64 * kSampleWindows);
+    if (seen < kMinRun * (int64_t)sample[0] || 2 * (int64_t)sample[1] > seen) return nullptr;
+    DevPtr ccnt = dev_alloc((n + 2) * 8), place = dev_alloc((n + 1) * 8);
+    unsigned int *state = reinterpret_cast<unsigned int *>(dp<int64_t>(ccnt) + n + 1);
+    fill_i64(s, dp<int64_t>(ccnt), n + 2, 0);
     const unsigned gt = grid_for(nt, 256, 1u << 14);
-    hipLaunchKernelGGL(k_run_count, dim3(gt), dim3(256), 0, s, J, nt, n, dp<unsigned long long>(ccnt), flags);
+    hipLaunchKernelGGL(k_run_count, dim3(gt), dim3(256), 0, s, J, nt, n, dp<unsigned long long>(ccnt), state);
     FEASM_HIP(hipGetLastError());
-    // the run total stays below 2^31 and the triples below 2^32, so the two
-    // words are scanned as one number
+    // both words of an entry stay below 2^32 (at most a run a triple), so they
+    // are scanned as one number and read back unsigned
     exclusive_scan_i64(ctx, dp<int64_t>(ccnt), dp<int64_t>(place), n + 1);
-    uint64_t total = 0;
-    unsigned int bad = 0;
-    const ReadBack rb1[2] = {{&total, dp<uint64_t>(place) + n, sizeof(total)}, {&bad, flags, sizeof(bad)}};
-    read_back(s, rb1, 2);
-    FEASM_REQUIRE(bad == 0, FEASM_EDOF, "sparse: row or column index out of range");
-    const int64_t nruns = (int64_t)(total >> 32);
-    if (nt < kMinRun * nruns) return nullptr;
-    DevPtr runs = dev_alloc(nruns * sizeof(uint2));
-    hipLaunchKernelGGL(k_run_fill, dim3(gt), dim3(256), 0, s, J, nt, dp<uint64_t>(place),
-                       dp<unsigned long long>(ccnt), dp<uint2>(runs));
-    FEASM_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_col_check, dim3(grid_for(n, 256)), dim3(256), 0, s, dp<uint64_t>(place), n, flags + 1);
     DevPtr cnt = dev_alloc((n + 1) * 4), trow = dev_alloc(nt * 4), tval = dev_alloc(nt * 8);
-    fill_i32(s, dp<int32_t>(cnt) + n, 1, 0);
+    hipLaunchKernelGGL(k_col_check, dim3(grid_for(n, 256)), dim3(256), 0, s, dp<uint64_t>(place), n, nt,
+                       dp<int32_t>(cnt), state);
+    DevPtr runs = dev_alloc(std::max<int64_t>(nt / kMinRun, 1) * sizeof(uint2));  // k_col_check: no more of them
+    hipLaunchKernelGGL(k_run_fill, dim3(gt), dim3(256), 0, s, J, nt, dp<uint64_t>(place),
+                       dp<unsigned long long>(ccnt), dp<uint2>(runs), state);
+    FEASM_HIP(hipGetLastError());
     const auto columns = [&](auto kern, unsigned most) {
         hipLaunchKernelGGL(kern, dim3(grid_for(n, 1, most)), dim3(64), 0, s, I, V, m, n, dp<uint64_t>(place),
-                           dp<uint2>(runs), dp<int32_t>(cnt), dp<int32_t>(trow), dp<double>(tval), flags + 1);
+                           dp<uint2>(runs), dp<int32_t>(cnt), dp<int32_t>(trow), dp<double>(tval), state);
         FEASM_HIP(hipGetLastError());
     };
     columns(k_columns<false>, 1u << 17);
@@ -384,11 +416,11 @@ static feasm_matrix *sparse_by_columns(feasm_ctx *ctx, int64_t nt, const int32_t
     M->n = n;
     M->colptr = dev_alloc((n + 1) * sizeof(int64_t));
     exclusive_scan_i32_to_i64(ctx, dp<int32_t>(cnt), dp<int64_t>(M->colptr), n + 1);
-    unsigned int state = 0;
-    const ReadBack rb2[2] = {{&M->nnz, dp<int64_t>(M->colptr) + n, sizeof(int64_t)}, {&state, flags + 1, sizeof(state)}};
-    read_back(s, rb2, 2);
-    if (state & kTooWide) return nullptr;
-    FEASM_REQUIRE(!(state & kBadRow), FEASM_EDOF, "sparse: row or column index out of range");
+    unsigned int st = 0;
+    const ReadBack rb[2] = {{&M->nnz, dp<int64_t>(M->colptr) + n, sizeof(int64_t)}, {&st, state, sizeof(st)}};
+    read_back(s, rb, 2);
+    FEASM_REQUIRE(!(st & (kBadRow | kBadColumn)), FEASM_EDOF, "sparse: row or column index out of range");
+    if (st & kGiveUp) return nullptr;
     M->rowval = dev_alloc(std::max<int64_t>(M->nnz, 1) * sizeof(int32_t));
     M->nzval = dev_alloc(std::max<int64_t>(M->nnz, 1) * sizeof(double));
     hipLaunchKernelGGL(k_columns_pack, dim3(grid_for(n, 4)), dim3(256), 0, s, dp<uint64_t>(place), n,
@@ -418,7 +450,7 @@ size_t sort_tmp_bytes(int64_t nt, unsigned end_bit, hipStream_t s) {
 // Phase A: keys + range check, stable sort, segment heads and numbers; one
 // read-back.  Returns nnz; FEASM_EDOF when an index is out of range.
 int64_t sparse_phase_a(hipStream_t s, int64_t nt, const int32_t *I, const int32_t *J, int64_t m, int64_t n,
-                       unsigned end_bit, SparseWork &w) {
+                       unsigned end_bit, SparseWork &w, bool pinned) {
     hipLaunchKernelGGL(k_zero_flag, dim3(1), dim3(64), 0, s, w.flag);
     hipLaunchKernelGGL(k_keys, dim3(grid_for(nt, 256)), dim3(256), 0, s, I, J, nt, m, n, w.keys, w.idx, w.flag);
     FEASM_HIP(hipGetLastError());
@@ -438,8 +470,12 @@ int64_t sparse_phase_a(hipStream_t s, int64_t nt, const int32_t *I, const int32_
                        (const unsigned int *)w.flag, w.count);
     FEASM_HIP(hipGetLastError());
     int64_t hc[2] = {0, 0};
-    FEASM_HIP(hipMemcpyAsync(hc, w.count, sizeof(hc), hipMemcpyDeviceToHost, s));
-    FEASM_HIP(hipStreamSynchronize(s));
+    if (pinned) {
+        read_back(s, hc, w.count, sizeof(hc));
+    } else {
+        FEASM_HIP(hipMemcpyAsync(hc, w.count, sizeof(hc), hipMemcpyDeviceToHost, s));
+        FEASM_HIP(hipStreamSynchronize(s));
+    }
     FEASM_REQUIRE(hc[1] == 0, FEASM_EDOF, "sparse: row or column index out of range");
     return hc[0];
 }
@@ -467,8 +503,13 @@ feasm_matrix *sparse_device(feasm_ctx *ctx, int64_t nt, const int32_t *I, const 
                             int64_t m, int64_t n) {
     check_sparse_args(nt, m, n);
     hipStream_t s = ctx->stream;
-    if (nt > 0)
-        if (feasm_matrix *M = sparse_by_columns(ctx, nt, I, J, V, m, n)) return M;
+    if (nt > 0) {
+        try {
+            if (feasm_matrix *M = sparse_by_columns(ctx, nt, I, J, V, m, n)) return M;
+        } catch (const Error &e) {
+            if (e.code != FEASM_ENOMEM) throw;  // 20 bytes a column more than the sort takes
+        }
+    }
     std::unique_ptr<feasm_matrix> M(new feasm_matrix);
     M->ctx = ctx;
     M->m = m;
@@ -493,7 +534,7 @@ feasm_matrix *sparse_device(feasm_ctx *ctx, int64_t nt, const int32_t *I, const 
     w.flag = reinterpret_cast<unsigned int *>(dp<int64_t>(small) + 2);
     w.tmp_bytes = sort_tmp_bytes(nt, end_bit, s);
     w.tmp = ctx->scratch_get(w.tmp_bytes);
-    const int64_t nnz = sparse_phase_a(s, nt, I, J, m, n, end_bit, w);
+    const int64_t nnz = sparse_phase_a(s, nt, I, J, m, n, end_bit, w, true);
     DevPtr start = dev_alloc(nnz * sizeof(int64_t));
     w.start = dp<int64_t>(start);
     M->nnz = nnz;

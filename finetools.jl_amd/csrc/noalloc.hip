@@ -85,7 +85,7 @@ extern "C" int feasm_sparse_device_noalloc(feasm_ctx *ctx, int64_t ntrip, const 
         FEASM_REQUIRE(w.tmp_bytes <= kNoAllocTmpBytes, FEASM_ENOMEM,
                       "feasm_sparse_device_noalloc: sort storage beyond the fixed scratch array");
         w.tmp_bytes = kNoAllocTmpBytes;
-        const int64_t count = sparse_phase_a(s, ntrip, d_I, d_J, m, n, end_bit, w);
+        const int64_t count = sparse_phase_a(s, ntrip, d_I, d_J, m, n, end_bit, w, false);
         sparse_phase_b(s, ntrip, d_V, m, n, count, w, d_colptr, d_rowval, d_nzval);
         FEASM_HIP(hipStreamSynchronize(s));
         *nnz = count;

@@ -1,0 +1,93 @@
+"""Which way the device sparse() takes: few triples, triples in no order and
+columns too long go to the radix sort, runs of one column to the wavefront per
+column.  Every input is bitwise the oracle's sparse() whichever it is: around
+the least number of triples, in wide matrices, with runs that a look at a part
+of the triples shows and the whole does not have, and the other way round."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle as O
+from feasm import _lib as L
+from feasm import core
+from test_gpu_device_entry_points import DeviceBuffers
+from test_gpu_sparse_runs import check, runs
+
+pytestmark = pytest.mark.gpu
+
+LEAST = 1 << 16  # triples from which runs are looked for
+
+
+def values(rng, n):
+    return rng.uniform(-1.0, 1.0, n) * 10.0 ** rng.integers(-8, 9, n)
+
+
+def in_runs(rng, nt, n, length):
+    J = np.repeat(rng.integers(1, n + 1, -(-nt // length)), length)[:nt]
+    return rng.integers(1, n + 1, nt), J
+
+
+@pytest.mark.parametrize("nt", [LEAST - 1, LEAST, LEAST + 1, 3 * LEAST + 17])
+@pytest.mark.parametrize("length", [1, 3, 4, 5, 24, 64, 100])
+def test_run_lengths_around_the_least_number(ctx, nt, length):
+    rng = np.random.default_rng(nt + length)
+    I, J = in_runs(rng, nt, 700, length)
+    check(ctx, I, J, values(rng, nt), 700, 700)
+
+
+@pytest.mark.parametrize("longest", [1, 63, 64, 65, 128, 129, 256, 257, 512, 513, 1024, 1025, 3000])
+@pytest.mark.parametrize("filler", [False, True])
+def test_column_lengths(ctx, longest, filler):
+    """Few triples of a wide matrix; and among enough others."""
+    rng = np.random.default_rng(longest)
+    n = 40
+    lengths = rng.integers(0, longest + 1, n)
+    lengths[[0, 7, n - 1]] = 0, longest, longest
+    I, J, V = runs(rng, np.arange(1, n + 1), lengths, max(1, longest // 3))
+    if filler:
+        i, j = in_runs(rng, LEAST, 900, 24)
+        I, J, V = np.r_[I, i], np.r_[J, j + 50], np.r_[V, values(rng, LEAST)]
+        check(ctx, I, J, V, 1100, 1000)
+    else:
+        check(ctx, I, J, V, max(1, longest // 3) + 2, n + len(V) + 3)
+
+
+def test_runs_only_where_one_looks(ctx):
+    """Every fourth stretch of 64 is looked at: runs there and nowhere else, and the reverse."""
+    rng = np.random.default_rng(8)
+    nt = 64 * 1024
+    J = rng.integers(1, 3001, nt).reshape(-1, 64)
+    for looked in (True, False):
+        K = J.copy()
+        at = (np.arange(1024) % 4 == 0) == looked
+        K[at] = np.repeat(rng.integers(1, 3001, (int(at.sum()), 2)), 32, axis=1)
+        check(ctx, rng.integers(1, 3001, nt), K.ravel(), values(rng, nt), 3000, 3000)
+
+
+@pytest.mark.parametrize("columns", [1, 20])
+def test_few_columns(ctx, columns):
+    rng = np.random.default_rng(columns)
+    nt = 2 * LEAST
+    J = np.repeat(np.arange(1, columns + 1), nt // columns)
+    check(ctx, rng.integers(1, 5001, len(J)), J, values(rng, len(J)), 5000, 5000)
+
+
+@pytest.mark.parametrize("bad", ["row", "column", "column of few"])
+def test_indices_out_of_range(ctx, hiprt, bad):
+    rng = np.random.default_rng(5)
+    I, J = in_runs(rng, LEAST + 100 if bad != "column of few" else 500, 400, 24)
+    i0, j0 = (I - 1).astype(np.int32), (J - 1).astype(np.int32)
+    n = 400 if bad != "column of few" else 1000
+    if bad == "row":
+        i0[333] = n
+    else:
+        j0[333] = -1
+    buf = DeviceBuffers(hiprt)
+    try:
+        d = [buf.upload(a) for a in (i0, j0, values(rng, len(i0)))]
+        h = ctypes.c_void_p()
+        rc = L.lib().feasm_sparse_device(ctx.h, len(i0), *d, n, n, ctypes.byref(h))
+    finally:
+        buf.free()
+    assert rc == L.EDOF and not h.value
