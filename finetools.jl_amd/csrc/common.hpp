@@ -265,6 +265,10 @@ __device__ __forceinline__ int32_t lane_xor(int32_t x, int j, int lane) {
         default: return __shfl_xor(x, j, 64);
     }
 }
+__device__ __forceinline__ int64_t lane_xor(int64_t x, int j, int lane) {
+    const uint32_t lo = (uint32_t)lane_xor((int32_t)(uint32_t)x, j, lane);
+    return (int64_t)(((uint64_t)(uint32_t)lane_xor((int32_t)(x >> 32), j, lane) << 32) | lo);
+}
 
 // fused.hip: D (6 x 6, row-major) has cubic symmetry -- D00 = D11 = D22,
 // D01 = D02 = D12, D33 = D44 = D55, every other entry zero

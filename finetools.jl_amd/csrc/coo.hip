@@ -23,6 +23,8 @@
 #include "common.hpp"
 #include "wavesort.hpp"
 
+#include <limits>
+
 #include <rocprim/rocprim.hpp>
 
 namespace feasm {
@@ -106,11 +108,13 @@ __global__ void k_fill_i64(int64_t *__restrict__ p, int64_t n, int64_t v) {
 constexpr int kSmallColumn = 256, kMaxColumn = 1024;  // triples of one column the wavefront sorts hold
 // mean run length from which this way pays: the lists take 8 bytes a run
 constexpr int64_t kMinRun = 4;
-// state bits: a row or column out of range; a column too long or its rows too
-// far apart; a column of more than kSmallColumn triples; runs too short
-constexpr unsigned kBadRow = 1, kTooWide = 2, kBigColumn = 4, kBadColumn = 8, kShortRuns = 16;
+// state bits: a row or column out of range; a column of more than kMaxColumn
+// triples; one of more than kSmallColumn; rows of a column too far apart for
+// 31-bit keys; runs too short
+constexpr unsigned kBadRow = 1, kTooLong = 2, kBigColumn = 4, kBadColumn = 8, kShortRuns = 16, kWideRows = 32;
 // states in which this way is given up: the kernels that follow return at once
-constexpr unsigned kGiveUp = kTooWide | kBadColumn | kShortRuns;
+constexpr unsigned kGiveUp = kTooLong | kBadColumn | kShortRuns;
+constexpr int kWide = -1;  // sort_column: the rows are too far apart for its keys
 constexpr int kSampleWindows = 256, kFarTriples = kMaxColumn;
 constexpr int64_t kMinTriples = 1 << 16;
 
@@ -199,7 +203,7 @@ __global__ __launch_bounds__(256) void k_col_check(const uint64_t *__restrict__ 
     }
     for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x) {
         const uint32_t L = (uint32_t)place[c + 1] - (uint32_t)place[c];
-        st |= (L > kMaxColumn ? kTooWide : 0u) | (L > kSmallColumn ? kBigColumn : 0u);
+        st |= (L > kMaxColumn ? kTooLong : 0u) | (L > kSmallColumn ? kBigColumn : 0u);
     }
     if (st) atomicOr(state, st);
 }
@@ -207,12 +211,14 @@ __global__ __launch_bounds__(256) void k_col_check(const uint64_t *__restrict__ 
 // One column of L <= 64 E triples in nr runs: its runs ordered, its rows sorted
 // (ties by input order: the key's low B bits are the place in the column),
 // duplicates folded left to right.  The distinct rows and their sums go to
-// trow / tval; returns their number.  lds: 4 * 64 E words of the wavefront's own.
-template <int E, int B>
+// trow / tval; returns their number.  Keys of 31 bits (T int32_t) hold rows up to
+// 2^(31-B) apart, else kWide is returned; keys of 63 any row.  lds: 4 * 64 E words
+// of the wavefront's own.
+template <int E, int B, typename T>
 __device__ __forceinline__ int sort_column(const int32_t *__restrict__ I, const double *__restrict__ V, int64_t m,
                                            const uint2 *__restrict__ runs, int nr, int L, int lane, int32_t *lds,
                                            int32_t *__restrict__ trow, double *__restrict__ tval, unsigned int &state) {
-    constexpr int32_t kPad = 0x7fffffff;
+    constexpr T kPad = std::numeric_limits<T>::max();
     // the places of the runs, in order of their first triple (by counting the
     // triples of earlier runs), and what takes a place to its triple
     uint32_t *const sS = reinterpret_cast<uint32_t *>(lds), *const sN = sS + 64 * E, *const sAt = sN + 64 * E,
@@ -247,22 +253,23 @@ __device__ __forceinline__ int sort_column(const int32_t *__restrict__ I, const 
     }
     wave_fence();
     double *const sV = reinterpret_cast<double *>(lds);
-    int32_t *const sK = lds + 2 * 64 * E;
-    int32_t x[E], lo = kPad, hi = -1;
+    T *const sK = reinterpret_cast<T *>(lds + 2 * 64 * E);
+    int32_t row[E], lo = 0x7fffffff, hi = -1;
+    T x[E];
     double v[E];
 #pragma unroll
     for (int e = 0; e < E; e++) {
         const int p = lane + 64 * e;
-        x[e] = p < L ? I[t[e]] : kPad;
+        row[e] = p < L ? I[t[e]] : 0;
         v[e] = p < L ? V[t[e]] : 0.0;
     }
     bool out = false;
 #pragma unroll
     for (int e = 0; e < E; e++) {
         const bool in = lane + 64 * e < L;
-        out |= in && (x[e] < 0 || (int64_t)x[e] >= m);
-        lo = in ? min(lo, x[e]) : lo;
-        hi = in ? max(hi, x[e]) : hi;
+        out |= in && (row[e] < 0 || (int64_t)row[e] >= m);
+        lo = in ? min(lo, row[e]) : lo;
+        hi = in ? max(hi, row[e]) : hi;
         sV[lane + 64 * e] = v[e];
     }
 #pragma unroll
@@ -272,18 +279,21 @@ __device__ __forceinline__ int sort_column(const int32_t *__restrict__ I, const 
     }
     if (__any(out)) {
         state |= kBadRow;
+        wave_fence();  // the words are reused for the next column
         return 0;
     }
-    if (hi - lo >= (1 << (31 - B)) - 1) {
-        state |= kTooWide;
-        return 0;
+    if constexpr (sizeof(T) == 4) {
+        if (hi - lo >= (1 << (31 - B)) - 1) {
+            wave_fence();
+            return kWide;
+        }
     }
 #pragma unroll
     for (int e = 0; e < E; e++) {
         const int p = lane + 64 * e;
-        x[e] = p < L ? ((x[e] - lo) << B) | p : kPad;
+        x[e] = p < L ? ((T)(row[e] - lo) << B) | p : kPad;
     }
-    wave_sort<E>(x, lane);
+    wave_sort(x, lane);
 #pragma unroll
     for (int e = 0; e < E; e++) sK[lane + 64 * e] = x[e];
     wave_fence();
@@ -294,52 +304,62 @@ __device__ __forceinline__ int sort_column(const int32_t *__restrict__ I, const 
         const bool head = i < L && (i == 0 || (sK[i > 0 ? i - 1 : 0] >> B) != (x[e] >> B));
         const uint64_t hm = __ballot(head);
         if (head) {
-            const int32_t row = x[e] >> B;
-            double a = sV[x[e] & ((1 << B) - 1)];
+            const T r = x[e] >> B;
+            double a = sV[(int)x[e] & ((1 << B) - 1)];
             for (int q = i + 1; q < L; q++) {
-                const int32_t y = sK[q];
-                if ((y >> B) != row) break;
-                a = a + sV[y & ((1 << B) - 1)];
+                const T y = sK[q];
+                if ((y >> B) != r) break;
+                a = a + sV[(int)y & ((1 << B) - 1)];
             }
             const int at = base + __popcll(hm & ((1ull << lane) - 1ull));
-            trow[at] = row + lo;
+            trow[at] = (int32_t)r + lo;
             tval[at] = a;
         }
         base += __popcll(hm);
     }
-    wave_fence();  // the words are reused for the next column
+    wave_fence();
     return base;
 }
 
-// One wavefront per column; BIG: the columns of more than kSmallColumn triples,
-// else the others.  A column's distinct rows and sums go to trow / tval from its
-// first place on, their number to cnt.
-template <bool BIG>
+// One wavefront per column: kSmall the columns of up to kSmallColumn triples,
+// kBig the longer ones; kWideKeys those that either found wide (cnt kWide), with
+// 63-bit keys: quadratic elements whose edge nodes are numbered after 700k
+// corners have such columns.  (A kernel of their own: in kBig's they would take
+// its registers from 121 to 194.)  A column's distinct rows and sums go to trow /
+// tval from its first place on, their number to cnt.
+enum { kSmall, kBig, kWideKeys };
+template <int WHICH>
 __global__ __launch_bounds__(64) void k_columns(const int32_t *__restrict__ I, const double *__restrict__ V, int64_t m,
                                                 int64_t n, const uint64_t *__restrict__ place,
                                                 const uint2 *__restrict__ runs, int32_t *__restrict__ cnt,
                                                 int32_t *__restrict__ trow, double *__restrict__ tval,
                                                 unsigned int *__restrict__ state) {
-    __shared__ __align__(16) int32_t lds[4 * (BIG ? kMaxColumn : kSmallColumn)];
+    __shared__ __align__(16) int32_t lds[4 * (WHICH == kSmall ? kSmallColumn : kMaxColumn)];
     const unsigned before = *state;
-    if ((before & kGiveUp) || (BIG && !(before & kBigColumn))) return;
+    if ((before & kGiveUp) || (WHICH == kBig && !(before & kBigColumn)) || (WHICH == kWideKeys && !(before & kWideRows)))
+        return;
     const int lane = threadIdx.x;
     unsigned int st = 0;
     for (int64_t c = blockIdx.x; c < n; c += gridDim.x) {
         const uint64_t a = place[c], b = place[c + 1];
         const int L = (int)((uint32_t)b - (uint32_t)a), nr = (int)((b >> 32) - (a >> 32));
-        if (BIG != (L > kSmallColumn)) continue;
+        if (WHICH == kWideKeys ? cnt[c] != kWide : (WHICH == kBig) != (L > kSmallColumn)) continue;
         const uint2 *ru = runs + (a >> 32);
         int32_t *tr = trow + (uint32_t)a;
         double *tv = tval + (uint32_t)a;
         int k = 0;
-        if constexpr (BIG)
-            k = L <= 512 ? sort_column<8, 10>(I, V, m, ru, nr, L, lane, lds, tr, tv, st)
-                         : sort_column<16, 10>(I, V, m, ru, nr, L, lane, lds, tr, tv, st);
+        if constexpr (WHICH == kWideKeys)
+            k = L <= 256   ? sort_column<4, 10, int64_t>(I, V, m, ru, nr, L, lane, lds, tr, tv, st)
+                : L <= 512 ? sort_column<8, 10, int64_t>(I, V, m, ru, nr, L, lane, lds, tr, tv, st)
+                           : sort_column<16, 10, int64_t>(I, V, m, ru, nr, L, lane, lds, tr, tv, st);
+        else if constexpr (WHICH == kBig)
+            k = L <= 512 ? sort_column<8, 10, int32_t>(I, V, m, ru, nr, L, lane, lds, tr, tv, st)
+                         : sort_column<16, 10, int32_t>(I, V, m, ru, nr, L, lane, lds, tr, tv, st);
         else if (L > 0)
-            k = L <= 64    ? sort_column<1, 8>(I, V, m, ru, nr, L, lane, lds, tr, tv, st)
-                : L <= 128 ? sort_column<2, 8>(I, V, m, ru, nr, L, lane, lds, tr, tv, st)
-                           : sort_column<4, 8>(I, V, m, ru, nr, L, lane, lds, tr, tv, st);
+            k = L <= 64    ? sort_column<1, 8, int32_t>(I, V, m, ru, nr, L, lane, lds, tr, tv, st)
+                : L <= 128 ? sort_column<2, 8, int32_t>(I, V, m, ru, nr, L, lane, lds, tr, tv, st)
+                           : sort_column<4, 8, int32_t>(I, V, m, ru, nr, L, lane, lds, tr, tv, st);
+        if (k == kWide) st |= kWideRows;
         if (lane == 0) cnt[c] = k;
     }
     if (st && lane == 0) atomicOr(state, st);
@@ -368,7 +388,7 @@ void fill_i64(hipStream_t s, int64_t *p, int64_t n, int64_t v) {
 }
 
 // The shorter way; null when the triples are few or not in runs, or a column is
-// too long or too wide for the wavefront sort.  Throws FEASM_EDOF for an index out
+// too long for the wavefront sort.  Throws FEASM_EDOF for an index out
 // of range, as the general way does.
 static feasm_matrix *sparse_by_columns(feasm_ctx *ctx, int64_t nt, const int32_t *I, const int32_t *J, const double *V,
                                        int64_t m, int64_t n) {
@@ -408,8 +428,9 @@ static feasm_matrix *sparse_by_columns(feasm_ctx *ctx, int64_t nt, const int32_t
                            dp<uint2>(runs), dp<int32_t>(cnt), dp<int32_t>(trow), dp<double>(tval), state);
         FEASM_HIP(hipGetLastError());
     };
-    columns(k_columns<false>, 1u << 17);
-    columns(k_columns<true>, 1u << 11);  // what the LDS of 256 CUs holds; most matrices have no such column
+    columns(k_columns<kSmall>, 1u << 17);
+    columns(k_columns<kBig>, 1u << 11);  // what the LDS of 256 CUs holds; most matrices have no such column
+    columns(k_columns<kWideKeys>, 1u << 11);
     std::unique_ptr<feasm_matrix> M(new feasm_matrix);
     M->ctx = ctx;
     M->m = m;

@@ -187,7 +187,7 @@ __device__ __forceinline__ int adj_registers(const uint32_t *__restrict__ n2e, c
         const int i = lane + 64 * m;
         x[m] = i < L ? (conn[(int64_t)(n2e[s0 + i / npe] >> 4) * npe + i % npe] << S) | (S ? i : 0) : kPad;
     }
-    wave_sort<E>(x, lane);
+    wave_sort(x, lane);
     const int tot = wave_unique<E, S>(x, lane, L, out, mult);
     if (S && contrib) {
 #pragma unroll

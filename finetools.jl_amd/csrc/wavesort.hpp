@@ -16,8 +16,8 @@ __device__ __forceinline__ void wave_fence() {
 // registers: lane l holds entries l + 64 m.  Partners less than 64 apart
 // are exchanged with lane shuffles, partners 64 or more apart sit in two
 // registers of the same lane.
-template <int E>
-__device__ __forceinline__ void wave_sort(int32_t (&x)[E], int lane) {
+template <int E, typename T>
+__device__ __forceinline__ void wave_sort(T (&x)[E], int lane) {
 #pragma unroll
     for (int k = 2; k <= 64 * E; k <<= 1)
 #pragma unroll
@@ -29,9 +29,9 @@ __device__ __forceinline__ void wave_sort(int32_t (&x)[E], int lane) {
                     const int mp = m ^ jj;
                     if (mp > m) {
                         const bool up = ((lane + 64 * m) & k) == 0;
-                        int32_t &a = x[m];
-                        int32_t &b = x[mp < E ? mp : m];
-                        const int32_t lo = min(a, b), hi = max(a, b);
+                        T &a = x[m];
+                        T &b = x[mp < E ? mp : m];
+                        const T lo = min(a, b), hi = max(a, b);
                         a = up ? lo : hi;
                         b = up ? hi : lo;
                     }
@@ -40,7 +40,7 @@ __device__ __forceinline__ void wave_sort(int32_t (&x)[E], int lane) {
 #pragma unroll
                 for (int m = 0; m < E; m++) {
                     const int i = lane + 64 * m;
-                    const int32_t y = lane_xor(x[m], j, lane);
+                    const T y = lane_xor(x[m], j, lane);
                     const bool take_min = ((i & k) == 0) == ((i & j) == 0);
                     x[m] = take_min ? min(x[m], y) : max(x[m], y);
                 }

@@ -91,3 +91,20 @@ def test_indices_out_of_range(ctx, hiprt, bad):
     finally:
         buf.free()
     assert rc == L.EDOF and not h.value
+
+
+@pytest.mark.parametrize("length", [30, 200, 256, 257, 500, 600, 1024])
+@pytest.mark.parametrize("span", [(1 << 21) - 2, (1 << 21) + 5, (1 << 23) - 2, (1 << 23) + 5, (1 << 31) - 1])
+def test_rows_far_apart_beside_others(ctx, length, span):
+    """Some columns have rows too far apart for 31-bit keys (20 bits and more
+    beside the place in the column), the others do not."""
+    rng = np.random.default_rng(length)
+    I, J, V = runs(rng, np.arange(1, 9), [length] * 8, 50)
+    far = [np.flatnonzero(J == c)[-1] for c in (2, 5, 8)]
+    I[far] = span
+    I[np.flatnonzero(J == 3)[0]] = span  # at the front of a column
+    i, j = in_runs(rng, LEAST, 900, 24)
+    order = rng.permutation(2)
+    parts = [(I, J, V), (i, j + 8, values(rng, LEAST))]
+    I, J, V = (np.concatenate([parts[k][x] for k in order]) for x in range(3))
+    check(ctx, I, J, V, span, 910)
