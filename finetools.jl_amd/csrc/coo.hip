@@ -79,12 +79,26 @@ __global__ void k_seg_sum(const uint64_t *__restrict__ keys, const uint32_t *__r
     }
 }
 
+// One thread per segment fills the column pointers since the last column; a gap
+// of many empty columns is the whole wavefront's (25 ns a column for one thread).
 __global__ void k_colptr(const uint64_t *__restrict__ keys, const int64_t *__restrict__ start, int64_t nnz,
                          int64_t m, int64_t n, int64_t *__restrict__ colptr) {
-    for (int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; s <= nnz; s += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t c = (s < nnz) ? (int64_t)(keys[start[s]] / (uint64_t)m) : n;
-        const int64_t prev = (s == 0) ? -1 : (int64_t)(keys[start[s - 1]] / (uint64_t)m);
-        for (int64_t j = prev + 1; j <= c; j++) colptr[j] = s;
+    const int lane = threadIdx.x & 63;
+    for (int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; s - lane <= nnz;
+         s += (int64_t)gridDim.x * blockDim.x) {
+        int64_t c = -1, prev = -1;
+        if (s <= nnz) {
+            c = (s < nnz) ? (int64_t)(keys[start[s]] / (uint64_t)m) : n;
+            prev = (s == 0) ? -1 : (int64_t)(keys[start[s - 1]] / (uint64_t)m);
+        }
+        const bool gap = c - prev > 16;
+        if (!gap)
+            for (int64_t j = prev + 1; j <= c; j++) colptr[j] = s;
+        for (uint64_t todo = __ballot(gap); todo; todo &= todo - 1) {
+            const int l = __ffsll((unsigned long long)todo) - 1;
+            const int64_t b = __shfl(prev, l, 64), e = __shfl(c, l, 64), v = __shfl(s, l, 64);
+            for (int64_t j = b + 1 + lane; j <= e; j += 64) colptr[j] = v;
+        }
     }
 }
 
@@ -106,14 +120,22 @@ __global__ void k_fill_i64(int64_t *__restrict__ p, int64_t n, int64_t v) {
 // first triple.
 
 constexpr int kSmallColumn = 256, kMaxColumn = 1024;  // triples of one column the wavefront sorts hold
+// (longer ones -- a constraint, a vertex of 35 T10 elasticity elements -- are
+// taken out and sorted by themselves: H8 11.3 M triples with one of 5000 670 us,
+// 1060 when it sent all to the sort, after most of this way's work)
 // mean run length from which this way pays: the lists take 8 bytes a run
 constexpr int64_t kMinRun = 4;
 // state bits: a row or column out of range; a column of more than kMaxColumn
 // triples; one of more than kSmallColumn; rows of a column too far apart for
 // 31-bit keys; runs too short
-constexpr unsigned kBadRow = 1, kTooLong = 2, kBigColumn = 4, kBadColumn = 8, kShortRuns = 16, kWideRows = 32;
+constexpr unsigned kBadRow = 1, kLongColumn = 2, kBigColumn = 4, kBadColumn = 8, kShortRuns = 16, kWideRows = 32;
 // states in which this way is given up: the kernels that follow return at once
-constexpr unsigned kGiveUp = kTooLong | kBadColumn | kShortRuns;
+constexpr unsigned kGiveUp = kBadColumn | kShortRuns;
+// (also when more than half of the nt triples are in columns too long: their
+// number is the 8-byte word after the state's)
+__device__ __forceinline__ bool given_up(const unsigned int *state, int64_t nt) {
+    return (*state & kGiveUp) || 2 * reinterpret_cast<const unsigned long long *>(state)[1] > (unsigned long long)nt;
+}
 constexpr int kWide = -1;  // sort_column: the rows are too far apart for its keys
 constexpr int kSampleWindows = 256, kFarTriples = kMaxColumn;
 constexpr int64_t kMinTriples = 1 << 16;
@@ -180,7 +202,7 @@ __global__ __launch_bounds__(256) void k_run_fill(const int32_t *__restrict__ J,
                                                   const uint64_t *__restrict__ place,
                                                   unsigned long long *__restrict__ cnt, uint2 *__restrict__ runs,
                                                   const unsigned int *__restrict__ state) {
-    if (*state & kGiveUp) return;
+    if (given_up(state, nt)) return;
     const int lane = threadIdx.x & 63;
     const int64_t step = (int64_t)gridDim.x * blockDim.x;
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t - lane < nt; t += step) {
@@ -193,9 +215,11 @@ __global__ __launch_bounds__(256) void k_run_fill(const int32_t *__restrict__ J,
     }
 }
 
-// (cnt: the end of the columns' entry counts, which the scan of them reads)
+// (cnt: the end of the columns' entry counts, which the scan of them reads;
+// longs: the triples of the columns of more than kMaxColumn)
 __global__ __launch_bounds__(256) void k_col_check(const uint64_t *__restrict__ place, int64_t n, int64_t nt,
-                                                   int32_t *__restrict__ cnt, unsigned int *__restrict__ state) {
+                                                   int32_t *__restrict__ cnt, unsigned int *__restrict__ state,
+                                                   unsigned long long *__restrict__ longs) {
     unsigned st = 0;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         cnt[n] = 0;
@@ -203,7 +227,8 @@ __global__ __launch_bounds__(256) void k_col_check(const uint64_t *__restrict__ 
     }
     for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x) {
         const uint32_t L = (uint32_t)place[c + 1] - (uint32_t)place[c];
-        st |= (L > kMaxColumn ? kTooLong : 0u) | (L > kSmallColumn ? kBigColumn : 0u);
+        st |= (L > kMaxColumn ? kLongColumn : 0u) | (L > kSmallColumn ? kBigColumn : 0u);
+        if (L > kMaxColumn) atomicAdd(longs, (unsigned long long)L);  // few: each is more than 1024 triples
     }
     if (st) atomicOr(state, st);
 }
@@ -329,21 +354,24 @@ __device__ __forceinline__ int sort_column(const int32_t *__restrict__ I, const 
 // tval from its first place on, their number to cnt.
 enum { kSmall, kBig, kWideKeys };
 template <int WHICH>
-__global__ __launch_bounds__(64) void k_columns(const int32_t *__restrict__ I, const double *__restrict__ V, int64_t m,
-                                                int64_t n, const uint64_t *__restrict__ place,
+__global__ __launch_bounds__(64) void k_columns(const int32_t *__restrict__ I, const double *__restrict__ V, int64_t nt,
+                                                int64_t m, int64_t n, const uint64_t *__restrict__ place,
                                                 const uint2 *__restrict__ runs, int32_t *__restrict__ cnt,
                                                 int32_t *__restrict__ trow, double *__restrict__ tval,
                                                 unsigned int *__restrict__ state) {
     __shared__ __align__(16) int32_t lds[4 * (WHICH == kSmall ? kSmallColumn : kMaxColumn)];
     const unsigned before = *state;
-    if ((before & kGiveUp) || (WHICH == kBig && !(before & kBigColumn)) || (WHICH == kWideKeys && !(before & kWideRows)))
-        return;
+    if (given_up(state, nt) || (WHICH == kBig && !(before & kBigColumn))) return;
     const int lane = threadIdx.x;
     unsigned int st = 0;
     for (int64_t c = blockIdx.x; c < n; c += gridDim.x) {
         const uint64_t a = place[c], b = place[c + 1];
         const int L = (int)((uint32_t)b - (uint32_t)a), nr = (int)((b >> 32) - (a >> 32));
-        if (WHICH == kWideKeys ? cnt[c] != kWide : (WHICH == kBig) != (L > kSmallColumn)) continue;
+        if (WHICH == kWideKeys ? cnt[c] != kWide : (WHICH == kBig) != ((uint32_t)L > kSmallColumn)) continue;
+        if (WHICH == kBig && (uint32_t)L > kMaxColumn) {  // sorted with the other long columns' triples
+            if (lane == 0) cnt[c] = 0;
+            continue;
+        }
         const uint2 *ru = runs + (a >> 32);
         int32_t *tr = trow + (uint32_t)a;
         double *tv = tval + (uint32_t)a;
@@ -365,14 +393,58 @@ __global__ __launch_bounds__(64) void k_columns(const int32_t *__restrict__ I, c
     if (st && lane == 0) atomicOr(state, st);
 }
 
-// the columns' entries, packed
+// what the host decides by, into pinned memory: one launch for three copies
+struct ColumnsEnd {
+    int64_t nnz;
+    uint64_t nlong;
+    unsigned int state;
+};
+__global__ void k_columns_end(const int64_t *__restrict__ colptr_end, const unsigned int *__restrict__ state,
+                              ColumnsEnd *__restrict__ out) {
+    if (threadIdx.x == 0)
+        *out = ColumnsEnd{*colptr_end, reinterpret_cast<const unsigned long long *>(state)[1], *state};
+}
+
+// the triples of the columns of more than kMaxColumn
+struct InLongColumn {
+    const int32_t *J;
+    const uint64_t *place;
+    __device__ bool operator()(uint32_t t) const {
+        const int32_t j = J[t];
+        return (uint32_t)place[j + 1] - (uint32_t)place[j] > (uint32_t)kMaxColumn;
+    }
+};
+
+__global__ __launch_bounds__(256) void k_take(const uint32_t *__restrict__ at, int64_t n, const int32_t *__restrict__ I,
+                                              const int32_t *__restrict__ J, const double *__restrict__ V,
+                                              int32_t *__restrict__ i, int32_t *__restrict__ j,
+                                              double *__restrict__ v) {
+    for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x) {
+        const uint32_t t = at[k];
+        i[k] = I[t];
+        j[k] = J[t];
+        v[k] = V[t];
+    }
+}
+
+// the long columns' entry counts, from the matrix of their triples
+__global__ __launch_bounds__(256) void k_long_counts(const int64_t *__restrict__ colptr, int64_t n,
+                                                     int32_t *__restrict__ cnt) {
+    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x)
+        if (colptr[c + 1] != colptr[c]) cnt[c] = (int32_t)(colptr[c + 1] - colptr[c]);
+}
+
+// the columns' entries, packed; LONG: the long columns' alone, from the matrix of
+// their triples (place: its column pointers)
+template <bool LONG>
 __global__ __launch_bounds__(256) void k_columns_pack(const uint64_t *__restrict__ place, int64_t n, const int64_t *__restrict__ colptr,
                                                       const int32_t *__restrict__ trow, const double *__restrict__ tval,
                                                       int32_t *__restrict__ rowval, double *__restrict__ nzval) {
     const int lane = threadIdx.x & 63;
     for (int64_t c = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6; c < n;
          c += ((int64_t)gridDim.x * blockDim.x) >> 6) {
-        const int64_t src = (uint32_t)place[c], dst = colptr[c], k = colptr[c + 1] - dst;
+        const int64_t src = LONG ? (int64_t)place[c] : (int64_t)(uint32_t)place[c], dst = colptr[c];
+        const int64_t k = LONG ? (int64_t)(place[c + 1] - place[c]) : colptr[c + 1] - dst;
         for (int64_t i = lane; i < k; i += 64) {
             rowval[dst + i] = trow[src + i];
             nzval[dst + i] = tval[src + i];
@@ -387,8 +459,11 @@ void fill_i64(hipStream_t s, int64_t *p, int64_t n, int64_t v) {
     FEASM_HIP(hipGetLastError());
 }
 
-// The shorter way; null when the triples are few or not in runs, or a column is
-// too long for the wavefront sort.  Throws FEASM_EDOF for an index out
+static feasm_matrix *sparse_by_sort(feasm_ctx *ctx, int64_t nt, const int32_t *I, const int32_t *J, const double *V,
+                                    int64_t m, int64_t n);
+
+// The shorter way; null when the triples are few or not in runs, or most are in
+// columns too long for the wavefront sort.  Throws FEASM_EDOF for an index out
 // of range, as the general way does.
 static feasm_matrix *sparse_by_columns(feasm_ctx *ctx, int64_t nt, const int32_t *I, const int32_t *J, const double *V,
                                        int64_t m, int64_t n) {
@@ -401,15 +476,17 @@ static feasm_matrix *sparse_by_columns(feasm_ctx *ctx, int64_t nt, const int32_t
     // A look at a few of the triples first: what this way does before it knows
     // all the runs (an atomic a run, two passes over the columns) would cost
     // triples in no order half of their sort again (11.3 M: 1030 us, 560 more).
-    unsigned int *sample = static_cast<unsigned int *>(pinned_buffer(2 * sizeof(unsigned int)));
+    void *const pinned = pinned_buffer(sizeof(ColumnsEnd));
+    unsigned int *sample = static_cast<unsigned int *>(pinned);
     hipLaunchKernelGGL(k_run_sample, dim3(1), dim3(1024), 0, s, J, nt, sample);
     FEASM_HIP(hipGetLastError());
     FEASM_HIP(hipStreamSynchronize(s));
     const int64_t seen = std::min<int64_t>(nt, 64 * kSampleWindows);
     if (seen < kMinRun * (int64_t)sample[0] || 2 * (int64_t)sample[1] > seen) return nullptr;
-    DevPtr ccnt = dev_alloc((n + 2) * 8), place = dev_alloc((n + 1) * 8);
+    DevPtr ccnt = dev_alloc((n + 3) * 8), place = dev_alloc((n + 1) * 8);
     unsigned int *state = reinterpret_cast<unsigned int *>(dp<int64_t>(ccnt) + n + 1);
-    fill_i64(s, dp<int64_t>(ccnt), n + 2, 0);
+    unsigned long long *longs = dp<unsigned long long>(ccnt) + n + 2;  // where given_up() looks
+    fill_i64(s, dp<int64_t>(ccnt), n + 3, 0);
     const unsigned gt = grid_for(nt, 256, 1u << 14);
     hipLaunchKernelGGL(k_run_count, dim3(gt), dim3(256), 0, s, J, nt, n, dp<unsigned long long>(ccnt), state);
     FEASM_HIP(hipGetLastError());
@@ -418,36 +495,72 @@ static feasm_matrix *sparse_by_columns(feasm_ctx *ctx, int64_t nt, const int32_t
     exclusive_scan_i64(ctx, dp<int64_t>(ccnt), dp<int64_t>(place), n + 1);
     DevPtr cnt = dev_alloc((n + 1) * 4), trow = dev_alloc(nt * 4), tval = dev_alloc(nt * 8);
     hipLaunchKernelGGL(k_col_check, dim3(grid_for(n, 256)), dim3(256), 0, s, dp<uint64_t>(place), n, nt,
-                       dp<int32_t>(cnt), state);
+                       dp<int32_t>(cnt), state, longs);
     DevPtr runs = dev_alloc(std::max<int64_t>(nt / kMinRun, 1) * sizeof(uint2));  // k_col_check: no more of them
     hipLaunchKernelGGL(k_run_fill, dim3(gt), dim3(256), 0, s, J, nt, dp<uint64_t>(place),
                        dp<unsigned long long>(ccnt), dp<uint2>(runs), state);
     FEASM_HIP(hipGetLastError());
     const auto columns = [&](auto kern, unsigned most) {
-        hipLaunchKernelGGL(kern, dim3(grid_for(n, 1, most)), dim3(64), 0, s, I, V, m, n, dp<uint64_t>(place),
+        hipLaunchKernelGGL(kern, dim3(grid_for(n, 1, most)), dim3(64), 0, s, I, V, nt, m, n, dp<uint64_t>(place),
                            dp<uint2>(runs), dp<int32_t>(cnt), dp<int32_t>(trow), dp<double>(tval), state);
         FEASM_HIP(hipGetLastError());
     };
     columns(k_columns<kSmall>, 1u << 17);
     columns(k_columns<kBig>, 1u << 11);  // what the LDS of 256 CUs holds; most matrices have no such column
-    columns(k_columns<kWideKeys>, 1u << 11);
+
     std::unique_ptr<feasm_matrix> M(new feasm_matrix);
     M->ctx = ctx;
     M->m = m;
     M->n = n;
     M->colptr = dev_alloc((n + 1) * sizeof(int64_t));
     exclusive_scan_i32_to_i64(ctx, dp<int32_t>(cnt), dp<int64_t>(M->colptr), n + 1);
-    unsigned int st = 0;
-    const ReadBack rb[2] = {{&M->nnz, dp<int64_t>(M->colptr) + n, sizeof(int64_t)}, {&st, state, sizeof(st)}};
-    read_back(s, rb, 2);
+    hipLaunchKernelGGL(k_columns_end, dim3(1), dim3(64), 0, s, dp<int64_t>(M->colptr) + n, state,
+                       static_cast<ColumnsEnd *>(pinned));
+    FEASM_HIP(hipGetLastError());
+    FEASM_HIP(hipStreamSynchronize(s));
+    const ColumnsEnd end = *static_cast<const ColumnsEnd *>(pinned);
+    M->nnz = end.nnz;
+    const uint64_t nlong = end.nlong;
+    const unsigned int st = end.state;
     FEASM_REQUIRE(!(st & (kBadRow | kBadColumn)), FEASM_EDOF, "sparse: row or column index out of range");
-    if (st & kGiveUp) return nullptr;
+    if ((st & kGiveUp) || 2 * (int64_t)nlong > nt) return nullptr;
+    // the long columns' triples by the sort of theirs alone, in input order
+    std::unique_ptr<feasm_matrix> far;
+    if (nlong > 0) {
+        DevPtr at = dev_alloc(nlong * 4), count = dev_alloc(8);
+        DevPtr li = dev_alloc(nlong * 4), lj = dev_alloc(nlong * 4), lv = dev_alloc(nlong * 8);
+        const InLongColumn pick{J, dp<uint64_t>(place)};
+        const auto select = [&](void *tmp, size_t &bytes) {
+            FEASM_HIP(rocprim::select(tmp, bytes, rocprim::counting_iterator<uint32_t>(0), dp<uint32_t>(at),
+                                      dp<unsigned long long>(count), (size_t)nt, pick, s));
+        };
+        size_t bytes = 0;
+        select(nullptr, bytes);
+        void *tmp = ctx->scratch_get(bytes);
+        select(tmp, bytes);
+        hipLaunchKernelGGL(k_take, dim3(grid_for(nlong, 256)), dim3(256), 0, s, dp<uint32_t>(at), (int64_t)nlong, I, J, V,
+                           dp<int32_t>(li), dp<int32_t>(lj), dp<double>(lv));
+        FEASM_HIP(hipGetLastError());
+        far.reset(sparse_by_sort(ctx, nlong, dp<int32_t>(li), dp<int32_t>(lj), dp<double>(lv), m, n));
+        hipLaunchKernelGGL(k_long_counts, dim3(grid_for(n, 256)), dim3(256), 0, s, dp<int64_t>(far->colptr), n,
+                           dp<int32_t>(cnt));
+        FEASM_HIP(hipGetLastError());
+    }
+    if (nlong > 0 || (st & kWideRows)) {  // the entry counts are complete now
+        if (st & kWideRows) columns(k_columns<kWideKeys>, 1u << 11);
+        exclusive_scan_i32_to_i64(ctx, dp<int32_t>(cnt), dp<int64_t>(M->colptr), n + 1);
+        read_back(s, &M->nnz, dp<int64_t>(M->colptr) + n, sizeof(int64_t));
+    }
     M->rowval = dev_alloc(std::max<int64_t>(M->nnz, 1) * sizeof(int32_t));
     M->nzval = dev_alloc(std::max<int64_t>(M->nnz, 1) * sizeof(double));
-    hipLaunchKernelGGL(k_columns_pack, dim3(grid_for(n, 4)), dim3(256), 0, s, dp<uint64_t>(place), n,
-                       dp<int64_t>(M->colptr), dp<int32_t>(trow), dp<double>(tval), dp<int32_t>(M->rowval),
-                       dp<double>(M->nzval));
-    FEASM_HIP(hipGetLastError());
+    const auto pack = [&](auto kern, const void *from, const DevPtr &row, const DevPtr &val) {
+        hipLaunchKernelGGL(kern, dim3(grid_for(n, 4)), dim3(256), 0, s, static_cast<const uint64_t *>(from), n,
+                           dp<int64_t>(M->colptr), dp<int32_t>(row), dp<double>(val), dp<int32_t>(M->rowval),
+                           dp<double>(M->nzval));
+        FEASM_HIP(hipGetLastError());
+    };
+    pack(k_columns_pack<false>, place->p, trow, tval);
+    if (far) pack(k_columns_pack<true>, far->colptr->p, far->rowval, far->nzval);
     FEASM_HIP(hipStreamSynchronize(s));
     return M.release();
 }
@@ -520,28 +633,15 @@ void check_sparse_args(int64_t nt, int64_t m, int64_t n) {
     FEASM_REQUIRE(nt == 0 || (m >= 1 && n >= 1), FEASM_EDOF, "sparse: row or column index out of range");
 }
 
-feasm_matrix *sparse_device(feasm_ctx *ctx, int64_t nt, const int32_t *I, const int32_t *J, const double *V,
-                            int64_t m, int64_t n) {
-    check_sparse_args(nt, m, n);
+// The radix sort of all triples (nt > 0).
+static feasm_matrix *sparse_by_sort(feasm_ctx *ctx, int64_t nt, const int32_t *I, const int32_t *J, const double *V,
+                                    int64_t m, int64_t n) {
     hipStream_t s = ctx->stream;
-    if (nt > 0) {
-        try {
-            if (feasm_matrix *M = sparse_by_columns(ctx, nt, I, J, V, m, n)) return M;
-        } catch (const Error &e) {
-            if (e.code != FEASM_ENOMEM) throw;  // 20 bytes a column more than the sort takes
-        }
-    }
     std::unique_ptr<feasm_matrix> M(new feasm_matrix);
     M->ctx = ctx;
     M->m = m;
     M->n = n;
     M->colptr = dev_alloc((n + 1) * sizeof(int64_t));
-    if (nt == 0) {
-        fill_i64(s, dp<int64_t>(M->colptr), n + 1, 0);
-        FEASM_HIP(hipStreamSynchronize(s));
-        M->nnz = 0;
-        return M.release();
-    }
     const unsigned end_bit = (unsigned)bits_for((uint64_t)m * (uint64_t)n);
     SparseWork w;
     DevPtr keys = dev_alloc(nt * sizeof(uint64_t)), keys2 = dev_alloc(nt * sizeof(uint64_t));
@@ -563,6 +663,28 @@ feasm_matrix *sparse_device(feasm_ctx *ctx, int64_t nt, const int32_t *I, const 
     M->nzval = dev_alloc(nnz * sizeof(double));
     sparse_phase_b(s, nt, V, m, n, nnz, w, dp<int64_t>(M->colptr), dp<int32_t>(M->rowval), dp<double>(M->nzval));
     FEASM_HIP(hipStreamSynchronize(s));
+    return M.release();
+}
+
+feasm_matrix *sparse_device(feasm_ctx *ctx, int64_t nt, const int32_t *I, const int32_t *J, const double *V,
+                            int64_t m, int64_t n) {
+    check_sparse_args(nt, m, n);
+    if (nt > 0) {
+        try {
+            if (feasm_matrix *M = sparse_by_columns(ctx, nt, I, J, V, m, n)) return M;
+        } catch (const Error &e) {
+            if (e.code != FEASM_ENOMEM) throw;  // it takes more than the sort in a matrix of many columns
+        }
+        return sparse_by_sort(ctx, nt, I, J, V, m, n);
+    }
+    std::unique_ptr<feasm_matrix> M(new feasm_matrix);
+    M->ctx = ctx;
+    M->m = m;
+    M->n = n;
+    M->nnz = 0;
+    M->colptr = dev_alloc((n + 1) * sizeof(int64_t));
+    fill_i64(ctx->stream, dp<int64_t>(M->colptr), n + 1, 0);
+    FEASM_HIP(hipStreamSynchronize(ctx->stream));
     return M.release();
 }
 

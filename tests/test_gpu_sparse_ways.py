@@ -94,7 +94,7 @@ def test_indices_out_of_range(ctx, hiprt, bad):
 
 
 @pytest.mark.parametrize("length", [30, 200, 256, 257, 500, 600, 1024])
-@pytest.mark.parametrize("span", [(1 << 21) - 2, (1 << 21) + 5, (1 << 23) - 2, (1 << 23) + 5, (1 << 31) - 1])
+@pytest.mark.parametrize("span", [(1 << 21) - 2, (1 << 21) + 5, (1 << 23) - 2, (1 << 23) + 5, (1 << 26) + 1])
 def test_rows_far_apart_beside_others(ctx, length, span):
     """Some columns have rows too far apart for 31-bit keys (20 bits and more
     beside the place in the column), the others do not."""
@@ -108,3 +108,45 @@ def test_rows_far_apart_beside_others(ctx, length, span):
     parts = [(I, J, V), (i, j + 8, values(rng, LEAST))]
     I, J, V = (np.concatenate([parts[k][x] for k in order]) for x in range(3))
     check(ctx, I, J, V, span, 910)
+
+
+@pytest.mark.parametrize("lengths", [[1025], [1024, 1025, 5000], [3000] * 9, [40000]])
+@pytest.mark.parametrize("where", ["first", "last", "spread"])
+def test_long_columns_beside_others(ctx, lengths, where):
+    """Columns of more than 1024 triples are sorted apart from the others."""
+    rng = np.random.default_rng(len(lengths))
+    n = 5000
+    at = {"first": np.arange(len(lengths)), "last": n - 1 - np.arange(len(lengths)),
+          "spread": 3 + 500 * np.arange(len(lengths))}[where]
+    I, J, V = runs(rng, at + 1, lengths, 700)
+    i, j = in_runs(rng, LEAST, n, 24)
+    parts = [(I, J, V), (i, j, values(rng, LEAST))]
+    for order in ([0, 1], [1, 0]):
+        a, b, c = (np.concatenate([parts[k][x] for k in order]) for x in range(3))
+        check(ctx, a, b, c, n, n)
+
+
+@pytest.mark.parametrize("share", [1, 3])
+def test_most_triples_in_long_columns(ctx, share):
+    """Up to half of the triples in long columns, and more than that."""
+    rng = np.random.default_rng(share)
+    nt = 40000 * share
+    I, J = rng.integers(1, 901, nt), np.repeat(rng.integers(1, 8, nt // 16), 16)
+    i, j = in_runs(rng, LEAST, 900, 24)
+    check(ctx, np.r_[i, I], np.r_[j + 50, J], values(rng, nt + LEAST), 900, 1000)
+
+
+def test_row_out_of_range_in_a_long_column(ctx, hiprt):
+    rng = np.random.default_rng(6)
+    i, j = in_runs(rng, LEAST, 400, 24)
+    i0 = np.r_[i, rng.integers(1, 401, 2000)].astype(np.int32) - 1
+    j0 = np.r_[j, np.full(2000, 17)].astype(np.int32) - 1
+    i0[-5] = 400
+    buf = DeviceBuffers(hiprt)
+    try:
+        d = [buf.upload(a) for a in (i0, j0, values(rng, len(i0)))]
+        h = ctypes.c_void_p()
+        rc = L.lib().feasm_sparse_device(ctx.h, len(i0), *d, 400, 400, ctypes.byref(h))
+    finally:
+        buf.free()
+    assert rc == L.EDOF and not h.value
