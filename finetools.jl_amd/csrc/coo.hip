@@ -125,10 +125,9 @@ constexpr int kSmallColumn = 256, kMaxColumn = 1024;  // triples of one column t
 // 1060 when it sent all to the sort, after most of this way's work)
 // mean run length from which this way pays: the lists take 8 bytes a run
 constexpr int64_t kMinRun = 4;
-// state bits: a row or column out of range; a column of more than kMaxColumn
-// triples; one of more than kSmallColumn; rows of a column too far apart for
-// 31-bit keys; runs too short
-constexpr unsigned kBadRow = 1, kLongColumn = 2, kBigColumn = 4, kBadColumn = 8, kShortRuns = 16, kWideRows = 32;
+// state bits: a row or column out of range; a column of more than kSmallColumn
+// triples; rows of a column too far apart for 31-bit keys; runs too short
+constexpr unsigned kBadRow = 1, kBadColumn = 2, kBigColumn = 4, kWideRows = 8, kShortRuns = 16;
 // states in which this way is given up: the kernels that follow return at once
 constexpr unsigned kGiveUp = kBadColumn | kShortRuns;
 // (also when more than half of the nt triples are in columns too long: their
@@ -227,7 +226,7 @@ __global__ __launch_bounds__(256) void k_col_check(const uint64_t *__restrict__ 
     }
     for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x) {
         const uint32_t L = (uint32_t)place[c + 1] - (uint32_t)place[c];
-        st |= (L > kMaxColumn ? kLongColumn : 0u) | (L > kSmallColumn ? kBigColumn : 0u);
+        st |= L > kSmallColumn ? kBigColumn : 0u;
         if (L > kMaxColumn) atomicAdd(longs, (unsigned long long)L);  // few: each is more than 1024 triples
     }
     if (st) atomicOr(state, st);

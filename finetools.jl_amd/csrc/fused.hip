@@ -771,18 +771,32 @@ __device__ __forceinline__ void load_tables(const FusedParams &kp, unsigned char
 // XCD-aware persistent walk: consecutive workgroups land on different XCDs,
 // so each XCD takes a contiguous range of the (Morton-ordered) tile list.  The
 // workgroups stride through the first kAhead tiles each; the rest of a range
-// (QUEUE: at least kAhead tiles per workgroup) is handed out one tile at a
+// (QUEUE: queue_tiles() per workgroup at least) is handed out one tile at a
 // time, and a workgroup whose range has run out goes on with the next one's:
 // tiles differ in time (T10: by a quarter of the mean), and with a fixed stride
 // the last workgroup ended 20 % (T10), 5 % (H8) after the mean.  Measured: H8
 // elasticity, 1M elements 1010 -> 984 us, T10 elasticity, 178k elements 233 ->
-// 216.  With fewer tiles there is nothing to hand out, and the stride alone
-// (scalar header loads, no claims) is 0.4 us shorter in launches of 8 to 18 us.
+// 216.
 //
 // A workgroup runs tile t, loads the blob of t1, reads the header of t2 and
 // claims the tile after it.  One lane claims: the atomic is issued before phase
 // 1 and its result goes to the other wavefronts through LDS.
 constexpr int kAhead = 3;
+// Tiles per workgroup from which a launch hands its tiles out, 0 for never.
+// The claim costs a tile of 4 to 15 us up to 0.3 us, and what it evens out is a
+// part of the last tile.  Times with the queue against the stride's, at these
+// tiles per workgroup:
+//   FP64 gradient records   H8 3.7 1.05, 8.6 .99, 45 .98; T10 6 .97, 12 .95, 26 .87
+//   packed                  4.3 1.11, 11 .99, 24 .94
+//   DOT of 2 or 3           H8 4 1.10, 9 1.01, 17 .98; T10 5 1.08, 9 1.01, 18 .97
+//   FP32 gradient records   H8 4.5 1.04, 9 1.00, 48 .98; T10 5 1.04, 9 1.05, 18 .97
+//   DOT of 1                H8 (4 us a tile) 4 1.24, 17 1.05, 99 1.00 (FP32 1.36, 1.25, 1.25);
+//                           T10 9 1.03, 18 1.01, 38 .98
+constexpr int queue_tiles(int npe, int form, int ndn, size_t rbytes) {
+    if (form == FEASM_FORM_DOT && ndn == 1) return npe == 8 ? 0 : 32;
+    const bool packed = npe == 8 && (form == FEASM_FORM_DIFFUSION_ISO || form == FEASM_FORM_DIFFUSION_MAT);
+    return rbytes == 8 && form != FEASM_FORM_DOT && !packed ? 6 : 12;
+}
 constexpr int kQueuePad = 32;  // words between counters: a cache line each
 template <bool QUEUE>
 struct TileWalk {
@@ -1430,13 +1444,15 @@ template <int NPE, int NQP, int FORM, int NDN, typename R>
 void go(feasm_ctx *ctx, const feasm_mesh *m, const Pattern &p, const TileSet &t, const FusedParams &kp,
         double *nzval) {
     constexpr bool PACKED = NPE == 8 && sizeof(R) == 8 && (FORM == FEASM_FORM_DIFFUSION_ISO || FORM == FEASM_FORM_DIFFUSION_MAT);
+    constexpr int QT = queue_tiles(NPE, FORM, NDN, sizeof(R));
+    static_assert(QT == 0 || QT >= kAhead, "a workgroup strides through its first tiles");
     const unsigned grid = persistent_grid(ctx, t.shape.budget, t.ntiles);
-    uint32_t *queue = t.ntiles >= (int64_t)kAhead * grid ? ctx_tile_queue(ctx) : nullptr;
+    uint32_t *queue = QT > 0 && t.ntiles >= (int64_t)QT * grid ? ctx_tile_queue(ctx) : nullptr;
     auto kern = [&] {
         if constexpr (PACKED)
             return queue ? k_packed<NPE, NQP, FORM, NDN, R, true> : k_packed<NPE, NQP, FORM, NDN, R, false>;
         else
-            return queue ? k_fused<NPE, NQP, FORM, NDN, R, true> : k_fused<NPE, NQP, FORM, NDN, R, false>;
+            return queue ? k_fused<NPE, NQP, FORM, NDN, R, QT != 0> : k_fused<NPE, NQP, FORM, NDN, R, false>;
     }();
     const int budget = (int)t.shape.budget;
     FEASM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, budget));
@@ -1479,7 +1495,8 @@ void go_batch(feasm_ctx *ctx, const BatchLaunch &b) {
         if constexpr (PACKED)
             return b.queue ? k_packed_batch<NPE, NQP, FORM, NDN, R, true> : k_packed_batch<NPE, NQP, FORM, NDN, R, false>;
         else
-            return b.queue ? k_fused_batch<NPE, NQP, FORM, NDN, R, true> : k_fused_batch<NPE, NQP, FORM, NDN, R, false>;
+            return b.queue ? k_fused_batch<NPE, NQP, FORM, NDN, R, queue_tiles(NPE, FORM, NDN, sizeof(R)) != 0>
+                           : k_fused_batch<NPE, NQP, FORM, NDN, R, false>;
     }();
     FEASM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b.budget));
     hipLaunchKernelGGL(kern, dim3(b.grid), dim3(b.threads), b.budget, ctx->stream,
@@ -1530,7 +1547,8 @@ void prepare_batch_launch(feasm_ctx *ctx, BatchLaunch &b, const std::vector<Batc
                                  (size_t)items[i].tiles->ntiles * sizeof(TileHdr), hipMemcpyDeviceToDevice,
                                  ctx->stream));
     b.grid = persistent_grid(ctx, b.budget, b.ntiles);
-    if (b.ntiles >= (int64_t)kAhead * b.grid) {
+    const int qt = queue_tiles(b.npe, b.kform, b.ndn, (size_t)b.rbytes);
+    if (qt > 0 && b.ntiles >= (int64_t)qt * b.grid) {
         b.queue = dev_alloc(kQueueBytes);
         FEASM_HIP(hipMemsetAsync(b.queue->p, 0, kQueueBytes, ctx->stream));
     }

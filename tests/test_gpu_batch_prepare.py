@@ -25,8 +25,8 @@ def test_first_run_of_new_batches(ctx):
         batch = core.Batch(ctx)
         for i, m in enumerate(mesh):
             batch.add(m, L.DIFFUSION_ISO, L.RULE_GAUSS, 2, [1.0 + i], L.FP64)
-        batch.prepare(use_graph=False, max_nodes=4)
-        assert batch.stats()["tiles"] >= 3 * 512  # three tiles a workgroup, two workgroups a CU: the queue is on
+        batch.prepare(use_graph=False, max_nodes=2)
+        assert batch.stats()["tiles"] >= 12 * 512  # 12 tiles a workgroup, two workgroups a CU: the queue is on
         # another entry drops the launches: the next run makes them again and starts at once
         batch.add(mesh[0], L.DIFFUSION_ISO, L.RULE_GAUSS, 2, [7.0], L.FP64)
         batch.run()
