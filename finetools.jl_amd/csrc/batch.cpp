@@ -13,6 +13,7 @@
 #include <atomic>
 #include <fstream>
 #include <thread>
+#include <set>
 #include <sstream>
 
 #include "common.hpp"
@@ -301,9 +302,12 @@ extern "C" int feasm_batch_stats(feasm_batch *b, int64_t *nmeshes, int64_t *nele
     B_CATCH(b ? b->ctx : nullptr)
 }
 
-// Autotuner: tries tile sizes (owned nodes per tile) and LDS budgets per
-// workgroup (one or two workgroups per CU), times `reps` direct runs of each
-// after one warm-up, keeps the fastest.  Results are appended to a small text
+// Autotuner: tries tile sizes (owned nodes per tile), LDS budgets per
+// workgroup (one or two workgroups per CU) and threads, times `reps` direct runs
+// of each after one warm-up, keeps the fastest.  Candidates that give every mesh
+// the tile shape of an earlier one (the packed kernels have one budget and one
+// number of threads) are not run again, and the budget and threads kept are
+// those of the shapes where the meshes agree on them.  Results are appended to a small text
 // database (one line per key: "key max_nodes budget_kib ms") when db_path is
 // given, and read back from it on later calls for the same key.
 extern "C" int feasm_batch_autotune(feasm_batch *b, const char *db_path, const char *key, int reps, int *best_nodes,
@@ -339,20 +343,31 @@ extern "C" int feasm_batch_autotune(feasm_batch *b, const char *db_path, const c
     const int thr_c[] = {512, 1024};
     double best = 1e300;
     int bn = 64, bk = 160, bt = 1024;
+    std::set<std::vector<int64_t>> tried;
     for (int th : thr_c)
         for (int kb : kib_c)
             for (int n : nodes_c) {
                 b->max_nodes = n;
                 b->budget = (size_t)kb * 1024;
                 b->threads = th;
+                std::vector<int64_t> keys;
+                bool one_budget = true, one_threads = true;
+                const TileShape s0 = shape_for(b, b->items[0]);
+                for (auto &it : b->items) {
+                    const TileShape s = shape_for(b, it);
+                    keys.push_back(s.key());
+                    one_budget &= s.budget == s0.budget;
+                    one_threads &= s.threads == s0.threads;
+                }
+                if (!tried.insert(std::move(keys)).second) continue;
                 prepare(b);
                 run_direct(b);  // warm-up
                 const double ms = time_runs(b, reps);
                 if (ms < best) {
                     best = ms;
                     bn = n;
-                    bk = kb;
-                    bt = th;
+                    bk = one_budget ? (int)(s0.budget / 1024) : kb;
+                    bt = one_threads ? s0.threads : th;
                 }
             }
     b->max_nodes = bn;

@@ -174,7 +174,7 @@ int feasm_bilform_coo(feasm_mesh *mesh, int form, int rule, int order, const dou
 int feasm_mesh_set_numeric_path(feasm_mesh *mesh, int path);
 /* Tile parameters of the fused kernel for this mesh (0 = default):
  * owned nodes per tile (<= 255), LDS per workgroup in KiB, threads (256/512/1024;
- * H8 FP64 scalar diffusion always runs 256). */
+ * H8 FP64 diffusion always runs 256, and takes at most 80 KiB). */
 int feasm_mesh_set_tile_params(feasm_mesh *mesh, int max_nodes, int budget_kib, int threads);
 /* Tiles built for the fused kernel so far (summed over forms/precisions). */
 int feasm_mesh_tile_info(feasm_mesh *mesh, int64_t *ntiles, int64_t *nhalo);
