@@ -792,10 +792,18 @@ constexpr int kAhead = 3;
 //   FP32 gradient records   H8 4.5 1.04, 9 1.00, 48 .98; T10 5 1.04, 9 1.05, 18 .97
 //   DOT of 1                H8 (4 us a tile) 4 1.24, 17 1.05, 99 1.00 (FP32 1.36, 1.25, 1.25);
 //                           T10 9 1.03, 18 1.01, 38 .98
-constexpr int queue_tiles(int npe, int form, int ndn, size_t rbytes) {
-    if (form == FEASM_FORM_DOT && ndn == 1) return npe == 8 ? 0 : 32;
-    const bool packed = npe == 8 && (form == FEASM_FORM_DIFFUSION_ISO || form == FEASM_FORM_DIFFUSION_MAT);
-    return rbytes == 8 && form != FEASM_FORM_DOT && !packed ? 6 : 12;
+// and in a batch of 24 uneven meshes, whose tiles differ more:
+//   FP32 gradient records   H8 5 .94, 13 .97, 22 .91; T10 5 .97, 9 1.00, 37 .93
+//   FP64 ones and packed    H8 7 1.02, 11 1.00, 19 .97, 34 .93; T10 5 1.01, 9 .99, 42 .95
+//   DOT of 2 or 3           H8 6 1.07, 11 .94, 47 .97; T10 10 1.02, 18 .99, 76 .91
+//   DOT of 1                H8 11 1.03, 47 1.02, 157 .99; T10 18 1.00, 40 .99, 76 .94
+constexpr int queue_tiles(int npe, int form, int ndn, size_t rbytes, bool batch) {
+    if (form == FEASM_FORM_DOT && ndn == 1) return npe == 10 ? 32 : batch ? 128 : 0;
+    if (form == FEASM_FORM_DOT) return batch ? 10 : 12;
+    const bool packed =
+        npe == 8 && rbytes == 8 && (form == FEASM_FORM_DIFFUSION_ISO || form == FEASM_FORM_DIFFUSION_MAT);
+    if (batch) return rbytes == 8 ? 8 : 4;
+    return rbytes == 8 && !packed ? 6 : 12;
 }
 constexpr int kQueuePad = 32;  // words between counters: a cache line each
 template <bool QUEUE>
@@ -1444,7 +1452,7 @@ template <int NPE, int NQP, int FORM, int NDN, typename R>
 void go(feasm_ctx *ctx, const feasm_mesh *m, const Pattern &p, const TileSet &t, const FusedParams &kp,
         double *nzval) {
     constexpr bool PACKED = NPE == 8 && sizeof(R) == 8 && (FORM == FEASM_FORM_DIFFUSION_ISO || FORM == FEASM_FORM_DIFFUSION_MAT);
-    constexpr int QT = queue_tiles(NPE, FORM, NDN, sizeof(R));
+    constexpr int QT = queue_tiles(NPE, FORM, NDN, sizeof(R), false);
     static_assert(QT == 0 || QT >= kAhead, "a workgroup strides through its first tiles");
     const unsigned grid = persistent_grid(ctx, t.shape.budget, t.ntiles);
     uint32_t *queue = QT > 0 && t.ntiles >= (int64_t)QT * grid ? ctx_tile_queue(ctx) : nullptr;
@@ -1495,8 +1503,7 @@ void go_batch(feasm_ctx *ctx, const BatchLaunch &b) {
         if constexpr (PACKED)
             return b.queue ? k_packed_batch<NPE, NQP, FORM, NDN, R, true> : k_packed_batch<NPE, NQP, FORM, NDN, R, false>;
         else
-            return b.queue ? k_fused_batch<NPE, NQP, FORM, NDN, R, queue_tiles(NPE, FORM, NDN, sizeof(R)) != 0>
-                           : k_fused_batch<NPE, NQP, FORM, NDN, R, false>;
+            return b.queue ? k_fused_batch<NPE, NQP, FORM, NDN, R, true> : k_fused_batch<NPE, NQP, FORM, NDN, R, false>;
     }();
     FEASM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b.budget));
     hipLaunchKernelGGL(kern, dim3(b.grid), dim3(b.threads), b.budget, ctx->stream,
@@ -1547,8 +1554,7 @@ void prepare_batch_launch(feasm_ctx *ctx, BatchLaunch &b, const std::vector<Batc
                                  (size_t)items[i].tiles->ntiles * sizeof(TileHdr), hipMemcpyDeviceToDevice,
                                  ctx->stream));
     b.grid = persistent_grid(ctx, b.budget, b.ntiles);
-    const int qt = queue_tiles(b.npe, b.kform, b.ndn, (size_t)b.rbytes);
-    if (qt > 0 && b.ntiles >= (int64_t)qt * b.grid) {
+    if (b.ntiles >= (int64_t)queue_tiles(b.npe, b.kform, b.ndn, (size_t)b.rbytes, true) * b.grid) {
         b.queue = dev_alloc(kQueueBytes);
         FEASM_HIP(hipMemsetAsync(b.queue->p, 0, kQueueBytes, ctx->stream));
     }
