@@ -440,7 +440,8 @@ __global__ void k_tile_starts(const uint8_t *start, const int32_t *inc, int64_t 
 }
 
 // per tile: halo-node count and slot size (for the scans), maxima for the
-// build kernel's LDS; rep_max: the most times an element lists one node
+// build kernel's LDS; rep_max: the most times an element lists one node (0 when
+// none lists a node twice)
 struct PrepStats {
     unsigned long long ntu_max, niu_max, k_max, h_max, nh_max, p_max, rep_max;
 };
@@ -472,12 +473,15 @@ __global__ __launch_bounds__(256) void k_tile_prep(const int64_t *ts, int64_t nt
                                                    int64_t *nh, int64_t *slot, PrepStats *st) {
     __shared__ unsigned long long sh[256];
     unsigned long long ntu = 0, niu = 0, km = 0, hm = 0, nhm = 0, pm = 0, rm = 1;
+    const int64_t tiles0 = blockIdx.x * (int64_t)blockDim.x;
     for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < nelem; e += (int64_t)gridDim.x * blockDim.x)
         for (int a = 0; a < npe; a++) {
             unsigned long long r = 1;
             for (int b = a + 1; b < npe; b++) r += conn[e * npe + a] == conn[e * npe + b] ? 1 : 0;
             rm = max(rm, r);
         }
+    if (rm > 1) atomicMax(&st->rep_max, rm);
+    if (tiles0 > ntiles) return;
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t <= ntiles; t += (int64_t)gridDim.x * blockDim.x) {
         if (t == ntiles) {
             nh[t] = 0;
@@ -503,7 +507,6 @@ __global__ __launch_bounds__(256) void k_tile_prep(const int64_t *ts, int64_t nt
     block_max_to(hm, &st->h_max, sh);
     block_max_to(nhm, &st->nh_max, sh);
     block_max_to(pm, &st->p_max, sh);
-    block_max_to(rm, &st->rep_max, sh);
 }
 
 // ---- 3. one tile
@@ -1403,7 +1406,7 @@ std::shared_ptr<TileSet> build_tiles_device(feasm_mesh *m, const TileShape &shap
     // a block of the nodes n and m has (times an element lists n) * (times it
     // lists m) items of each element: an element that lists a node r times
     // (a collapsed hexahedron) has r incidences of it, and r * r items
-    caps.kb = (int)std::min<unsigned long long>(255, ps.k_max * ps.rep_max);
+    caps.kb = (int)std::min<unsigned long long>(255, ps.k_max * std::max(ps.rep_max, 1ull));
     caps.nc = caps.h * npe;
     caps.nh = (int)ps.nh_max + 2;
     int words = kTB;
