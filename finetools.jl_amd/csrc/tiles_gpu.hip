@@ -468,20 +468,37 @@ __device__ void block_sum_to(unsigned long long v, unsigned long long *out, unsi
     __syncthreads();
 }
 
+// the most times one of the calling thread's elements lists one node
+template <int NPE>
+__device__ __forceinline__ int repeats(const int32_t *__restrict__ conn, int64_t nelem) {
+    int most = 1;
+    for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < nelem; e += (int64_t)gridDim.x * blockDim.x) {
+        int32_t c[NPE];
+        const int2 *row = reinterpret_cast<const int2 *>(conn + e * NPE);
+#pragma unroll
+        for (int i = 0; i < NPE / 2; i++) {
+            c[2 * i] = row[i].x;
+            c[2 * i + 1] = row[i].y;
+        }
+#pragma unroll
+        for (int a = 0; a < NPE; a++) {
+            int r = 1;
+#pragma unroll
+            for (int b = a + 1; b < NPE; b++) r += c[a] == c[b] ? 1 : 0;
+            most = max(most, r);
+        }
+    }
+    return most;
+}
+
 __global__ __launch_bounds__(256) void k_tile_prep(const int64_t *ts, int64_t ntiles, const int64_t *info,
                                                    TileShape shape, const int32_t *conn, int64_t nelem, int npe,
                                                    int64_t *nh, int64_t *slot, PrepStats *st) {
     __shared__ unsigned long long sh[256];
-    unsigned long long ntu = 0, niu = 0, km = 0, hm = 0, nhm = 0, pm = 0, rm = 1;
-    const int64_t tiles0 = blockIdx.x * (int64_t)blockDim.x;
-    for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < nelem; e += (int64_t)gridDim.x * blockDim.x)
-        for (int a = 0; a < npe; a++) {
-            unsigned long long r = 1;
-            for (int b = a + 1; b < npe; b++) r += conn[e * npe + a] == conn[e * npe + b] ? 1 : 0;
-            rm = max(rm, r);
-        }
-    if (rm > 1) atomicMax(&st->rep_max, rm);
-    if (tiles0 > ntiles) return;
+    unsigned long long ntu = 0, niu = 0, km = 0, hm = 0, nhm = 0, pm = 0;
+    const int rep = npe == 8 ? repeats<8>(conn, nelem) : repeats<10>(conn, nelem);
+    if (rep > 1) atomicMax(&st->rep_max, (unsigned long long)rep);
+    if (blockIdx.x * (int64_t)blockDim.x > ntiles) return;
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t <= ntiles; t += (int64_t)gridDim.x * blockDim.x) {
         if (t == ntiles) {
             nh[t] = 0;
