@@ -19,7 +19,9 @@
 // column by column, 24 triples at a time for an H8 elasticity element -- take a
 // shorter way (sparse_by_columns): the runs are listed by column, then one
 // wavefront per column sorts the column's rows in registers and folds the
-// duplicates, reading every triple once and in place.
+// duplicates, reading every triple once and in place.  A look at a few of the
+// triples decides; columns too long for a wavefront's registers are taken out
+// and sorted by steps 1-4 alone.
 #include "common.hpp"
 #include "wavesort.hpp"
 
@@ -149,13 +151,24 @@ __global__ __launch_bounds__(1024) void k_run_sample(const int32_t *__restrict__
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t all = (nt + 63) / 64, windows = min(all, (int64_t)kSampleWindows);
+    // all of a wavefront's stretches are loaded before any is looked at (one after
+    // the other they took 13 us, so 10)
+    constexpr int W = kSampleWindows / 16;
+    int32_t j[W], f[W];
+    bool in[W];
+#pragma unroll
+    for (int i = 0; i < W; i++) {
+        const int64_t k = wave + 16 * i, t = all * k / windows * 64 + lane;
+        in[i] = k < windows && t < nt;
+        j[i] = in[i] ? J[t] : 0;
+        f[i] = in[i] && t + kFarTriples < nt ? J[t + kFarTriples] : -1;
+    }
     unsigned int runs = 0, far = 0;
-    for (int64_t k = wave; k < windows; k += 16) {
-        const int64_t t = all * k / windows * 64 + lane;
-        const int32_t j = t < nt ? J[t] : 0, f = t + kFarTriples < nt ? J[t + kFarTriples] : ~j;
-        const int32_t prev = __shfl_up(j, 1, 64);
-        runs += (unsigned)__popcll(__ballot(t < nt && (lane == 0 || prev != j)));
-        far += (unsigned)__popcll(__ballot(t < nt && f == j));
+#pragma unroll
+    for (int i = 0; i < W; i++) {
+        const int32_t prev = __shfl_up(j[i], 1, 64);
+        runs += (unsigned)__popcll(__ballot(in[i] && (lane == 0 || prev != j[i])));
+        far += (unsigned)__popcll(__ballot(in[i] && f[i] == j[i] && j[i] >= 0));
     }
     if (lane == 0) {
         atomicAdd(&sum[0], runs);

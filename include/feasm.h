@@ -163,7 +163,7 @@ int feasm_bilform_into(feasm_mesh *mesh, int form, int rule, int order, const do
                        int precision, feasm_matrix *mat);
 /* Generic path used for numberings that share DOFs between nodes, and
  * selectable for testing: element kernels write COO triples in assemble!'s order, then the
- * device sparse() (radix sort + ordered duplicate summation). */
+ * device sparse(). */
 int feasm_bilform_coo(feasm_mesh *mesh, int form, int rule, int order, const double *coeff, int ncoeff,
                       int precision, feasm_matrix **out);
 /* Numeric path of the resident-pattern assembly: 0 automatic (the fused
@@ -302,8 +302,10 @@ int feasm_coo_makematrix(feasm_coo *coo, feasm_matrix **out);
 int64_t feasm_coo_ntriples(const feasm_coo *coo);
 int feasm_coo_destroy(feasm_coo *coo);
 /* Device sparse(I, J, V, m, n) on device arrays (0-based int32 indices):
- * stable radix sort by (col, row), duplicates summed left to right in input
- * order, explicit zeros kept -- SparseArrays.sparse as called by makematrix!. */
+ * rows sorted within columns, duplicates summed left to right in input order,
+ * explicit zeros kept -- SparseArrays.sparse as called by makematrix!.  Triples
+ * in runs of one column (an element loop's) are sorted column by column, others
+ * by a stable radix sort; the result is the same bits. */
 int feasm_sparse_device(feasm_ctx *ctx, int64_t ntrip, const int32_t *d_I, const int32_t *d_J, const double *d_V,
                         int64_t m, int64_t n, feasm_matrix **out);
 
