@@ -627,6 +627,14 @@ __device__ __forceinline__ int task_bucket(uint32_t w, int K, bool grad) {
 }
 
 constexpr uint32_t kDropBit = 1u << 27;  // builder-internal: computed by the transposed block's task
+// the bits of a task word that its bucket follows from, and bucket b's (the
+// inverse of task_order)
+constexpr uint32_t kBucketMask = (255u << 16) | (1u << 26) | kDropBit;
+__device__ __forceinline__ uint32_t bucket_word(int b, int K, bool grad) {
+    const bool sym = grad ? b <= K : !(b & 1);
+    const int k = grad ? K - (sym ? b : b - (K + 1)) : K - (b >> 1);
+    return ((uint32_t)k << 16) | (sym ? 1u << 26 : 0u);
+}
 
 // the owned column whose node block list starts at or before task u
 __device__ __forceinline__ int column_of(const uint32_t *coff, int P, int u) {
@@ -843,12 +851,15 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
     const int nsym = shape.grad ? (int)bcount[K + 1] : 0;
     __syncthreads();
     // each bucket's tasks in task order, one wavefront per bucket
+    // (a word is compared with the bucket's: its bucket computed for every pair of
+    // the two took a T10 tile 36 us instead of 24)
     for (int b = wave; b < nb; b += kTB / 64) {
         uint32_t pos = bcount[b];
+        const uint32_t want = bucket_word(b, K, shape.grad);
         for (int base = 0; base < NTu; base += 64) {
             const int u = base + lane;
             const uint32_t w = u < NTu ? word[u] : kDropBit;
-            const bool hit = !(w & kDropBit) && task_bucket(w, K, shape.grad) == b;
+            const bool hit = (w & kBucketMask) == want;
             const uint64_t mask = __ballot(hit);
             if (hit) sorted[pos + __popcll(mask & ((1ull << lane) - 1ull))] = (uint16_t)u;
             pos += (uint32_t)__popcll(mask);
@@ -963,6 +974,7 @@ __global__ __launch_bounds__(kTB) void k_tile_build(MeshView mv, const double *x
         // element's reads, then the greedy class choice, most-read first.
         uint32_t *gk = reinterpret_cast<uint32_t *>(dyn + B.gk);
         uint32_t *sinfo = reinterpret_cast<uint32_t *>(dyn + B.sinfo);  // first item | items << 16, or none
+#pragma unroll 4
         for (int sl = tid; sl < NT; sl += kTB) {
             const uint64_t w = rec[sl];
             sinfo[sl] = (uint32_t)w == kNullTask ? 0xffffffffu
