@@ -312,9 +312,11 @@ void build_node_to_element(feasm_mesh *m);
 std::shared_ptr<Pattern> build_pattern(feasm_mesh *m, int ndn, bool with_contrib = false, bool dof_level = true);
 // the DOF-level CSC of the mesh's own (distinct, not node-major) numbering
 std::shared_ptr<GeneralPattern> build_general_pattern(feasm_mesh *m);
-// every entry of the device connectivity d_conn[0..n) lies in [0, nnodes)
 // d[i] = i on the context's stream (pattern.hip)
 void fill_iota(feasm_ctx *ctx, int32_t *d, int64_t n);
+// 16-byte pieces from pinned host memory, read by a kernel on the context's stream
+void copy_from_pinned(feasm_ctx *ctx, void *dev, const void *pinned, size_t pieces);
+// every entry of the device connectivity d_conn[0..n) lies in [0, nnodes)
 bool conn_in_range(feasm_ctx *ctx, const int32_t *d_conn, int64_t n, int64_t nnodes);
 void build_contributions(feasm_mesh *m, Pattern &p);
 

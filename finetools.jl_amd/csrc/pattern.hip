@@ -549,6 +549,18 @@ void fill_iota(feasm_ctx *ctx, int32_t *d, int64_t n) {
     FEASM_HIP(hipGetLastError());
 }
 
+__global__ void k_copy_from_pinned(uint4 *__restrict__ d, const uint4 *__restrict__ s, size_t n) {
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+        d[i] = s[i];
+}
+
+void copy_from_pinned(feasm_ctx *ctx, void *dev, const void *pinned, size_t pieces) {
+    if (pieces == 0) return;
+    hipLaunchKernelGGL(k_copy_from_pinned, dim3(grid_for((int64_t)pieces, 256, 1024)), dim3(256), 0, ctx->stream,
+                       static_cast<uint4 *>(dev), static_cast<const uint4 *>(pinned), pieces);
+    FEASM_HIP(hipGetLastError());
+}
+
 bool conn_in_range(feasm_ctx *ctx, const int32_t *d_conn, int64_t n, int64_t nnodes) {
     if (n == 0) return true;
     DevPtr flag = dev_alloc(sizeof(unsigned int));
