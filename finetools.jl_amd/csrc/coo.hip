@@ -405,7 +405,7 @@ __global__ __launch_bounds__(64) void k_columns(const int32_t *__restrict__ I, c
     if (st && lane == 0) atomicOr(state, st);
 }
 
-// what the host decides by, into pinned memory: one launch for three copies
+// what the host decides by, into pinned memory: one launch for two copies
 struct ColumnsEnd {
     int64_t nnz;
     uint64_t nlong;
@@ -481,8 +481,8 @@ static feasm_matrix *sparse_by_columns(feasm_ctx *ctx, int64_t nt, const int32_t
                                        int64_t m, int64_t n) {
     // few triples: both ways are launches and waits, and the sort has fewer of
     // them (H8 elasticity in runs: 37k triples 135 us by the sort, 146 this way; 72k
-    // 169, 127); but the sort fills the gaps of a wide matrix's column pointers one
-    // by one (37k triples of 20 M columns 501 ms, this way 2.5)
+    // 169, 127); but the sort fills a wide matrix's column pointers gap by gap, a
+    // wavefront each (37k triples of 20 M columns 7.9 ms, this way 2.5)
     if (nt < kMinTriples && n <= nt) return nullptr;
     hipStream_t s = ctx->stream;
     // A look at a few of the triples first: what this way does before it knows
@@ -519,7 +519,6 @@ static feasm_matrix *sparse_by_columns(feasm_ctx *ctx, int64_t nt, const int32_t
     };
     columns(k_columns<kSmall>, 1u << 17);
     columns(k_columns<kBig>, 1u << 11);  // what the LDS of 256 CUs holds; most matrices have no such column
-
     std::unique_ptr<feasm_matrix> M(new feasm_matrix);
     M->ctx = ctx;
     M->m = m;
